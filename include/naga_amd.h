@@ -316,7 +316,7 @@ int naga_knn(const float* ref, int64_t n_ref, const float* query, int64_t n_q,
  * harnesses that forbid hipMalloc): the same neighbours, bit for bit, with
  * every pointer a DEVICE pointer (ref[n_ref*dims], query[n_q*dims],
  * d2_out/idx_out[n_q*k]) and the cell binning in a static device scratch
- * array of the library (about 21 MB per GPU, held until the process ends),
+ * array of the library (about 38 MB per GPU, held until the process ends),
  * so n_ref <= NAGA_KNN_NOALLOC_MAX_REF; larger n_ref is rejected with
  * NAGA_INVALID_ARGUMENT.  Work is queued on `stream` (a hipStream_t; NULL:
  * the null stream) and the call returns without waiting.  All calls on one

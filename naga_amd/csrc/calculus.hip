@@ -73,10 +73,10 @@ Advection::Advection(const float* pts, int64_t n, int D, int k, int rbf) : n_(n)
     try {
         DeviceBuffer<float> dp(n * D);
         dp.upload(pts, n * D, st_);
-        const DeviceCells cells = bin_points_device(D, dp.get(), n, st_);
+        const DeviceCells cells = bin_points_device(D, dp.get(), n, st_, knn_points_per_cell(D, k));
         DeviceBuffer<float> d2(n * k);
         idx_.allocate(n * k);
-        launch_knn(cells.bins, dp.get(), dp.get(), n, k, d2.get(), idx_.get(), st_);
+        launch_knn(D, cells.bins, dp.get(), n, k, d2.get(), idx_.get(), st_);
         // multiquadric shape parameter per 16384-query batch (divergence.cuh:118-160)
         const int64_t nbatch = (n + 16383) / 16384;
         std::vector<double> hbar(nbatch, 1.0);

@@ -79,8 +79,8 @@ void knn_host(int D, const float* ref, int64_t n_ref, const float* query, int64_
     DeviceBuffer<uint32_t> didx(n_q * k);
     dref.upload(ref, n_ref * D, st);
     dq.upload(query, n_q * D, st);
-    const DeviceCells cells = bin_points_device(D, dref.get(), n_ref, st);
-    launch_knn(cells.bins, dref.get(), dq.get(), n_q, k, dd2.get(), didx.get(), st);
+    const DeviceCells cells = bin_points_device(D, dref.get(), n_ref, st, knn_points_per_cell(D, k));
+    launch_knn(D, cells.bins, dq.get(), n_q, k, dd2.get(), didx.get(), st);
     dd2.download(d2, n_q * k, st);
     didx.download(idx, n_q * k, st);
     NAGA_HIP(hipStreamSynchronize(st));
@@ -174,10 +174,10 @@ void Engine::init_domain(const float* pts, int64_t nbulk, int64_t nlayer, int64_
 
     // divergence operator over all nodes (init_domain :169-181)
     {
-        const DeviceCells cells = bin_points_device(D, pts_.get(), N, st);
+        const DeviceCells cells = bin_points_device(D, pts_.get(), N, st, knn_points_per_cell(D, k));
         DeviceBuffer<float> d2(N * k);
         idx_.allocate(N * k);
-        launch_knn(cells.bins, pts_.get(), pts_.get(), N, k, d2.get(), idx_.get(), st);
+        launch_knn(D, cells.bins, pts_.get(), N, k, d2.get(), idx_.get(), st);
         marks.mark();  // binning and kNN done
         // multiquadric shape parameter: mean nearest distance per 16384-query
         // batch (nonlocal_calculus/divergence.cuh:118-160, operators.cuh:96-117)
@@ -454,10 +454,11 @@ void Engine::init_domain(const float* pts, int64_t nbulk, int64_t nlayer, int64_
     // boundary interpolator (init_domain :223-258): kNN of boundary nodes
     // among the bulk and layer nodes, RPIM weights at spacing h
     if (nbnd > 0) {
-        const DeviceCells cells = bin_points_device(D, pts_.get(), nfluid, st);
+        const DeviceCells cells = bin_points_device(D, pts_.get(), nfluid, st,
+                                                    knn_points_per_cell(D, kb));
         DeviceBuffer<float> bd2(nbnd * kb);
         bidx_.allocate(nbnd * kb);
-        launch_knn(cells.bins, pts_.get(), pts_.get() + nfluid * D, nbnd, kb, bd2.get(),
+        launch_knn(D, cells.bins, pts_.get() + nfluid * D, nbnd, kb, bd2.get(),
                    bidx_.get(), st);
         bw_.allocate(nbnd * kb);
         DeviceBuffer<int> info(nbnd);

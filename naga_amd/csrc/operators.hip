@@ -72,7 +72,7 @@ void Segmentation::knn(const float* query, int64_t n_q, int k, float* d2, uint32
     DeviceBuffer<float> dq(size_t(n_q) * D_), dd2(size_t(n_q) * k);
     DeviceBuffer<uint32_t> didx(size_t(n_q) * k);
     dq.upload(query, dq.size(), st_);
-    launch_knn(cells_.bins, pts_.get(), dq.get(), n_q, k, dd2.get(), didx.get(), st_);
+    launch_knn(D_, cells_.bins, dq.get(), n_q, k, dd2.get(), didx.get(), st_);
     dd2.download(d2, dd2.size(), st_);
     didx.download(idx, didx.size(), st_);
     NAGA_HIP(hipStreamSynchronize(st_));

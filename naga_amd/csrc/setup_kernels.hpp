@@ -32,16 +32,17 @@ struct CellBins {
     uint32_t* start;    // cap + 1
     uint32_t* counts;   // cap + 1
     uint32_t* sorted;   // n
+    float4* pts;        // n: {x, y, z (0 in 2D), index bits} in the order of sorted
     int64_t cap;        // cell capacity
     int64_t n;
 };
 // Scratch layout of one binning of n points (offsets 256-byte aligned):
 // the grid, per-block bounds, cell counts and starts, scan block sums, the
-// sorted indices.
+// sorted indices and the points in that order.
 constexpr int kBoundBlocks = 256;
 constexpr int kScanChunk = 2048;  // elements per scan block: 256 threads x 8
 struct BinLayout {
-    size_t grid, partial, counts, start, bsum, sorted, total;
+    size_t grid, partial, counts, start, bsum, sorted, pts, total;
     int64_t cap, nblocks;
 };
 constexpr size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
@@ -63,6 +64,8 @@ constexpr BinLayout bin_layout(int64_t n) {
     off = align256(off + size_t(L.nblocks) * 4);
     L.sorted = off;
     off = align256(off + size_t(n) * 4);
+    L.pts = off;
+    off = align256(off + size_t(n) * 16);
     L.total = off;
     return L;
 }
@@ -80,12 +83,16 @@ struct DeviceCells {
     CellBins bins{};
 };
 DeviceCells bin_points_device(int D, const float* pts, int64_t n, hipStream_t stream,
-                              double per_cell = 2.0, double width = 0.0);
+                              double per_cell, double width = 0.0);
+// Points per cell for a search of k neighbours: the cell width is then 1.1
+// times the radius that holds k points at the cloud's mean density, so the
+// 3^D cells around a query bound a ball that holds its k nearest.
+double knn_points_per_cell(int D, int k);
 
 // Exact k-nearest neighbours of each query among ref, key (d2, index)
 // ascending, d2 in FP32 as dz^2 + (dy^2 + dx^2) with no contraction.
-// All pointers are device pointers; bins are those of ref.
-void launch_knn(const CellBins& bins, const float* ref, const float* query, int64_t n_q, int k,
+// All pointers are device pointers; bins are those of ref (D-dimensional).
+void launch_knn(int D, const CellBins& bins, const float* query, int64_t n_q, int k,
                 float* d2_out, uint32_t* idx_out, hipStream_t stream);
 
 // Batched dense LU with partial pivoting + solve, FP64, one wavefront per
