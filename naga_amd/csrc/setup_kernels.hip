@@ -6,6 +6,7 @@
 
 #include <algorithm>
 #include <mutex>
+#include <utility>
 #include <vector>
 
 namespace naga_amd {
@@ -24,26 +25,6 @@ __device__ __forceinline__ uint64_t shfl_xor64(uint64_t v, int m) {
     const int lo = __shfl_xor(int(uint32_t(v)), m);
     const int hi = __shfl_xor(int(uint32_t(v >> 32)), m);
     return (uint64_t(uint32_t(hi)) << 32) | uint32_t(lo);
-}
-
-__device__ __forceinline__ double shfl_xor_d(double v, int m) {
-    return __longlong_as_double(
-        (long long)shfl_xor64(uint64_t(__double_as_longlong(v)), m));
-}
-
-__device__ __forceinline__ float shfl_xor_d(float v, int m) { return __shfl_xor(v, m); }
-
-// value of lane `src` (wave-uniform) for every lane
-__device__ __forceinline__ float bcast_d(float v, int src) {
-    const int s = __builtin_amdgcn_readfirstlane(src);
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), s));
-}
-__device__ __forceinline__ double bcast_d(double v, int src) {
-    const int s = __builtin_amdgcn_readfirstlane(src);
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_readlane(int(uint32_t(b)), s);
-    const int hi = __builtin_amdgcn_readlane(int(uint32_t(uint64_t(b) >> 32)), s);
-    return __longlong_as_double((long long)((uint64_t(uint32_t(hi)) << 32) | uint32_t(lo)));
 }
 
 // FP32 squared distance, fixed order, no contraction (the kNN key).
@@ -391,88 +372,203 @@ __global__ __launch_bounds__(256) void k_knn(const CellGrid* __restrict__ gp,
 
 // ---------------------------------------------------------------------------
 // Wavefront LU with partial pivoting (Golub & Van Loan, Alg. 3.4.1).  Lane r
-// holds row r of A (row[c] = A[r][c]) and its right-hand sides.  Row swaps
-// are tracked as positions instead of moving data; ties in |pivot| go to the
-// smallest current position, as a row-swapping LU scanning downwards picks.
-// On return the lane at position p holds unknown p in rhs[].
-// Returns the lane's position, or -1 for a zero pivot (wave-uniform).
+// holds row r of A in registers and its right-hand sides.  Rows stay in
+// their lanes: the pivot row reaches the others through v_readlane (scalar
+// operands of the update).  Every step works on register 0 and shifts the
+// row down by one, so the steps are a loop with constant register indices;
+// the loop's width drops by four columns every four steps.  A pivot row's
+// entries right of its pivot are dropped by the shift one per step and kept
+// in LDS, packed by column, for the back substitution.  Row swaps are
+// tracked as positions, ties in |pivot| going to the smallest current
+// position, as a row-swapping LU scanning downwards picks.
+//
+// With the rows in LDS (two reads and a write per element and lane, two
+// barriers per step) and a 64-bit pivot search by shuffles the steps were
+// bound by LDS latency at 13 wavefronts per CU; the pivot is now found on
+// the high words by DPP, the low words only deciding between equal ones.
+// Weights of 132,651 cube nodes, k = 32 (36 x 36 systems): 6.85 -> 2.66 ms.
 // ---------------------------------------------------------------------------
-// The rows live in LDS (lu[lane * LD + c], LD = lu_stride(NMAX), filled by
-// the caller): the steps run as loops over the system's own size, whose
-// indices are not compile-time constants (a register array indexed at run
-// time would be placed in scratch memory; one unrolled for every size is
-// too large to build).  The odd stride spreads the lanes' rows over banks.
-// Only lanes below NMAX >= n own a row (lu holds NMAX rows); the others
-// read row 0 where a value is needed but never used, and write nothing.
-constexpr int lu_stride(int nmax) { return nmax + 1; }
-template <int NMAX, class T>
-__device__ __forceinline__ T* lu_row(T* lu) {
-    const int lane = threadIdx.x & 63;
-    return lu + (lane < NMAX ? lane : 0) * lu_stride(NMAX);
+__device__ __forceinline__ float lane_value(float v, int lane) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
+}
+__device__ __forceinline__ double lane_value(double v, int lane) {
+    const uint64_t b = uint64_t(__double_as_longlong(v));
+    const uint32_t lo = __builtin_amdgcn_readlane(int(uint32_t(b)), lane);
+    const uint32_t hi = __builtin_amdgcn_readlane(int(uint32_t(b >> 32)), lane);
+    return __longlong_as_double((long long)((uint64_t(hi) << 32) | lo));
+}
+// |v| in order as unsigned words: the high one first
+__device__ __forceinline__ uint32_t abs_high(float v) { return __float_as_uint(v) & 0x7fffffffu; }
+__device__ __forceinline__ uint32_t abs_low(float) { return 0; }
+__device__ __forceinline__ uint32_t abs_high(double v) {
+    return uint32_t(uint64_t(__double_as_longlong(v)) >> 32) & 0x7fffffffu;
+}
+__device__ __forceinline__ uint32_t abs_low(double v) {
+    return uint32_t(uint64_t(__double_as_longlong(v)));
 }
 
-template <int NMAX, int NR, class T>
-__device__ int wave_lu_solve(T* lu, T (&rhs)[NR], int n) {
-    constexpr int LD = lu_stride(NMAX);
-    const int lane = threadIdx.x & 63;
-    T* r = lu_row<NMAX>(lu);
-    __syncthreads();  // the rows are in place
-    int pos = lane;
-    bool done = lane >= n;
+// Largest v over the wavefront (uniform).
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
+#define NAGA_DPP_MAX(ctrl)                                                                  \
+    v = max(v, uint32_t(__builtin_amdgcn_update_dpp(int(v), int(v), ctrl, 0xf, 0xf, false)))
+    NAGA_DPP_MAX(0xb1);   // quad_perm [1, 0, 3, 2]
+    NAGA_DPP_MAX(0x4e);   // quad_perm [2, 3, 0, 1]
+    NAGA_DPP_MAX(0x141);  // row_half_mirror
+    NAGA_DPP_MAX(0x140);  // row_mirror: every lane of a row holds its maximum
+    NAGA_DPP_MAX(0x142);  // row_bcast15
+    NAGA_DPP_MAX(0x143);  // row_bcast31: lane 63 holds the wavefront's
+#undef NAGA_DPP_MAX
+    return uint32_t(__builtin_amdgcn_readlane(int(v), 63));
+}
+
+// a / b given y ~ 1 / b.  Quick: y from v_rcp_f64 by two Newton steps, the
+// quotient corrected by its residual (Markstein), for systems whose entries
+// stay far from the ends of the exponent range; else the plain division.
+template <bool QUICK>
+struct Divisor {
+    double b, y;
+    __device__ explicit Divisor(double v) : b(v), y(0.0) {
+        if (QUICK) {
+            y = __builtin_amdgcn_rcp(v);
+            y = fma(fma(-v, y, 1.0), y, y);
+            y = fma(fma(-v, y, 1.0), y, y);
+        }
+    }
+    __device__ double of(double a) const {
+        if (!QUICK) return a / b;
+        const double q = a * y;
+        return fma(fma(-q, b, a), y, q);
+    }
+};
+
+// LDS of one factorisation: the entries right of the diagonal, column j from
+// j (j - 1) / 2.
+constexpr int lu_upper(int nmax) { return nmax * (nmax - 1) / 2; }
+
+// QUICK: entries are finite and far from the ends of the exponent range
+// (quotients by reciprocals; finished rows take part in the shift with a
+// zero multiplier instead of a branch).
+template <int NMAX, int NR, bool QUICK, class T>
+struct WaveLu {
+    T (&row)[NMAX];
+    T (&rhs)[NR];
+    T* upper;
+    const int n, lane;
+    int j = 0, pos, col = 64;
+    bool open;                 // not yet a pivot row
     bool singular = false;
-    for (int j = 0; j < n; ++j) {
-        T v = done ? T(-1) : fabs(r[j]);
-        int bp = done ? 1 << 20 : pos, bl = lane;
+    T own = T(0);              // this row's pivot
+    double recip = 0.0;        // quick: its reciprocal
+
+    __device__ __forceinline__ WaveLu(T (&r)[NMAX], T (&b)[NR], T* u, int n_)
+        : row(r), rhs(b), upper(u), n(n_), lane(threadIdx.x & 63), pos(lane), open(lane < n_) {}
+
+    // Steps while more than W0 - 4 columns are left, on the first W0 registers.
+    template <int W0>
+    __device__ __forceinline__ void steps() {
+        constexpr int W = W0 < NMAX ? W0 : NMAX;
+        while (n - j > W0 - 4 && j < n && !singular) {
+            const uint32_t hi = abs_high(row[0]);
+            const uint32_t most = wave_max_u32(open ? hi : 0u);
+            uint64_t same = __ballot(open && hi == most);
+            int p = int(__ffsll((unsigned long long)same)) - 1;
+            if (same & (same - 1)) {  // equal high words: low words, then positions
+                uint32_t plo = __builtin_amdgcn_readlane(int(abs_low(row[0])), p);
+                int ppos = __builtin_amdgcn_readlane(pos, p);
+                for (same &= same - 1; same; same &= same - 1) {
+                    const int l = int(__ffsll((unsigned long long)same)) - 1;
+                    const uint32_t llo = __builtin_amdgcn_readlane(int(abs_low(row[0])), l);
+                    const int lpos = __builtin_amdgcn_readlane(pos, l);
+                    if (llo > plo || (llo == plo && lpos < ppos)) {
+                        p = l;
+                        plo = llo;
+                        ppos = lpos;
+                    }
+                }
+            }
+            p = __builtin_amdgcn_readfirstlane(p);
+            const T piv = lane_value(row[0], p);
+            if (!(fabs(piv) > T(0))) {
+                singular = true;
+                break;
+            }
+            const int pos_p = __builtin_amdgcn_readlane(pos, p);
+            if (pos == j) pos = pos_p;
+            if (col < j) upper[j * (j - 1) / 2 + col] = row[0];
+            T l;
+            if constexpr (sizeof(T) == 8) {
+                const Divisor<QUICK> d(piv);
+                l = d.of(row[0]);
+                if (lane == p) recip = d.y;
+            } else {
+                l = row[0] / piv;
+            }
+            if (lane == p) {
+                pos = j;
+                col = j;
+                own = piv;
+                open = false;
+            }
+            if constexpr (QUICK) {
+                l = open ? l : T(0);
 #pragma unroll
-        for (int o = 32; o >= 1; o >>= 1) {
-            const T ov = shfl_xor_d(v, o);
-            const int op = __shfl_xor(bp, o), ol = __shfl_xor(bl, o);
-            if (ov > v || (ov == v && op < bp)) {
-                v = ov;
-                bp = op;
-                bl = ol;
+                for (int c = 1; c < W; ++c) row[c - 1] = row[c] - l * lane_value(row[c], p);
+#pragma unroll
+                for (int m = 0; m < NR; ++m) rhs[m] -= l * lane_value(rhs[m], p);
+            } else {
+#pragma unroll
+                for (int c = 1; c < W; ++c) {
+                    const T pr = lane_value(row[c], p);
+                    row[c - 1] = open ? row[c] - l * pr : row[c];
+                }
+#pragma unroll
+                for (int m = 0; m < NR; ++m) {
+                    const T b = lane_value(rhs[m], p);
+                    rhs[m] = open ? rhs[m] - l * b : rhs[m];
+                }
+            }
+            ++j;
+        }
+    }
+    template <int... I>
+    __device__ __forceinline__ void all_steps(std::integer_sequence<int, I...>) {
+        (steps<(NMAX + 3) / 4 * 4 - 4 * I>(), ...);
+    }
+
+    // Unknown c lives in the lane whose pivot step was c.
+    __device__ __forceinline__ void back() {
+        const int mine = col < 64 ? col : 0;
+#pragma unroll 4
+        for (int c = n - 1; c >= 0; --c) {
+            const T u = upper[c * (c - 1) / 2 + (mine < c ? mine : 0)];
+            const int p = int(__ffsll((unsigned long long)__ballot(col == c))) - 1;
+#pragma unroll
+            for (int m = 0; m < NR; ++m) {
+                T q;  // of the pivot lane's own values
+                if constexpr (sizeof(T) == 8 && QUICK) {
+                    q = rhs[m] * recip;
+                    q = fma(fma(-q, own, rhs[m]), recip, q);
+                } else {
+                    q = rhs[m] / own;
+                }
+                const T x = lane_value(q, p);
+                rhs[m] = col == c ? x : col < c ? rhs[m] - u * x : rhs[m];
             }
         }
-        const int p = __builtin_amdgcn_readfirstlane(bl);
-        if (!(v > T(0))) singular = true;
-        const int pos_p = __builtin_amdgcn_readlane(pos, p);
-        if (pos == j) pos = pos_p;
-        if (lane == p) pos = j;
-        const T* pr = lu + p * LD;  // the pivot row (every lane reads the same words)
-        const T piv = pr[j];
-        T prhs[NR];
-#pragma unroll
-        for (int m = 0; m < NR; ++m) prhs[m] = bcast_d(rhs[m], p);
-        const bool upd = !done && lane != p;
-        const T l = upd ? r[j] / piv : T(0);
-        if (upd) {
-            // columns n and above are zero in every row: nothing to update
-            for (int c = j + 1; c < n; ++c) r[c] -= l * pr[c];
-            r[j] = l;
-#pragma unroll
-            for (int m = 0; m < NR; ++m) rhs[m] -= l * prhs[m];
-        }
-        if (lane == p) done = true;
-        __syncthreads();  // this step's rows before the next pivot is read
     }
-    if (singular) return -1;
-    // back substitution, unknown j lives in the lane at position j
-    T s[NR];
-#pragma unroll
-    for (int m = 0; m < NR; ++m) s[m] = rhs[m];
-    for (int j = n - 1; j >= 0; --j) {
-        const unsigned long long mask = __ballot(pos == j && lane < n);
-        const int lj = __builtin_amdgcn_readfirstlane(int(__ffsll((long long)mask) - 1));
-        const T ujj = lu[lj * LD + j];
-        const T rj = r[j];
-#pragma unroll
-        for (int m = 0; m < NR; ++m) {
-            const T xj = bcast_d(s[m], lj) / ujj;
-            if (pos == j) rhs[m] = xj;
-            if (pos < j && lane < n) s[m] -= rj * xj;
-        }
-    }
-    return lane < n ? pos : 64;
+};
+
+// Solves for NR right-hand sides; upper: lu_upper(NMAX) values of LDS (at
+// least one).  Returns the unknown that the lane then holds in rhs[] (64:
+// none), or -1 in every lane for a zero pivot.
+template <int NMAX, int NR, bool QUICK, class T>
+__device__ __forceinline__ int wave_lu_solve(T (&row)[NMAX], T (&rhs)[NR], T* upper, int n) {
+    WaveLu<NMAX, NR, QUICK, T> w(row, rhs, upper, __builtin_amdgcn_readfirstlane(n));
+    w.all_steps(std::make_integer_sequence<int, (NMAX + 3) / 4>());
+    if (w.singular) return -1;
+    __syncthreads();  // the entries kept in LDS
+    w.back();
+    return w.col;
 }
 
 // unscaled quadrature points, [0]: 2D (16 used), [1]: 3D (64); both
@@ -487,40 +583,64 @@ __device__ __forceinline__ double dist2_f64(int D, const double* a, const double
     return s;
 }
 
-__device__ __forceinline__ double rbf_eval(int rbf, double r2, double spacing) {
-    if (rbf == 1) return r2 * sqrt(r2);
-    const double c = spacing * 0.1;
-    return sqrt(r2 + c * c);
+// Square root of x = 0 or 2^-700 < x < 2^700 (squared distances of FP32
+// points): v_rsq_f64 refined by one Goldschmidt step and the residual of the
+// result; without the scaling a full-range square root needs.
+__device__ __forceinline__ double sqrt_mid(double x) {
+    const double y = __builtin_amdgcn_rsq(x);
+    double g = x * y, h = 0.5 * y;
+    const double r = fma(-h, g, 0.5);
+    g = fma(g, r, g);
+    h = fma(h, r, h);
+    g = fma(fma(-g, g, x), h, g);
+    return x > 0.0 ? g : 0.0;
 }
 
-// Row r of the augmented RBF matrix [[Phi, P], [P^T, 0]] in raw coordinates
-// (interpolation/detail/radial_point_method.cuh:349-398).
-template <int NMAX, class T>
-__device__ void g0_row(int D, const double (*xs)[3], int k, int rbf,
-                       double spacing, int r, T* row) {
+__device__ __forceinline__ double rbf_eval(int rbf, double r2, double spacing) {
+    if (rbf == 1) return r2 * sqrt_mid(r2);
+    const double c = spacing * 0.1;
+    return sqrt_mid(r2 + c * c);
+}
+
+// Row `lane` of the augmented RBF matrix [[Phi, P], [P^T, 0]] in raw
+// coordinates (interpolation/detail/radial_point_method.cuh:349-398), zeros
+// past its n = k + D + 1 columns.
+template <int NMAX, int D, class T>
+__device__ __forceinline__ void g0_row(const double (*xs)[4], int k, int rbf, double spacing,
+                                       T (&row)[NMAX]) {
+    const int lane = threadIdx.x & 63;
     const int n = k + D + 1;
+    const int axis = lane > k && lane < n ? lane - k - 1 : 0;
+    double mine[D];
+#pragma unroll
+    for (int d = 0; d < D; ++d) mine[d] = xs[lane][d];
 #pragma unroll
     for (int c = 0; c < NMAX; ++c) {
         double v = 0.0;
-        if (r < n && c < n) {
-            if (r < k && c < k)
-                v = rbf_eval(rbf, dist2_f64(D, xs[r], xs[c]), spacing);
-            else if (r < k)
-                v = (c == k) ? 1.0 : xs[r][c - k - 1];
-            else if (c < k)
-                v = (r == k) ? 1.0 : xs[c][r - k - 1];
+        if (c < k) {
+            double o[D];
+#pragma unroll
+            for (int d = 0; d < D; ++d) o[d] = xs[c][d];
+            v = rbf_eval(rbf, dist2_f64(D, mine, o), spacing);
+            v = lane < k ? v : lane == k ? 1.0 : xs[c][axis];
+        } else if (c == k) {
+            v = lane < k ? 1.0 : 0.0;
+        } else if (c < n) {
+            v = lane < k ? xs[lane][c - k - 1] : 0.0;
         }
-        if (r < NMAX) row[c] = T(v);
+        row[c] = lane < n ? T(v) : T(0);
     }
 }
 
-// entry r of G_x (:400-433)
-__device__ __forceinline__ double gx_entry(int D, const double (*xs)[3], int k,
-                                           int rbf, double spacing, int r,
-                                           const double* xq) {
-    if (r < k) return rbf_eval(rbf, dist2_f64(D, xs[r], xq), spacing);
-    if (r == k) return 1.0;
-    return xq[r - k - 1];
+// entry `lane` of G_x (:400-433)
+template <int D>
+__device__ __forceinline__ double gx_entry(const double (*xs)[4], const double* mine, int k,
+                                           int rbf, double spacing, const double* xq) {
+    const int lane = threadIdx.x & 63;
+    double v = rbf_eval(rbf, dist2_f64(D, mine, xq), spacing);
+#pragma unroll
+    for (int d = 0; d < D; ++d) v = lane == k + 1 + d ? xq[d] : v;
+    return lane == k ? 1.0 : v;
 }
 
 // antisymmetric w4 B-spline kernel times the quadrature weight
@@ -563,13 +683,23 @@ __device__ void quad_term(int D, double delta, const double* xi, const double* x
 // write W(d, s) = y_d[s] (+ sum_q alpha_d w for s = 0).  By linearity this
 // equals the reference's per-quadrature-point RPIM weights summed against
 // the kernel (detail/divergence.inl:203-215) with D solves instead of Nq.
+// Lane q forms quadrature point q and its kernel weights once; the points
+// then reach every lane (a row of the system each) as broadcast LDS reads.
 template <int NMAX, int D, class T>
-__global__ __launch_bounds__(64) void k_divw(const float* src, const float* query,
-                                             int64_t n_q, const uint32_t* idx,
-                                             const float* d2, int kmax, int rbf,
-                                             const double* hbar, const uint8_t* kvar,
-                                             float* W, double* W64, int* info) {
-    __shared__ double xs[64][3];
+__global__ __launch_bounds__(64) void k_divw(const float* __restrict__ src,
+                                             const float* __restrict__ query, int64_t n_q,
+                                             const uint32_t* __restrict__ idx,
+                                             const float* __restrict__ d2, int kmax, int rbf,
+                                             const double* __restrict__ hbar,
+                                             const uint8_t* __restrict__ kvar,
+                                             float* __restrict__ W, double* __restrict__ W64,
+                                             int* __restrict__ info) {
+    constexpr int Nq = D == 2 ? 16 : 64;
+    __shared__ double xs[64][4];
+    // quadrature points and their kernel weights, then the factorisation
+    constexpr size_t kQuad = sizeof(double) * Nq * 2 * D, kUpper = sizeof(T) * lu_upper(NMAX);
+    __shared__ double pool[((kQuad > kUpper ? kQuad : kUpper) + 7) / 8];
+    double(*quad)[2 * D] = reinterpret_cast<double(*)[2 * D]>(pool);
     const int lane = threadIdx.x;
     const int64_t i = blockIdx.x;
     if (i >= n_q) return;
@@ -581,78 +711,80 @@ __global__ __launch_bounds__(64) void k_divw(const float* src, const float* quer
             W[(i * kmax + lane) * D + d] = 0.0f;
             if (W64) W64[(i * kmax + lane) * D + d] = 0.0;
         }
+    double mine[3] = {0.0, 0.0, 0.0};
     if (lane < k) {
         const int64_t j = idx[i * kmax + lane];
-        for (int d = 0; d < D; ++d) xs[lane][d] = double(src[j * D + d]);
+        for (int d = 0; d < D; ++d) mine[d] = double(src[j * D + d]);
     }
-    __syncthreads();
+    for (int d = 0; d < D; ++d) xs[lane][d] = mine[d];
     double xi[3] = {0.0, 0.0, 0.0};
     for (int d = 0; d < D; ++d) xi[d] = double(query[i * D + d]);
     const double delta = 0.05 * sqrt(double(d2[i * kmax + 1]));
     const double spacing = hbar[i / 16384];
-    __shared__ T lu[NMAX * lu_stride(NMAX)];
-    g0_row<NMAX>(D, xs, k, rbf, spacing, lane, lu_row<NMAX>(lu));
+    if (lane < Nq) {
+        double xq[3] = {0.0, 0.0, 0.0}, aw[3];
+        for (int d = 0; d < D; ++d) xq[d] = c_quad_unit[D - 2][lane][d] * delta + xi[d];
+        quad_term(D, delta, xi, xq, lane, aw);
+        for (int d = 0; d < D; ++d) {
+            quad[lane][d] = xq[d];
+            quad[lane][D + d] = aw[d];
+        }
+    }
+    __syncthreads();
     double b64[D], S[D];
     for (int d = 0; d < D; ++d) b64[d] = S[d] = 0.0;
-    const int Nq = D == 2 ? 16 : 64;
+#pragma unroll 4
     for (int q = 0; q < Nq; ++q) {
-        double xq[3] = {0.0, 0.0, 0.0};
-        for (int d = 0; d < D; ++d) xq[d] = c_quad_unit[D - 2][q][d] * delta + xi[d];
-        double aw[3];
-        quad_term(D, delta, xi, xq, q, aw);
-        const double gx = lane < n ? gx_entry(D, xs, k, rbf, spacing, lane, xq) : 0.0;
+        const double gx = gx_entry<D>(xs, mine, k, rbf, spacing, quad[q]);
+#pragma unroll
         for (int d = 0; d < D; ++d) {
-            b64[d] += aw[d] * gx;
-            S[d] += aw[d];
+            b64[d] += quad[q][D + d] * gx;
+            S[d] += quad[q][D + d];
         }
     }
-    T b[D];
+    T b[D], row[NMAX];
     for (int d = 0; d < D; ++d) b[d] = T(b64[d]);
-    const int pos = wave_lu_solve<NMAX, D, T>(lu, b, n);
-    if (pos < 0) {
-        if (lane == 0) info[i] = 1;
-        return;
-    }
-    if (lane == 0) info[i] = 0;
-    if (pos < k) {
-        for (int d = 0; d < D; ++d) {
-            const double v = double(b[d]) + (pos == 0 ? S[d] : 0.0);
-            W[(i * kmax + pos) * D + d] = float(v);
-            if (W64) W64[(i * kmax + pos) * D + d] = v;
-        }
+    g0_row<NMAX, D>(xs, k, rbf, spacing, row);
+    __syncthreads();  // every lane is done with the quadrature points
+    const int col = wave_lu_solve<NMAX, D, true, T>(row, b, reinterpret_cast<T*>(pool), n);
+    if (lane == 0) info[i] = col < 0 ? 1 : 0;
+    if (col < 0 || col >= k) return;
+    for (int d = 0; d < D; ++d) {
+        const double v = double(b[d]) + (col == 0 ? S[d] : 0.0);
+        W[(i * kmax + col) * D + d] = float(v);
+        if (W64) W64[(i * kmax + col) * D + d] = v;
     }
 }
 
 template <int NMAX, int D, class T>
-__global__ __launch_bounds__(64) void k_rpim(const float* src, const float* query,
-                                             int64_t n_q, const uint32_t* idx,
-                                             int k, int rbf, double spacing,
-                                             float* w, double* w64, int* info, int group) {
-    __shared__ double xs[64][3];
+__global__ __launch_bounds__(64) void k_rpim(const float* __restrict__ src,
+                                             const float* __restrict__ query, int64_t n_q,
+                                             const uint32_t* __restrict__ idx, int k, int rbf,
+                                             double spacing, float* __restrict__ w,
+                                             double* __restrict__ w64, int* __restrict__ info,
+                                             int group) {
+    __shared__ double xs[64][4];
     const int lane = threadIdx.x;
     const int64_t i = blockIdx.x;
     if (i >= n_q) return;
-    const int n = k + D + 1;
+    double mine[3] = {0.0, 0.0, 0.0};
     if (lane < k) {  // the queries of a group share their group's stencil
         const int64_t j = idx[(i / group) * k + lane];
-        for (int d = 0; d < D; ++d) xs[lane][d] = double(src[j * D + d]);
+        for (int d = 0; d < D; ++d) mine[d] = double(src[j * D + d]);
     }
+    for (int d = 0; d < D; ++d) xs[lane][d] = mine[d];
     __syncthreads();
     double xq[3] = {0.0, 0.0, 0.0};
     for (int d = 0; d < D; ++d) xq[d] = double(query[i * D + d]);
-    __shared__ T lu[NMAX * lu_stride(NMAX)];
-    g0_row<NMAX>(D, xs, k, rbf, spacing, lane, lu_row<NMAX>(lu));
-    T b[1] = {T(lane < n ? gx_entry(D, xs, k, rbf, spacing, lane, xq) : 0.0)};
-    const int pos = wave_lu_solve<NMAX, 1, T>(lu, b, n);
-    if (pos < 0) {
-        if (lane == 0) info[i] = 1;
-        return;
-    }
-    if (lane == 0) info[i] = 0;
-    if (pos < k) {
-        w[i * k + pos] = float(b[0]);
-        if (w64) w64[i * k + pos] = double(b[0]);
-    }
+    __shared__ T upper[lu_upper(NMAX)];
+    T row[NMAX];
+    g0_row<NMAX, D>(xs, k, rbf, spacing, row);
+    T b[1] = {T(gx_entry<D>(xs, mine, k, rbf, spacing, xq))};
+    const int col = wave_lu_solve<NMAX, 1, true, T>(row, b, upper, k + D + 1);
+    if (lane == 0) info[i] = col < 0 ? 1 : 0;
+    if (col < 0 || col >= k) return;
+    w[i * k + col] = float(b[0]);
+    if (w64) w64[i * k + col] = double(b[0]);
 }
 
 template <int NMAX>
@@ -663,25 +795,27 @@ __global__ __launch_bounds__(64) void k_batched_lu(int n, int nrhs, int64_t batc
     if (b >= batch) return;
     const double* Ab = A + b * int64_t(n) * n;
     double* Bb = B + b * int64_t(n) * nrhs;
-    __shared__ double lu[NMAX * lu_stride(NMAX)];
-    double* r = lu_row<NMAX>(lu);
+    __shared__ double upper[lu_upper(NMAX)];
     // right-hand sides are processed four at a time, each group against a
     // fresh copy of the matrix
     for (int m0 = 0; m0 < nrhs; m0 += 4) {
-        __syncthreads();  // the previous group's factorisation is done with lu
-#pragma unroll 4
+        double row[NMAX], rhs[4];
+#pragma unroll
         for (int c = 0; c < NMAX; ++c)
-            if (lane < NMAX) r[c] = (lane < n && c < n) ? Ab[lane + int64_t(c) * n] : 0.0;
-        double rhs[4];
+            row[c] = (lane < n && c < n) ? Ab[lane + int64_t(c) * n] : 0.0;
+#pragma unroll
         for (int m = 0; m < 4; ++m)
             rhs[m] = (lane < n && m0 + m < nrhs) ? Bb[lane + int64_t(m0 + m) * n] : 0.0;
-        const int pos = wave_lu_solve<NMAX, 4, double>(lu, rhs, n);
-        if (pos < 0) {
+        const int col = wave_lu_solve<NMAX, 4, false, double>(row, rhs, upper, n);
+        if (col < 0) {
             if (lane == 0) info[b] = 1;
             return;
         }
-        if (pos < n)
-            for (int m = 0; m < 4 && m0 + m < nrhs; ++m) Bb[pos + int64_t(m0 + m) * n] = rhs[m];
+        if (col < n)
+#pragma unroll
+            for (int m = 0; m < 4; ++m)
+                if (m0 + m < nrhs) Bb[col + int64_t(m0 + m) * n] = rhs[m];
+        __syncthreads();  // before the next group's factorisation
     }
     if (lane == 0) info[b] = 0;
 }
