@@ -82,9 +82,13 @@ __device__ __forceinline__ uint64_t knn_key(const float* x, const float4& c) {
     return (uint64_t(__float_as_uint(dist2_f32(D, x, p))) << 32) | __float_as_uint(c.w);
 }
 
-// One query by rings of cells around its own: every cell row of a ring is
+// One query by rings of cells around its own: the ring's rows of cells are
+// looked up 64 at a time, one per lane, and those that hold points are
 // merged, 64 points at a time, into the running list, until the k-th distance
 // is inside the searched box.  Takes any cloud; knn_box serves most queries.
+// (Queries far from a hollow cloud pass many empty rings: visiting every row
+// by the whole wavefront made the nodes' distance to the boundary most of a
+// grid's set-up.)
 template <int D>
 __device__ void knn_rings(const CellGrid& G, const float4* cpts, const uint32_t* start,
                           const float* x, int64_t q, int k, float* d2o, uint32_t* idxo) {
@@ -96,42 +100,46 @@ __device__ void knn_rings(const CellGrid& G, const float4* cpts, const uint32_t*
     }
     uint64_t top = kMaxKey, kth = kMaxKey;
     for (int64_t r = 0;; ++r) {
-        const int64_t zr = D == 3 ? r : 0;
-        for (int64_t dz = -zr; dz <= zr; ++dz) {
-            const int64_t cz = qc[2] + dz;
-            if (cz < 0 || cz >= G.dims[2]) continue;
-            for (int64_t dy = -r; dy <= r; ++dy) {
-                const int64_t cy = qc[1] + dy;
-                if (cy < 0 || cy >= G.dims[1]) continue;
-                const bool face = (dy == r || dy == -r) || (D == 3 && (dz == r || dz == -r));
+        // rows of the ring inside the grid
+        const int64_t y0 = qc[1] - r < 0 ? 0 : qc[1] - r;
+        const int64_t y1 = qc[1] + r >= G.dims[1] ? G.dims[1] - 1 : qc[1] + r;
+        const int64_t z0 = D == 2 ? 0 : qc[2] - r < 0 ? 0 : qc[2] - r;
+        const int64_t z1 = D == 2 ? 0 : qc[2] + r >= G.dims[2] ? G.dims[2] - 1 : qc[2] + r;
+        const int64_t ny = y1 - y0 + 1, nrow = ny * (z1 - z0 + 1);
+        const int64_t xa = qc[0] - r, xb = qc[0] + r;
+        const int64_t xl = xa < 0 ? 0 : xa, xr = xb >= G.dims[0] ? G.dims[0] - 1 : xb;
+        for (int64_t b0 = 0; b0 < nrow; b0 += 64) {
+            // the row's points: a whole row of cells on the ring's faces in
+            // y and z, else the cells at its two ends
+            uint32_t p0 = 0, p1 = 0, s0 = 0, s1 = 0;
+            if (b0 + lane < nrow) {
+                const int64_t cz = z0 + (b0 + lane) / ny, cy = y0 + (b0 + lane) % ny;
                 const int64_t row = G.dims[0] * (cy + G.dims[1] * cz);
-                int64_t seg[2][2];
-                int nseg = 0;
+                const bool face = cy == qc[1] - r || cy == qc[1] + r ||
+                                  (D == 3 && (cz == qc[2] - r || cz == qc[2] + r));
                 if (face) {
-                    int64_t a = qc[0] - r, b = qc[0] + r;
-                    if (a < 0) a = 0;
-                    if (b >= G.dims[0]) b = G.dims[0] - 1;
-                    seg[nseg][0] = a;
-                    seg[nseg++][1] = b;
+                    p0 = start[row + xl];
+                    p1 = start[row + xr + 1];
                 } else {
-                    if (qc[0] - r >= 0) {
-                        seg[nseg][0] = qc[0] - r;
-                        seg[nseg++][1] = qc[0] - r;
+                    if (xa >= 0) {
+                        p0 = start[row + xa];
+                        p1 = start[row + xa + 1];
                     }
-                    if (qc[0] + r < G.dims[0]) {
-                        seg[nseg][0] = qc[0] + r;
-                        seg[nseg++][1] = qc[0] + r;
+                    if (xb < G.dims[0]) {
+                        s0 = start[row + xb];
+                        s1 = start[row + xb + 1];
                     }
                 }
-                for (int t = 0; t < nseg; ++t) {
-                    const int64_t p0 = start[row + seg[t][0]];
-                    const int64_t p1 = start[row + seg[t][1] + 1];  // cells are row-major in x
-                    for (int64_t base = p0; base < p1; base += 64) {
-                        const int64_t p = base + lane;
-                        uint64_t key = kMaxKey;
-                        if (p < p1) {
-                            key = knn_key<D>(x, cpts[p]);
-                        }
+            }
+            for (uint64_t has = __ballot(p0 < p1 || s0 < s1); has; has &= has - 1) {
+                const int l = int(__ffsll((unsigned long long)has)) - 1;
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    const uint32_t a = __builtin_amdgcn_readlane(int(t ? s0 : p0), l);
+                    const uint32_t e = __builtin_amdgcn_readlane(int(t ? s1 : p1), l);
+                    for (uint32_t base = a; base < e; base += 64) {
+                        const uint64_t key =
+                            base + lane < e ? knn_key<D>(x, cpts[base + lane]) : kMaxKey;
                         knn_merge(key, top, kth, k);
                     }
                 }
@@ -177,7 +185,7 @@ __device__ void knn_rings(const CellGrid& G, const float4* cpts, const uint32_t*
 // keys took 11 wavefront sorts per query; here a candidate costs about 20
 // instructions once and only 64 keys are ordered, by counting smaller ones
 // (broadcast LDS reads, no shuffles).  1,030,301 cube nodes, k = 32: 14.4 ->
-// 1.7 ms; 1M random points 2.0 ms; 1M square nodes, k = 16: 0.8 ms.
+// 1.4 ms; 1M random points 1.7 ms; 1M square nodes, k = 16: 0.8 ms.
 constexpr int kKnnKeep = 256;   // points kept of one query (four per lane)
 constexpr int kKnnMaxBox = 4096;  // points of a box visited by one wavefront
 constexpr int kKnnBlockQueries = 16;  // queries per block: four per wavefront
@@ -239,6 +247,7 @@ __device__ bool knn_box(const CellGrid& G, double inv_w, const float4* __restric
                 open = true;
             }
         }
+        if (T == 0) return false;  // far from the cloud
         if (T < k || (open && bound <= 0.0)) {
             if (!open) return false;
             continue;
