@@ -194,13 +194,13 @@ int naga_batch_set_graph(naga_batch* b, int32_t on);  /* default on */
 /* Autotuner: times trial_steps steps of the batch for each gather batch
  * (neighbours gathered per unrolled step: 8, 16, 32), with and without
  * graph replay and, when the batch holds D2Q9 scenes, for each D2Q9 kernel
- * form (3 lanes per node on 84-node tiles reading the tile unions staged in
- * LDS, the same gathering directly, 9 lanes per node on 28-node tiles);
- * keeps the fastest, and restores every scene's state afterwards. */
+ * form (several distributions per lane on 128-node blocks, one per lane on
+ * 28-node blocks); keeps the fastest, and restores every scene's state afterwards. */
 int naga_batch_autotune(naga_batch* b, int32_t trial_steps, int32_t* gather_batch);
-/* D2Q9 kernel form of the batch's stencil passes: lanes per node 3
- * (default) or 9; unions 1 (default; lanes 3 only): scenes with tile
- * unions read them from LDS. */
+/* D2Q9 kernel form of the batch's stencil passes: lanes 9 is one lane per
+ * distribution, 3 (default) several distributions per lane.  unions (0 or,
+ * with lanes 3 only, 1, the default) is kept and reported: D2Q9 scenes gather
+ * their rows directly either way. */
 int naga_batch_set_q9_kernels(naga_batch* b, int32_t lanes, int32_t unions);
 /* The batch's current choices: gather batch (0: the kernels' default), D2Q9
  * lanes per node and unions, graph replay (1 or 0); null outputs are

@@ -1107,9 +1107,10 @@ class SceneBatch:
         return gb.value
 
     def set_q9_kernels(self, lanes: int, unions: bool | None = None):
-        """D2Q9 kernel form of the stencil passes: 3 or 9 lanes per node;
-        with 3, whether scenes with tile unions read them from LDS (default:
-        yes for 3 lanes, no for 9)."""
+        """D2Q9 kernel form of the stencil passes: 9, one lane per
+        distribution, or 3, several distributions per lane.  unions (only with
+        3, and by default with it) is kept and reported by tuning(); D2Q9
+        scenes gather their rows directly either way."""
         if unions is None:
             unions = int(lanes) == 3
         _check(load().naga_batch_set_q9_kernels(self._h, int(lanes), int(bool(unions))),

@@ -1110,10 +1110,13 @@ int naga_rk4_stage(int32_t q, int64_t n, int64_t n_fluid, int32_t k, const uint3
         hipStream_t s;
         NAGA_HIP(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
         try {
-            auto rows = [&](const float* src) {  // [n][q] -> [n][RS]
+            auto at = [&](int64_t i, int a) {  // place in a device row buffer
+                return size_t(q == 27 ? row_at<27>(i, a, n) : row_at<9>(i, a, n));
+            };
+            auto rows = [&](const float* src) {  // [n][q] -> device rows
                 std::vector<float> r(size_t(n) * RS, 0.0f);
                 for (int64_t i = 0; i < n; ++i)
-                    std::memcpy(&r[size_t(i) * RS], src + size_t(i) * q, sizeof(float) * q);
+                    for (int a = 0; a < q; ++a) r[at(i, a)] = src[size_t(i) * q + a];
                 return r;
             };
             DeviceBuffer<float> g(size_t(n) * RS), A(size_t(n) * RS), B(size_t(n) * RS),
@@ -1132,11 +1135,13 @@ int naga_rk4_stage(int32_t q, int64_t n, int64_t n_fluid, int32_t k, const uint3
             }
             DeviceBuffer<uint32_t> didx(std::max<int64_t>(n_fluid * k, 1));
             DeviceBuffer<float> dW(std::max<int64_t>(n_fluid * k * D, 1));
-            DeviceBuffer<float> slab(std::max<int64_t>(n_fluid * k * (1 + D), 1));
+            DeviceBuffer<float> slab(std::max<int64_t>(
+                n_fluid * (q == 9 ? 4 * q9_units(k, 2) : k * (1 + D)), 1));
             if (n_fluid) {
                 didx.upload(idx, size_t(n_fluid) * k, s);
                 dW.upload(W, size_t(n_fluid) * k * D, s);
-                launch_make_slab(n_fluid, k, D, didx.get(), dW.get(), slab.get(), s);
+                if (q == 9) launch_make_slab_q9(n_fluid, k, D, didx.get(), dW.get(), slab.get(), s);
+                else launch_make_slab(n_fluid, k, D, didx.get(), dW.get(), slab.get(), s);
             }
             StepGeom G{};
             G.N = n;
@@ -1163,7 +1168,7 @@ int naga_rk4_stage(int32_t q, int64_t n, int64_t n_fluid, int32_t k, const uint3
                                                                           s);
             NAGA_HIP(hipStreamSynchronize(s));
             for (int64_t i = 0; i < n; ++i)
-                std::memcpy(out + size_t(i) * q, &res[size_t(i) * RS], sizeof(float) * q);
+                for (int a = 0; a < q; ++a) out[size_t(i) * q + a] = res[at(i, a)];
         } catch (...) {
             (void)hipStreamDestroy(s);
             throw;

@@ -126,12 +126,6 @@ void Engine::require_domain() const {
     require(ready_, "init_domain must be called first");
 }
 
-// D2Q9 tile unions: built when NAGA_Q9_UNIONS=1 (off by default).
-static bool q9_unions_wanted(int64_t /*N*/) {
-    const char* e = std::getenv("NAGA_Q9_UNIONS");
-    return e && e[0] == '1';
-}
-
 void Engine::init_domain(const float* pts, int64_t nbulk, int64_t nlayer, int64_t nbnd,
                          const float* normals, const float* sigma) {
     require(batch == nullptr, "remove the engine from its batch before init_domain");
@@ -238,10 +232,17 @@ void Engine::init_domain(const float* pts, int64_t nbulk, int64_t nlayer, int64_
     filt_.allocate(N * k);
     launch_filter_weights(D, pts_.get(), N, idx_.get(), k, cfg_.h, filt_.get(), st, kvar_.get());
     if (kvar_.size() == size_t(N)) launch_self_past_k(N, k, kvar_.get(), idx_.get(), st);
-    slab_.allocate(nfluid * k * (1 + D));
-    launch_make_slab(nfluid, k, D, idx_.get(), W_.get(), slab_.get(), st);
-    fslab_.allocate(nfluid * k * 2);
-    launch_make_slab(nfluid, k, 1, idx_.get(), filt_.get(), fslab_.get(), st);
+    if (Q == 9) {
+        slab_.allocate(nfluid * q9_units(k, 2) * 4);
+        launch_make_slab_q9(nfluid, k, 2, idx_.get(), W_.get(), slab_.get(), st);
+        fslab_.allocate(nfluid * q9_units(k, 1) * 4);
+        launch_make_slab_q9(nfluid, k, 1, idx_.get(), filt_.get(), fslab_.get(), st);
+    } else {
+        slab_.allocate(nfluid * k * (1 + D));
+        launch_make_slab(nfluid, k, D, idx_.get(), W_.get(), slab_.get(), st);
+        fslab_.allocate(nfluid * k * 2);
+        launch_make_slab(nfluid, k, 1, idx_.get(), filt_.get(), fslab_.get(), st);
+    }
     ucap_ = 0;
     ucap_f_ = 0;
     self_first_ = 0;
@@ -259,8 +260,6 @@ void Engine::init_domain(const float* pts, int64_t nbulk, int64_t nlayer, int64_
     p2usplit_ = DeviceBuffer<int32_t>();
     p2split_tiles_ = DeviceBuffer<int32_t>();
     p2slab_ = DeviceBuffer<float>();
-    uslab_ = DeviceBuffer<float>();
-    ufslab_ = DeviceBuffer<float>();
     p2split_of_.clear();
     p2n_split_ = 0;
     bulist_ = DeviceBuffer<uint32_t>();
@@ -413,41 +412,6 @@ void Engine::init_domain(const float* pts, int64_t nbulk, int64_t nlayer, int64_
             slab_ = std::move(rs);
             fslab_ = std::move(rf);
         }
-    } else if (q9_unions_wanted(N) && !(un_env && un_env[0] == '0') && q9_three(Q, N) &&
-               nfluid > 0 && k * kQ9TileNodes <= 4096) {
-        // D2Q9 tile unions over the three-per-lane kernels' 84-node tiles
-        // (no split tiles: a tile whose union is over the cap reads its rows
-        // through the list).  Copies of the stage and filter records get
-        // union positions in their index fields (uslab, ufslab); the
-        // records with node indices stay for the PML divergence (a node
-        // list) and for batches that step D2Q9 scenes without unions.
-        const int T = kQ9TileNodes;
-        const int64_t ntiles = (nfluid + T - 1) / T;
-        uslab_.allocate(slab_.size());
-        ufslab_.allocate(fslab_.size());
-        NAGA_HIP(hipMemcpyAsync(uslab_.get(), slab_.get(), slab_.size() * sizeof(float),
-                                hipMemcpyDeviceToDevice, st));
-        NAGA_HIP(hipMemcpyAsync(ufslab_.get(), fslab_.get(), fslab_.size() * sizeof(float),
-                                hipMemcpyDeviceToDevice, st));
-        DeviceBuffer<int32_t> counts(ntiles);
-        launch_tile_unions(nfluid, k, T, idx_.get(), 0, counts.get(), nullptr, nullptr, nullptr,
-                           nullptr, 0, nullptr, 0, st);
-        std::vector<int32_t> hc(static_cast<size_t>(ntiles));
-        counts.download(hc.data(), size_t(ntiles), st);
-        NAGA_HIP(hipStreamSynchronize(st));
-        std::vector<int64_t> off(static_cast<size_t>(ntiles) + 1, 0);
-        int maxu = 0;
-        for (int64_t t = 0; t < ntiles; ++t) {
-            off[size_t(t) + 1] = off[size_t(t)] + hc[size_t(t)];
-            maxu = std::max(maxu, hc[size_t(t)]);
-        }
-        uoff_ = to_device(off, st);
-        ulist_.allocate(std::max<int64_t>(off[size_t(ntiles)], 1));
-        launch_tile_unions(nfluid, k, T, idx_.get(), 0, nullptr, nullptr, uoff_.get(),
-                           ulist_.get(), uslab_.get(), D, ufslab_.get(), 1, st);
-        NAGA_HIP(hipStreamSynchronize(st));
-        ucap_ = std::min(maxu, kQ9UnionRowsMax);
-        ucap_f_ = ucap_;
     }
 
     marks.mark();  // filter weights, slabs and tile unions done
@@ -630,8 +594,6 @@ StepBuffers Engine::buffers() {
     S.split_tiles = split_tiles_.get();
     S.n_split = n_split_;
     S.p2slab = p2slab_.get();
-    S.uslab = uslab_.get();
-    S.ufslab = ufslab_.get();
     S.p2ulist = p2ulist_.get();
     S.p2uoff = p2uoff_.get();
     S.p2usplit = p2usplit_.get();
@@ -768,7 +730,7 @@ void Engine::sample_probes(int set, bool fresh, double* values) {
     require(values != nullptr, "null output");
     ProbeSet& ps = *probes_[set];
     launch_probe(cfg_.Q, ps.n, ps.k, ps.idx.get(), ps.w.get(), fresh ? nullptr : rho_.get(),
-                 g_.get(), cfg_.rho0, ps.out.get(), stream_);
+                 g_.get(), N_, cfg_.rho0, ps.out.get(), stream_);
     ps.out.download(values, ps.n, stream_);
     NAGA_HIP(hipStreamSynchronize(stream_));
 }
@@ -818,7 +780,8 @@ struct StateHeader {
     int64_t N, frame;
     double time;
 };
-// version 02: the PML history is the previous step's (rho - 1, u) per node
+// version 02: the PML history is the previous step's (rho - 1, u) per node;
+// rows lie as RS floats per node whatever the device layout
 constexpr char kStateMagic[8] = {'N', 'A', 'G', 'A', 'S', 'T', '0', '2'};
 }  // namespace
 
@@ -843,7 +806,16 @@ void Engine::save_state(void* buf, int64_t capacity) {
     std::memcpy(p, &h, sizeof(h));
     p += sizeof(h);
     for (DeviceBuffer<float>* b : {&g_, &E_, &Qp_}) {
-        b->download(reinterpret_cast<float*>(p), b->size(), stream_);
+        if (cfg_.Q == 9 && b != &E_) {
+            std::vector<float> rows(b->size());
+            b->download(rows.data(), rows.size(), stream_);
+            NAGA_HIP(hipStreamSynchronize(stream_));
+            float* out = reinterpret_cast<float*>(p);
+            for (int64_t i = 0; i < N_; ++i)
+                for (int a = 0; a < 9; ++a) std::memcpy(out + i * 9 + a, &rows[row_of(i, a)], 4);
+        } else {
+            b->download(reinterpret_cast<float*>(p), b->size(), stream_);
+        }
         p += b->size() * sizeof(float);
     }
     rho_.download(reinterpret_cast<float*>(p), size_t(N_), stream_);
@@ -862,7 +834,16 @@ void Engine::load_state(const void* buf, int64_t bytes) {
     require(bytes >= state_bytes(), "state buffer truncated");
     const char* p = static_cast<const char*>(buf) + sizeof(h);
     for (DeviceBuffer<float>* b : {&g_, &E_, &Qp_}) {
-        b->upload(reinterpret_cast<const float*>(p), b->size(), stream_);
+        if (cfg_.Q == 9 && b != &E_) {
+            std::vector<float> rows(b->size());
+            const float* in = reinterpret_cast<const float*>(p);
+            for (int64_t i = 0; i < N_; ++i)
+                for (int a = 0; a < 9; ++a) std::memcpy(&rows[row_of(i, a)], in + i * 9 + a, 4);
+            b->upload(rows.data(), rows.size(), stream_);
+            NAGA_HIP(hipStreamSynchronize(stream_));
+        } else {
+            b->upload(reinterpret_cast<const float*>(p), b->size(), stream_);
+        }
         p += b->size() * sizeof(float);
     }
     rho_.upload(reinterpret_cast<const float*>(p), size_t(N_), stream_);
@@ -987,7 +968,7 @@ void Engine::profile_step(double* ms) {
 // ---------------------------------------------------------------------------
 // Batch
 // ---------------------------------------------------------------------------
-Batch::Batch() : q9_three_(q9_three(9, 1)) {
+Batch::Batch() : q9_pair_(q9_pair(9, 1)) {
     NAGA_HIP(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking));
 }
 
@@ -1034,14 +1015,14 @@ void Batch::set_graph(bool on) {
 void Batch::set_q9_kernels(int lanes, bool unions) {
     require(lanes == 3 || lanes == 9, "D2Q9 lanes per node must be 3 or 9");
     require(lanes == 3 || !unions, "D2Q9 tile unions need 3 lanes per node");
-    q9_three_ = lanes == 3;
+    q9_pair_ = lanes == 3;
     q9_unions_ = unions;
     dirty_ = true;
 }
 
 void Batch::tuning(int* gather_batch, int* q9_lanes, int* q9_unions, int* graph) const {
     if (gather_batch) *gather_batch = gather_batch_;
-    if (q9_lanes) *q9_lanes = q9_three_ ? 3 : 9;
+    if (q9_lanes) *q9_lanes = q9_pair_ ? 3 : 9;
     if (q9_unions) *q9_unions = q9_unions_ ? 1 : 0;
     if (graph) *graph = use_graph_ ? 1 : 0;
 }
@@ -1055,25 +1036,16 @@ int Batch::autotune(int trial_steps) {
     double best = 1e300;
     int best_gb = 8;
     bool best_graph = true;
-    std::pair<bool, bool> best_q9{q9_three_, q9_unions_};
-    bool any_q9 = false, any_q9_unions = false;
-    for (Engine* e : scenes_)
-        if (e->lattice() == 9) {
-            any_q9 = true;
-            any_q9_unions = any_q9_unions || e->scene_desc().S.ulist != nullptr;
-        }
-    // D2Q9 forms: (three per lane, unions); the union form where some
-    // scene has its tile unions built
-    std::vector<std::pair<bool, bool>> q9_forms{best_q9};
-    if (any_q9) q9_forms = {{true, false}, {false, false}};
-    if (any_q9_unions) q9_forms.push_back({true, true});
-    for (const auto& form : q9_forms)
+    bool best_q9 = q9_pair_, any_q9 = false;
+    for (Engine* e : scenes_) any_q9 = any_q9 || e->lattice() == 9;
+    std::vector<bool> q9_forms{best_q9};
+    if (any_q9) q9_forms = {true, false};
+    for (const bool form : q9_forms)
         for (int gb : {8, 16, 32})
             for (bool graph : {true, false}) {
                 gather_batch_ = gb;
                 use_graph_ = graph;
-                q9_three_ = form.first;
-                q9_unions_ = form.second;
+                q9_pair_ = form;
                 dirty_ = true;
                 step(1);  // builds the plan (and captures the graph)
                 const double ms = step_timed(trial_steps);
@@ -1086,8 +1058,8 @@ int Batch::autotune(int trial_steps) {
             }
     gather_batch_ = best_gb;
     use_graph_ = best_graph;
-    q9_three_ = best_q9.first;
-    q9_unions_ = best_q9.second;
+    q9_pair_ = best_q9;
+    if (any_q9) q9_unions_ = false;
     dirty_ = true;
     for (size_t i = 0; i < scenes_.size(); ++i) scenes_[i]->restore(saved[i]);
     return best_gb;
@@ -1102,23 +1074,18 @@ void Batch::rebuild() {
     any_sources_ = false;
     // groups: lattice, four-per-lane stencil width, and whether the tile
     // unions (and their padded slab layout) were built
-    auto three_of = [this](Engine* e) {
-        return e->lattice() == 9 && q9_three_ && q9_three_fits(e->nodes());
+    auto pair_of = [this](Engine* e) {
+        return e->lattice() == 9 && q9_pair_ && q9_pair_fits(e->nodes());
     };
-    // whether the scene's passes read its tile unions: D3Q27 scenes with
-    // unions always (their records hold union positions); D2Q9 scenes
-    // with unions when the batch runs them three per lane with unions
-    auto tiles_of = [&](Engine* e) {
-        const bool built = e->scene_desc().S.ulist != nullptr;
-        return e->lattice() == 27 ? built : built && three_of(e) && q9_unions_;
-    };
+    // scenes with tile unions (D3Q27): their records hold union positions
+    auto tiles_of = [](Engine* e) { return e->scene_desc().S.ulist != nullptr; };
     auto key_of = [&](Engine* e) {
         const int Q = e->lattice();
         const bool un = step_uses_unions(Q, e->stencil_k(), e->nodes());
         const bool tiles = tiles_of(e);
-        const bool three = three_of(e);
+        const bool pair = pair_of(e);
         const bool ragged = e->scene_desc().S.tile_ng != nullptr;
-        return Q * 1000 + (un ? e->stencil_k() : 0) + (tiles ? 500 : 0) + (three ? 250 : 0) +
+        return Q * 1000 + (un ? e->stencil_k() : 0) + (tiles ? 500 : 0) + (pair ? 250 : 0) +
                (ragged ? 125 : 0);
     };
     std::vector<int> keys;
@@ -1130,7 +1097,7 @@ void Batch::rebuild() {
             keys.push_back(key);
             groups_.push_back(std::make_unique<Group>());
             groups_.back()->Q = e->lattice();
-            groups_.back()->three = three_of(e);
+            groups_.back()->pair = pair_of(e);
             groups_.back()->tiles = tiles_of(e);
         }
         groups_[g]->members.push_back(e);
@@ -1144,7 +1111,7 @@ void Batch::rebuild() {
         P = BatchPlan{};
         P.Q = g.Q;
         P.nscenes = n;
-        P.three = g.three;
+        P.pair = g.pair;
         int kcommon = g.members[0]->stencil_k();
         for (int s = 0; s < n; ++s) {
             Engine* e = g.members[s];
@@ -1155,7 +1122,7 @@ void Batch::rebuild() {
             P.kmax = std::max(P.kmax, e->stencil_k());
             any_sources_ = any_sources_ || descs[s].S.src != nullptr;
             int64_t nb[kStepKernels];
-            step_block_counts(g.Q, descs[s].G, descs[s].S, nb, g.three ? 1 : 0);
+            step_block_counts(g.Q, descs[s].G, descs[s].S, nb, g.pair ? 1 : 0);
             for (int p = 0; p < kStepKernels; ++p) {
                 int32_t* row = bstart.data() + size_t(p) * (n + 1);
                 const int64_t next = int64_t(row[s]) + nb[p];
@@ -1170,8 +1137,7 @@ void Batch::rebuild() {
         P.tiles = g.tiles;
         P.ragged = descs[0].S.tile_ng != nullptr;
         for (const SceneDesc& d : descs)
-            require(g.Q == 9 ? (!P.tiles || d.S.ulist != nullptr) : (d.S.ulist != nullptr) == P.tiles,
-                    "scenes with and without tile unions");
+            require((d.S.ulist != nullptr) == P.tiles, "scenes with and without tile unions");
         require(!P.unions || P.k_template != 0, "four-per-lane scenes need a common k");
         g.table = to_device(descs, stream_);
         g.bstart = to_device(bstart, stream_);
@@ -1276,7 +1242,7 @@ void Engine::get_distributions(double* f, double* g) {
     for (int a = 0; a < Q; ++a) {
         const double w = weight(Q, a);
         for (int64_t i = 0; i < N_; ++i) {
-            const double v = double(rows[size_t(i) * RS_ + a]);
+            const double v = double(rows[row_of(i, a)]);
             if (g) g[a * N_ + i] = v;
             if (f) f[a * N_ + i] = w + v;
         }
@@ -1289,7 +1255,7 @@ void Engine::set_distributions(const double* f) {
     std::vector<float> rows(size_t(N_) * RS_, 0.0f);
     for (int a = 0; a < Q; ++a) {
         const double w = weight(Q, a);
-        for (int64_t i = 0; i < N_; ++i) rows[size_t(i) * RS_ + a] = float(f[a * N_ + i] - w);
+        for (int64_t i = 0; i < N_; ++i) rows[row_of(i, a)] = float(f[a * N_ + i] - w);
     }
     g_.upload(rows.data(), rows.size(), stream_);
     refresh_macroscopic_state();
@@ -1311,7 +1277,7 @@ void Engine::set_pulse(const double* center, double amp, double width) {
             r2 += t * t;
         }
         const double p = amp * std::exp(-r2 / (2.0 * width * width));
-        for (int a = 0; a < Q; ++a) rows[size_t(i) * RS_ + a] = float(weight(Q, a) * p);
+        for (int a = 0; a < Q; ++a) rows[row_of(i, a)] = float(weight(Q, a) * p);
     }
     g_.upload(rows.data(), rows.size(), stream_);
     refresh_macroscopic_state();
@@ -1467,7 +1433,7 @@ void Engine::get_pml(double* E, double* Qp) {
         for (int64_t i = 0; i < N_; ++i) {
             if (E) E[a * N_ + i] = Q == 27 ? feq_dev_host<27>(&e[size_t(i) * 4], a)
                                            : feq_dev_host<9>(&e[size_t(i) * 4], a);
-            if (Qp) Qp[a * N_ + i] = double(q[size_t(i) * RS_ + a]);
+            if (Qp) Qp[a * N_ + i] = double(q[row_of(i, a)]);
         }
 }
 

@@ -106,6 +106,10 @@ class Engine {
 
   private:
     void require_domain() const;
+    // place of distribution a of node i in a host copy of a row buffer
+    size_t row_of(int64_t i, int a) const {
+        return size_t(cfg_.Q == 27 ? row_at<27>(i, a, N_) : row_at<9>(i, a, N_));
+    }
     void launch_one_step(hipEvent_t* ev);
     // nsteps steps on the stream: one step captured once into a hipGraph and
     // replayed (no density sources; NAGA_ENGINE_GRAPH=0 disables), else
@@ -167,7 +171,6 @@ class Engine {
     // boundary-interpolation tiles: their distinct source nodes
     DeviceBuffer<uint32_t> bulist_;
     DeviceBuffer<int64_t> buoff_;
-    DeviceBuffer<float> uslab_, ufslab_;  // D2Q9 records with union positions
     int ucap_ = 0;
     int ucap_f_ = 0;
     int self_first_ = 0;
@@ -209,15 +212,14 @@ class Batch {
     void set_graph(bool on);
     // Times trial_steps steps for each gather batch (8, 16, 32), with and
     // without graph replay, and, when the batch holds D2Q9 scenes, for each
-    // D2Q9 kernel form: three distributions per lane (3 lanes per node,
-    // 84-node tiles) reading the tile unions staged in LDS, the same
-    // gathering directly, or one distribution per lane (9 lanes per node,
-    // 28-node tiles); keeps the fastest and restores every scene's state
-    // (the trials do not advance the scenes).  Returns the chosen gather
-    // batch, or 0 if the batch is empty.
+    // D2Q9 kernel form: two lanes per node (128-node blocks) or one lane per
+    // distribution (9 per node, 28-node blocks); keeps the fastest and
+    // restores every scene's state (the trials do not advance the scenes).
+    // Returns the chosen gather batch, or 0 if the batch is empty.
     int autotune(int trial_steps);
-    // D2Q9 kernel form: lanes per node 3 or 9; unions (lanes 3 only): read
-    // the tile unions in LDS where the scene has them.
+    // D2Q9 kernel form: lanes 9, one lane per distribution, or 3, several
+    // distributions per lane.  unions (with 3 only) is kept and reported;
+    // D2Q9 scenes gather their rows directly either way.
     void set_q9_kernels(int lanes, bool unions);
     // The current choices: gather batch (0: the kernels' default), D2Q9
     // lanes per node and unions, graph replay.
@@ -232,8 +234,8 @@ class Batch {
   private:
     struct Group {
         int Q = 9;
-        bool three = false;  // D2Q9 with three distributions per lane
-        bool tiles = false;  // the members' tile unions are read (D3Q27: always with them)
+        bool pair = false;   // D2Q9 with two lanes per node
+        bool tiles = false;  // the members have tile unions
         std::vector<Engine*> members;
         BatchPlan plan;
         DeviceBuffer<SceneDesc> table;
@@ -250,8 +252,8 @@ class Batch {
     bool use_graph_ = true;
     bool any_sources_ = false;
     int gather_batch_ = 0;
-    bool q9_three_ = true;   // D2Q9 scenes with three distributions per lane
-    bool q9_unions_ = true;  // ... reading their tile unions in LDS
+    bool q9_pair_ = true;    // D2Q9 scenes with two lanes per node
+    bool q9_unions_ = true;  // as set (reported only)
     hipGraph_t graph_ = nullptr;
     hipGraphExec_t exec_ = nullptr;
 };

@@ -47,7 +47,7 @@ struct Lattice {
     static_assert(Q_ == 9 || Q_ == 27, "D2Q9 and D3Q27 only");
     static constexpr int Q = Q_;
     static constexpr int D = Q_ == 9 ? 2 : 3;
-    // AoS row stride (floats) of per-node distribution rows in HBM.  D3Q27
+    // Floats per node of the distribution buffers in HBM (row_at).  D3Q27
     // rows are padded to one 128-byte line so a neighbour gather touches a
     // single line.
     static constexpr int RS = Q_ == 27 ? 32 : 9;

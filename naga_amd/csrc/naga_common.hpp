@@ -50,8 +50,13 @@ inline void require(bool ok, const std::string& msg) {
 // makes the row length odd in units so the records of consecutive nodes
 // fall in distinct LDS banks.  k must be a multiple of 8.
 constexpr int packed_div_units(int k) { return 7 * (k / 8) + 1; }
-// Filter records of a node with tile unions, packed the same way: per group
-// of 8 records two units of weights and one unit of 16-bit positions, then
+// 16-byte units of one D2Q9 node's records (launch_make_slab_q9): per group of
+// four records one unit of indices and one per weight; and the LDS row that
+// holds them, an odd number of units (distinct banks for consecutive nodes).
+NAGA_HD constexpr int q9_units(int k, int ncomp) { return (1 + ncomp) * ((k + 3) / 4); }
+NAGA_HD constexpr int q9_pitch(int units) { return units | 1; }
+// Filter records of a node with tile unions, packed like the divergence
+// records: per group of 8 records two units of weights and one unit of 16-bit positions, then
 // one zero unit.
 constexpr int packed_filter_units(int k) { return 3 * (k / 8) + 1; }
 // Record rows of a tile whose nodes use ng groups of 8 records (per-tile

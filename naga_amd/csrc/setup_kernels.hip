@@ -866,6 +866,20 @@ __global__ void k_make_slab(int64_t n, int k, int nc, const uint32_t* idx,
     for (int c = 0; c < nc; ++c) r[1 + c] = w[t * nc + c];
 }
 
+// One thread per (node, 32-bit word) of the D2Q9 records.
+__global__ void k_make_slab_q9(int64_t n, int k, int nc, const uint32_t* idx, const float* w,
+                               uint32_t* slab) {
+    const int words = 4 * q9_units(k, nc);
+    const int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (t >= n * words) return;
+    const int64_t i = t / words;
+    const int u = int(t - i * words) / 4, f = u % (1 + nc);  // field: index, weights
+    const int s = u / (1 + nc) * 4 + int(t % 4);             // record (words is a multiple of 4)
+    uint32_t v = f == 0 ? uint32_t(i) : 0u;
+    if (s < k) v = f == 0 ? idx[i * k + s] : __float_as_uint(w[(i * k + s) * nc + f - 1]);
+    slab[t] = v;
+}
+
 // One thread per (node, 32-bit word) of the packed divergence records.
 __global__ void k_pack_div_records(int64_t n, int k, const float* src, uint32_t* dst) {
     const int units = packed_div_units(k);
@@ -1534,6 +1548,15 @@ void launch_make_slab(int64_t n, int k, int nc, const uint32_t* idx, const float
                       float* slab, hipStream_t st) {
     if (n == 0) return;
     k_make_slab<<<(n * k + 255) / 256, 256, 0, st>>>(n, k, nc, idx, w, slab);
+    hip_check(hipGetLastError(), "slab");
+}
+
+void launch_make_slab_q9(int64_t n, int k, int nc, const uint32_t* idx, const float* w,
+                         float* slab, hipStream_t st) {
+    if (n == 0) return;
+    const int64_t tot = n * q9_units(k, nc) * 4;
+    k_make_slab_q9<<<(tot + 255) / 256, 256, 0, st>>>(n, k, nc, idx, w,
+                                                      reinterpret_cast<uint32_t*>(slab));
     hip_check(hipGetLastError(), "slab");
 }
 

@@ -151,6 +151,12 @@ void launch_filter_weights(int D, const float* pts, int64_t n,
 void launch_make_slab(int64_t n, int k, int ncomp, const uint32_t* idx,
                       const float* w, float* slab, hipStream_t stream);
 
+// D2Q9 records: per node ceil(k / 4) groups of four records, each group four
+// indices and then the four values of each of the ncomp weights (q9_units
+// 16-byte units per node); entries past k hold the node itself, weights zero.
+void launch_make_slab_q9(int64_t n, int k, int ncomp, const uint32_t* idx, const float* w,
+                         float* slab, hipStream_t stream);
+
 // Packs D3Q27 divergence records ({union position bits, wx, wy, wz} per
 // stencil entry, k per node) into the packed_div_units layout.
 void launch_pack_div_records(int64_t n, int k, const float* src, float* dst, hipStream_t st);

@@ -94,7 +94,7 @@ template <int Q, class Row>
 __device__ __forceinline__ float4 p1_node(const StepGeom& G, const StepBuffers& S,
                                           const CollisionParams& cp, int64_t i, Row r) {
     using L = Lattice<Q>;
-    constexpr int D = L::D, RS = L::RS;
+    constexpr int D = L::D;
     double f[Q];
     double rt = 0.0, mom[3] = {0.0, 0.0, 0.0};
 #pragma unroll
@@ -130,16 +130,14 @@ __device__ __forceinline__ float4 p1_node(const StepGeom& G, const StepBuffers& 
     for (int a = 0; a < Q; ++a) {
         const double v = bnd ? df[a] : double(r.get(a)) + L::w(a) * ws + df[a];
         r.set(a, float(v));
-        if (src_node) S.coll[i * RS + a] = float(df[a]);
+        if (src_node) S.coll[row_at<Q>(i, a, G.N)] = float(df[a]);
     }
     return ru;
 }
 
-template <int Q>
-__global__ __launch_bounds__(kP1Block) void k_p1(StepGeom G, StepBuffers S,
-                                                 CollisionParams cp, BatchArgs B) {
-    using L = Lattice<Q>;
-    constexpr int RS = L::RS, LS = RS + 1;
+__global__ __launch_bounds__(kP1Block) void k_p1_27(StepGeom G, StepBuffers S,
+                                                    CollisionParams cp, BatchArgs B) {
+    constexpr int RS = Lattice<27>::RS, LS = RS + 1;
     __shared__ float rows[kP1Block * LS];
     const BlockCtx bc = locate(B, G, S);
     if (B.scenes) cp = B.scenes[bc.scene].cp;
@@ -150,10 +148,38 @@ __global__ __launch_bounds__(kP1Block) void k_p1(StepGeom G, StepBuffers S,
     for (int e = threadIdx.x; e < cnt * RS; e += kP1Block) rows[(e / RS) * LS + e % RS] = src[e];
     __syncthreads();
     const int t = threadIdx.x;
-    if (t < cnt) S.ru[node0 + t] = p1_node<Q>(G, S, cp, node0 + t, FlatRow{rows + t * LS});
+    if (t < cnt) S.ru[node0 + t] = p1_node<27>(G, S, cp, node0 + t, FlatRow{rows + t * LS});
     __syncthreads();
     float* dst = S.A + node0 * RS;
     for (int e = threadIdx.x; e < cnt * RS; e += kP1Block) dst[e] = rows[(e / RS) * LS + e % RS];
+}
+
+// D2Q9: a node's row is two 16-byte pieces and its rest value, read and
+// written by its own thread (consecutive lanes, consecutive rows).
+__device__ __forceinline__ void load_row9(const float* p, int64_t i, int64_t N, float (&v)[9]) {
+    const float4* row = reinterpret_cast<const float4*>(p) + 2 * i;
+    const float4 a = row[0], b = row[1];
+    v[0] = p[8 * N + i];
+    v[1] = a.x, v[2] = a.y, v[3] = a.z, v[4] = a.w;
+    v[5] = b.x, v[6] = b.y, v[7] = b.z, v[8] = b.w;
+}
+__device__ __forceinline__ void store_row9(float* p, int64_t i, int64_t N, const float (&v)[9]) {
+    float4* row = reinterpret_cast<float4*>(p) + 2 * i;
+    row[0] = make_float4(v[1], v[2], v[3], v[4]);
+    row[1] = make_float4(v[5], v[6], v[7], v[8]);
+    p[8 * N + i] = v[0];
+}
+
+__global__ __launch_bounds__(kP1Block) void k_p1_9(StepGeom G, StepBuffers S, CollisionParams cp,
+                                                   BatchArgs B) {
+    const BlockCtx bc = locate(B, G, S);
+    if (B.scenes) cp = B.scenes[bc.scene].cp;
+    const int64_t i = bc.b * kP1Block + threadIdx.x;
+    if (i >= G.N) return;
+    float v[9];
+    load_row9(S.g, i, G.N, v);
+    S.ru[i] = p1_node<9>(G, S, cp, i, FlatRow{v});
+    store_row9(S.A, i, G.N, v);
 }
 
 // ---------------------------------------------------------------------------
@@ -204,7 +230,6 @@ __device__ __forceinline__ float feq_dev32(const float4& ru, int a) {
 template <int Q>
 __global__ __launch_bounds__(kBlock) void k_pml_local(StepGeom G, StepBuffers S, BatchArgs B) {
     using L = Lattice<Q>;
-    constexpr int RS = L::RS;
     constexpr int NPB = kBlock / 64 * L::NPW;
     __shared__ double red[NPB][2][Q];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -225,7 +250,7 @@ __global__ __launch_bounds__(kBlock) void k_pml_local(StepGeom G, StepBuffers S,
         // feq - w now and at the previous step's macroscopic values
         const double fte = feq_dev<Q>(ru, a);
         const double ftp = feq_dev<Q>(*prev, a);
-        const int64_t o = i * RS + a;
+        const int64_t o = row_at<Q>(i, a, G.N);
         const double q1 = (fte + ftp) * hdt;
         const double q2 = (q1 + double(S.Qp[o])) * hdt;
         // the node's lanes (one wavefront) have read prev: the store waits
@@ -283,8 +308,6 @@ __global__ __launch_bounds__(256) void k_means(StepGeom G, StepBuffers S, BatchA
 // zero, so the divergence pass needs no branch.
 template <int Q>
 __global__ __launch_bounds__(kBlock) void k_pml_field(StepGeom G, StepBuffers S, BatchArgs B) {
-    using L = Lattice<Q>;
-    constexpr int RS = L::RS;
     const BlockCtx bc = locate(B, G, S);
     const LaneMap<Q> m(xcd_tile(bc.b, bc.nb));
     if (m.node >= G.nlayer || !m.active) return;
@@ -292,8 +315,9 @@ __global__ __launch_bounds__(kBlock) void k_pml_field(StepGeom G, StepBuffers S,
     const int64_t p = G.pml_ref ? j - G.nbulk : j;
     const int a = m.a;
     const float sig = S.sigma[m.node];
-    const float q1 = S.Qp[p * RS + a], q2 = S.Q2v[p * RS + a];
-    S.Gf[j * RS + a] =
+    const int64_t o = row_at<Q>(p, a, G.N);
+    const float q1 = S.Qp[o], q2 = S.Q2v[o];
+    S.Gf[row_at<Q>(j, a, G.N)] =
         -2.0f * sig * (q1 - S.means[a]) + sig * sig * (q2 - S.means[means_stride(Q) + a]);
 }
 
@@ -309,35 +333,35 @@ struct Tile {
     static constexpr int NPB = kBlock / 64 * Lattice<Q>::NPW;  // node slots
 };
 
-// Copy the records of nodes [node0, node0 + cnt) (contiguous slab rows of
-// K*REC floats) into lds.
-template <int REC>
-__device__ __forceinline__ void stage_contiguous(const float* slab, int64_t node0, int cnt,
-                                                 int K, float* lds) {
-    const float* src = slab + node0 * int64_t(K) * REC;
-    const int tot = cnt * K * REC;
-    if (REC == 4) {
-        const float4* s4 = reinterpret_cast<const float4*>(src);
-        float4* d4 = reinterpret_cast<float4*>(lds);
-        for (int t = threadIdx.x; t < tot / 4; t += kBlock) d4[t] = s4[t];
-    } else if (REC == 2) {
-        const float2* s2 = reinterpret_cast<const float2*>(src);
-        float2* d2 = reinterpret_cast<float2*>(lds);
-        for (int t = threadIdx.x; t < tot / 2; t += kBlock) d2[t] = s2[t];
-    } else {
-        for (int t = threadIdx.x; t < tot; t += kBlock) lds[t] = src[t];
-    }
+// Floats of one node's record row for stencil width K and NC weights per
+// record: D3Q27 {index, weights} per record; D2Q9 groups of four records,
+// four indices and then the four values of each weight (q9_units).
+template <int Q, int NC>
+__device__ __forceinline__ int rec_floats(int K) {
+    return Q == 27 ? K * (1 + NC) : 4 * q9_units(K, NC);
+}
+// Field f (0: index) of record s in the row r.
+template <int Q, int NC>
+__device__ __forceinline__ float rec_field(const float* r, int s, int f) {
+    return Q == 27 ? r[s * (1 + NC) + f] : r[((s >> 2) * (1 + NC) + f) * 4 + (s & 3)];
+}
+
+// Copy the record rows (RW floats, a multiple of two) of nodes [node0, node0
+// + cnt) into lds.
+__device__ __forceinline__ void stage_contiguous(const float* slab, int64_t node0, int cnt, int RW,
+                                                 float* lds) {
+    const float2* s2 = reinterpret_cast<const float2*>(slab + node0 * int64_t(RW));
+    float2* d2 = reinterpret_cast<float2*>(lds);
+    for (int t = threadIdx.x; t < cnt * RW / 2; t += kBlock) d2[t] = s2[t];
 }
 
 // Copy the records of one node (lanes of the node share the work).
-template <int Q, int REC>
-__device__ __forceinline__ void stage_node(const float* slab, int64_t node, bool valid, int K,
+template <int Q>
+__device__ __forceinline__ void stage_node(const float* slab, int64_t node, bool valid, int RW,
                                            int a_lane, float* lds) {
     if (!valid) return;
-    const float* src = slab + node * int64_t(K) * REC;
-    for (int r = a_lane; r < K; r += Lattice<Q>::LPN)
-#pragma unroll
-        for (int c = 0; c < REC; ++c) lds[r * REC + c] = src[r * REC + c];
+    const float* src = slab + node * int64_t(RW);
+    for (int t = a_lane; t < RW; t += Lattice<Q>::LPN) lds[t] = src[t];
 }
 
 template <int Q>
@@ -356,12 +380,15 @@ struct Lanes {
     }
 };
 
-// sum_s (c_a . W_s) fin(idx_s)_a over the staged records rp (REC = 1 + D),
-// batches of 8 neighbours.
+// sum_s (c_a . W_s) fin(idx_s)_a over the staged records rp, batches of 8
+// neighbours.
 template <int Q, int KT, int BATCH = 8>
-__device__ __forceinline__ float stencil_sum(const float* rp, int K, const float* fin, int a) {
+__device__ __forceinline__ float stencil_sum(const float* rp, int K, const float* fin, int64_t N,
+                                             int a) {
     using L = Lattice<Q>;
-    constexpr int D = L::D, RS = L::RS, REC = 1 + D, KMAX = KT ? KT : 64;
+    constexpr int D = L::D, KMAX = KT ? KT : 64;
+    const float* col = fin + row_at<Q>(0, a, N);  // distribution a of node 0
+    const int64_t pitch = row_pitch<Q>(a);
     const float cx = lane_c<Q>(a, 0), cy = lane_c<Q>(a, 1),
                 cz = D == 3 ? lane_c<Q>(a, 2) : 0.0f;
     float acc = 0.0f;
@@ -374,14 +401,14 @@ __device__ __forceinline__ float stencil_sum(const float* rp, int K, const float
         for (int u = 0; u < BATCH; ++u) {
             const int s = s0 + u;
             const bool in = KT ? (s < KT) : (s < K);
-            const float* r = rp + (in ? s : 0) * REC;
-            j[u] = __float_as_uint(r[0]);
-            float w = cx * r[1] + cy * r[2];
-            if (D == 3) w += cz * r[3];
+            const int t = in ? s : 0;
+            j[u] = __float_as_uint(rec_field<Q, D>(rp, t, 0));
+            float w = cx * rec_field<Q, D>(rp, t, 1) + cy * rec_field<Q, D>(rp, t, 2);
+            if (D == 3) w += cz * rec_field<Q, D>(rp, t, 3);
             v[u] = in ? w : 0.0f;
         }
 #pragma unroll
-        for (int u = 0; u < BATCH; ++u) gv[u] = fin[int64_t(j[u]) * RS + a];
+        for (int u = 0; u < BATCH; ++u) gv[u] = col[int64_t(j[u]) * pitch];
 #pragma unroll
         for (int u = 0; u < BATCH; ++u) acc += v[u] * gv[u];
     }
@@ -396,7 +423,7 @@ __device__ __forceinline__ float stencil_sum(const float* rp, int K, const float
 template <int Q, int KT>
 __global__ __launch_bounds__(kBlock) void k_p2(StepGeom G, StepBuffers S, BatchArgs B) {
     using L = Lattice<Q>;
-    constexpr int D = L::D, RS = L::RS, REC = 1 + D, KMAX = KT ? KT : 64;
+    constexpr int D = L::D, REC = 1 + D, KMAX = KT ? KT : 64;
     constexpr int NPB = Tile<Q>::NPB;
     __shared__ float srec[NPB * KMAX * REC];
     const BlockCtx bc = locate(B, G, S);
@@ -405,12 +432,13 @@ __global__ __launch_bounds__(kBlock) void k_p2(StepGeom G, StepBuffers S, BatchA
     const int64_t item = xcd_tile(bc.b, bc.nb) * NPB + ln.slot;
     const bool valid = item < S.n_pml;
     const int64_t i = valid ? S.pml_list[item] : 0;
-    float* rp = srec + ln.slot * K * REC;
-    stage_node<Q, REC>(S.slab, i, valid && ln.in_wave, K, ln.al, rp);
+    const int RW = rec_floats<Q, D>(K);
+    float* rp = srec + ln.slot * RW;
+    stage_node<Q>(S.slab, i, valid && ln.in_wave, RW, ln.al, rp);
     __syncthreads();
     if (!valid) return;
-    const float acc = stencil_sum<Q, KT>(rp, K, S.Gf, ln.a);
-    if (ln.active) S.A[i * RS + ln.a] += acc;
+    const float acc = stencil_sum<Q, KT>(rp, K, S.Gf, G.N, ln.a);
+    if (ln.active) S.A[row_at<Q>(i, ln.a, G.N)] += acc;
 }
 
 // ---------------------------------------------------------------------------
@@ -423,8 +451,6 @@ __global__ __launch_bounds__(kBlock) void k_p2(StepGeom G, StepBuffers S, BatchA
 // ---------------------------------------------------------------------------
 template <int Q, bool ACCUMULATE>
 __global__ __launch_bounds__(kBlock) void k_binterp(StepGeom G, StepBuffers S, BatchArgs B) {
-    using L = Lattice<Q>;
-    constexpr int RS = L::RS;
     const BlockCtx bc = locate(B, G, S);
     float* field = ACCUMULATE ? S.A : S.g;
     const float* bslab = S.bslab;
@@ -437,11 +463,12 @@ __global__ __launch_bounds__(kBlock) void k_binterp(StepGeom G, StepBuffers S, B
     float acc = 0.0f;
     for (int s = 0; s < G.kb; ++s) {
         const int64_t j = int64_t(__float_as_uint(rec[2 * s]));
-        const float v = ACCUMULATE ? field[j * RS + a] - coll[j * RS + a] : field[j * RS + a];
+        const int64_t o = row_at<Q>(j, a, G.N);
+        const float v = ACCUMULATE ? field[o] - coll[o] : field[o];
         acc += rec[2 * s + 1] * v;
     }
-    const int64_t b = G.nfluid + m.node;
-    if (m.active) field[b * RS + a] = ACCUMULATE ? field[b * RS + a] + acc : acc;
+    const int64_t b = row_at<Q>(G.nfluid + m.node, a, G.N);
+    if (m.active) field[b] = ACCUMULATE ? field[b] + acc : acc;
 }
 
 // ---------------------------------------------------------------------------
@@ -452,24 +479,27 @@ __global__ __launch_bounds__(kBlock) void k_binterp(StepGeom G, StepBuffers S, B
 template <int Q, int KT>
 __global__ __launch_bounds__(kBlock) void k_p4(StepGeom G, StepBuffers S, BatchArgs B) {
     using L = Lattice<Q>;
-    constexpr int D = L::D, RS = L::RS, KMAX = KT ? KT : 64;
+    constexpr int D = L::D, KMAX = KT ? KT : 64;
     constexpr int NPB = Tile<Q>::NPB;
     __shared__ float srec[NPB * KMAX * 2];
     const BlockCtx bc = locate(B, G, S);
     const int K = KT ? KT : G.k;
     const int64_t node0 = xcd_tile(bc.b, bc.nb) * NPB;
     const int64_t nf = G.nfluid - node0;
-    stage_contiguous<2>(S.fslab, node0, nf <= 0 ? 0 : (nf < NPB ? int(nf) : NPB), K, srec);
+    const int RW = rec_floats<Q, 1>(K);
+    stage_contiguous(S.fslab, node0, nf <= 0 ? 0 : (nf < NPB ? int(nf) : NPB), RW, srec);
     __syncthreads();
     const Lanes<Q> ln;
     const int64_t i = node0 + ln.slot;
     if (i >= G.N) return;
     const int a = ln.a;
     const float* s1 = S.A;
+    const float* col = s1 + row_at<Q>(0, a, G.N);
+    const int64_t pitch = row_pitch<Q>(a);
     float out;
     if (i < G.nfluid) {
-        const float si = s1[i * RS + a];
-        const float* rp = srec + ln.slot * K * 2;
+        const float si = col[i * pitch];
+        const float* rp = srec + ln.slot * RW;
         float sum = 0.0f;
 #pragma unroll
         for (int s0 = 0; s0 < KMAX; s0 += 8) {
@@ -480,11 +510,11 @@ __global__ __launch_bounds__(kBlock) void k_p4(StepGeom G, StepBuffers S, BatchA
             for (int u = 0; u < 8; ++u) {
                 const int s = s0 + u;
                 const bool in = KT ? (s < KT) : (s < K);
-                j[u] = __float_as_uint(rp[(in ? s : 0) * 2]);
-                w[u] = in ? rp[s * 2 + 1] : 0.0f;
+                j[u] = __float_as_uint(rec_field<Q, 1>(rp, in ? s : 0, 0));
+                w[u] = in ? rec_field<Q, 1>(rp, s, 1) : 0.0f;
             }
 #pragma unroll
-            for (int u = 0; u < 8; ++u) gv[u] = s1[int64_t(j[u]) * RS + a];
+            for (int u = 0; u < 8; ++u) gv[u] = col[int64_t(j[u]) * pitch];
 #pragma unroll
             for (int u = 0; u < 8; ++u) sum += w[u] * (gv[u] - si);
         }
@@ -495,9 +525,9 @@ __global__ __launch_bounds__(kBlock) void k_p4(StepGeom G, StepBuffers S, BatchA
 #pragma unroll
         for (int d = 0; d < D; ++d) cn += lane_c<Q>(a, d) * S.normals[b * D + d];
         const int src = cn > 0.0f ? L::bb(a) : a;
-        out = s1[i * RS + src];
+        out = s1[row_at<Q>(i, src, G.N)];
     }
-    if (ln.active) S.g[i * RS + a] = out;
+    if (ln.active) S.g[row_at<Q>(i, a, G.N)] = out;
 }
 
 // ---------------------------------------------------------------------------
@@ -559,7 +589,7 @@ __device__ __forceinline__ float4 rk4_out4(const float4& y, const float4& k, flo
 template <int Q, int STAGE, int KT, int BATCH>
 __global__ __launch_bounds__(kBlock) void k_stage(StepGeom G, StepBuffers S, BatchArgs B) {
     using L = Lattice<Q>;
-    constexpr int D = L::D, RS = L::RS, REC = 1 + D, KMAX = KT ? KT : 64;
+    constexpr int D = L::D, REC = 1 + D, KMAX = KT ? KT : 64;
     constexpr int NPB = Tile<Q>::NPB;
     __shared__ float srec[NPB * KMAX * REC];
     const BlockCtx bc = locate(B, G, S);
@@ -568,7 +598,7 @@ __global__ __launch_bounds__(kBlock) void k_stage(StepGeom G, StepBuffers S, Bat
     const Lanes<Q> ln;
     const int64_t i = node0 + ln.slot;
     const int a = ln.a;
-    const int64_t o = i * RS + a;
+    const int64_t o = row_at<Q>(i, a, G.N);
     const float* gin = stage_in(S, STAGE);
     float* gout = stage_out(S, STAGE);
     // own rows first: their HBM latency overlaps the record staging
@@ -581,7 +611,8 @@ __global__ __launch_bounds__(kBlock) void k_stage(StepGeom G, StepBuffers S, Bat
         y3 = S.acc[o];
     }
     const int64_t nf = G.nfluid - node0;
-    stage_contiguous<REC>(S.slab, node0, nf <= 0 ? 0 : (nf < NPB ? int(nf) : NPB), K, srec);
+    const int RW = rec_floats<Q, D>(K);
+    stage_contiguous(S.slab, node0, nf <= 0 ? 0 : (nf < NPB ? int(nf) : NPB), RW, srec);
     __syncthreads();
     if (STAGE == 1 && !fluid && i < G.N) {
         if (ln.active) {
@@ -592,7 +623,7 @@ __global__ __launch_bounds__(kBlock) void k_stage(StepGeom G, StepBuffers S, Bat
         return;
     }
     if (!fluid) return;
-    const float rate = -stencil_sum<Q, KT, BATCH>(srec + ln.slot * K * REC, K, gin, a);
+    const float rate = -stencil_sum<Q, KT, BATCH>(srec + ln.slot * RW, K, gin, G.N, a);
     if (!ln.active) return;
     gout[o] = rk4_out<STAGE>(g0, rate, G.dt, y1, y2, y3);
 }
@@ -1192,418 +1223,331 @@ __global__ __launch_bounds__(NPB * kV4Lanes) __attribute__((amdgpu_waves_per_eu(
 }
 
 // ---------------------------------------------------------------------------
-// D2Q9 stencil passes with three distributions per lane: a node's 36-byte
-// row is three 12-byte pieces, so one wavefront gathers 21 neighbour rows
-// per instruction (the lane-over-alpha kernels gather 7), and the records
-// are read by 3 lanes per node instead of 9.  The records of the block's
-// nodes are staged in LDS with one pad float per node row (distinct banks
-// for the 21 nodes of a wavefront).  Same products in the same order as the
-// lane-over-alpha kernels.
+// D2Q9 stencil passes with two lanes per node: the row of moving
+// distributions is two 16-byte pieces, lane q serving distributions 4q + 1 ..
+// 4q + 4, whose velocities are those of lane 0 with the sign of q.  A
+// wavefront gathers 32 neighbour rows per instruction, each within one
+// 128-byte line.  The rest distribution has velocity zero: the RK4 stages and
+// the PML divergence leave it alone.  The records of the block's nodes are
+// staged in LDS in rows of an odd number of 16-byte units (distinct banks for
+// the 32 nodes of a wavefront).
 // ---------------------------------------------------------------------------
-constexpr int kQ9Lanes = 3;                          // lanes per node
-constexpr int kQ9Npw = 21;                           // nodes per wavefront
-constexpr int kQ9Npb = kQ9Npw * (kBlock / 64);       // nodes per block (84)
-static_assert(kQ9Npb == kQ9TileNodes, "D2Q9 union tiles are the three-per-lane blocks");
+constexpr int kQ9Npb = kBlock / 2;     // nodes per block
+constexpr int kQ9BndNpb = kBlock / 8;  // boundary nodes per block (eight lanes each)
 
-struct Q9Lane {
-    int slot, q;   // node slot in the block, piece (distributions 3q .. 3q + 2)
-    bool active;   // lane 63 of a wavefront serves no node
-    __device__ Q9Lane() {
-        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-        const int sub = lane / kQ9Lanes;
-        active = sub < kQ9Npw;
-        q = active ? lane - sub * kQ9Lanes : 0;
-        slot = wave * kQ9Npw + (active ? sub : 0);
-    }
-};
-
-typedef float f3v __attribute__((ext_vector_type(3)));
-__device__ __forceinline__ f3v ld3(__amdgpu_buffer_rsrc_t r, uint32_t off) {
-    const auto v = __builtin_amdgcn_raw_buffer_load_b96(r, off, 0, 0);
-    f3v o;
-    o.x = __uint_as_float(v[0]);
-    o.y = __uint_as_float(v[1]);
-    o.z = __uint_as_float(v[2]);
-    return o;
-}
-__device__ __forceinline__ void st3(__amdgpu_buffer_rsrc_t r, uint32_t off, f3v x) {
-    typedef unsigned u3v __attribute__((ext_vector_type(3)));
-    u3v v;
+__device__ __forceinline__ void stb4(__amdgpu_buffer_rsrc_t r, uint32_t off, const float4& x) {
+    typedef unsigned u4v __attribute__((ext_vector_type(4)));
+    u4v v;
     v.x = __float_as_uint(x.x);
     v.y = __float_as_uint(x.y);
     v.z = __float_as_uint(x.z);
-    __builtin_amdgcn_raw_buffer_store_b96(v, r, off, 0, 0);
+    v.w = __float_as_uint(x.w);
+    __builtin_amdgcn_raw_buffer_store_b128(v, r, off, 0, 0);
+}
+__device__ __forceinline__ float ld1(__amdgpu_buffer_rsrc_t r, uint32_t off) {
+    return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
 }
 
-// records of nodes [node0, node0 + cnt) (rows of RW floats) into lds rows
-// of RW + 1 floats by LDS DMA: the block's waves copy 64-float chunks of
-// the padded layout, lane l of chunk c filling LDS float 64 c + l with its
-// source float (a pad slot takes the tile's first float; lanes past the
-// last row copy nothing).  Wait with dma_fence.
-__device__ __forceinline__ void stage_padded(const float* slab, int64_t node0, int cnt, int RW,
-                                             float* lds) {
+// Records of the block's cnt nodes into LDS rows of UP = q9_pitch(U) 16-byte
+// units by LDS DMA: the block's waves copy 64-unit chunks of the padded
+// layout, the pad units reading past the resource (zero, no traffic).  The
+// node's slab row is node0 + its slot, or rows_of[slot].  Wait with dma_fence.
+// The copies are bound by their instructions: a million k = 16 nodes' stage
+// takes 73 us with 4-byte copies, 52 us with these and 24 us without any.
+__device__ __forceinline__ void stage_units(__amdgpu_buffer_rsrc_t src, const uint32_t* rows_of,
+                                            int cnt, int U, float4* lds) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int RP = RW + 1, tot = cnt * RP;
-    const __amdgpu_buffer_rsrc_t src = rsrc(slab + node0 * int64_t(RW), uint64_t(cnt) * RW * 4u);
-    const int nchunks = (tot + 63) / 64;
-    // t / RP by a float reciprocal: t < 2^15 and RP <= 193 keep (t + 1/2) / RP
-    // at least 1/(2 RP) from an integer, far above the rounding error
-    const float rinv = 1.0f / float(RP);
-    for (int c = wave; c < nchunks; c += kBlock / 64) {
+    const int UP = q9_pitch(U), tot = cnt * UP;
+    // t / UP by a float reciprocal: t < 2^13 and UP <= 49 keep (t + 1/2) / UP
+    // at least 1/(2 UP) from an integer, far above the rounding error
+    const float rinv = 1.0f / float(UP);
+    for (int c = wave; c < (tot + 63) / 64; c += kBlock / 64) {
         const int t = c * 64 + lane;
-        const int node = int((float(t) + 0.5f) * rinv), off = t - node * RP;
-        const uint32_t e = off < RW ? uint32_t(node * RW + off) : 0u;
-        if (t < tot)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(src, (lds_void_t*)(lds + c * 64), 4, e * 4u,
-                                                     0, 0, kStreamPolicy);
-    }
-}
-
-__device__ __forceinline__ float c9(int a, int d) { return float(Lattice<9>::c(a, d)); }
-
-// sum_s (c_a . W_s) fin(idx_s)_a for the lane's three distributions, the
-// neighbour pieces fetched by fetch(index field) (a node index, or a
-// position in the tile's union)
-template <int BATCH, class Fetch>
-__device__ __forceinline__ f3v stencil_sum3(const float* rp, int K, int q, Fetch fetch) {
-    float cx[3], cy[3];
-#pragma unroll
-    for (int e = 0; e < 3; ++e) {
-        cx[e] = c9(3 * q + e, 0);
-        cy[e] = c9(3 * q + e, 1);
-    }
-    f3v acc = {0.0f, 0.0f, 0.0f};
-    for (int s0 = 0; s0 < K; s0 += BATCH) {
-        float wx[BATCH], wy[BATCH];
-        f3v gv[BATCH];
-#pragma unroll
-        for (int u = 0; u < BATCH; ++u) {
-            const int s = s0 + u;
-            const bool in = s < K;
-            const float* r = rp + (in ? s : 0) * 3;
-            const uint32_t j = __float_as_uint(r[0]);
-            wx[u] = in ? r[1] : 0.0f;
-            wy[u] = in ? r[2] : 0.0f;
-            gv[u] = fetch(j);
-        }
-#pragma unroll
-        for (int u = 0; u < BATCH; ++u) {
-            acc.x += (cx[0] * wx[u] + cy[0] * wy[u]) * gv[u].x;
-            acc.y += (cx[1] * wx[u] + cy[1] * wy[u]) * gv[u].y;
-            acc.z += (cx[2] * wx[u] + cy[2] * wy[u]) * gv[u].z;
-        }
-    }
-    return acc;
-}
-
-// D2Q9 tile unions: the distinct stencil neighbours of the 84 fluid nodes
-// of a block's tile, their rows copied to LDS after the block's records
-// (urows[9 r + 3 q + e] = distribution 3 q + e of row ul[r]) so every
-// gather of the stencil sums reads LDS.  The block's threads copy the
-// 3 Uc 12-byte pieces: every index load first (past Uc they read zero
-// through the buffer resource), then every row load, then the stores.
-constexpr int kQ9CopyIt = (3 * kQ9UnionRowsMax + kBlock - 1) / kBlock;
-struct Q9UnionIdx {
-    uint32_t j[kQ9CopyIt];
-};
-__device__ __forceinline__ Q9UnionIdx q9_union_indices(const uint32_t* ul, int Uc) {
-    const __amdgpu_buffer_rsrc_t ur = rsrc(ul, uint64_t(Uc) * 4u);
-    const int nit = (3 * Uc + kBlock - 1) / kBlock;
-    Q9UnionIdx x;
-#pragma unroll
-    for (int it = 0; it < kQ9CopyIt; ++it) {
-        const uint32_t t = threadIdx.x + it * kBlock;
-        x.j[it] = it < nit ? __builtin_amdgcn_raw_buffer_load_b32(ur, (t / 3u) * 4u, 0, 0) : 0u;
-    }
-    return x;
-}
-__device__ __forceinline__ void q9_union_rows(float* urows, const Q9UnionIdx& x, int Uc,
-                                              __amdgpu_buffer_rsrc_t src) {
-    const int nit = (3 * Uc + kBlock - 1) / kBlock;
-    f3v v[kQ9CopyIt];
-#pragma unroll
-    for (int it = 0; it < kQ9CopyIt; ++it) {
-        const uint32_t t = threadIdx.x + it * kBlock;
-        if (it < nit) v[it] = ld3(src, x.j[it] * 36u + (t % 3u) * 12u);
-    }
-#pragma unroll
-    for (int it = 0; it < kQ9CopyIt; ++it) {
-        const int t = int(threadIdx.x) + it * kBlock;
-        if (it < nit && t < 3 * Uc) {
-            urows[3 * t] = v[it].x;
-            urows[3 * t + 1] = v[it].y;
-            urows[3 * t + 2] = v[it].z;
+        const int node = int((float(t) + 0.5f) * rinv), off = t - node * UP;
+        if (t < tot) {
+            const uint32_t row = rows_of ? rows_of[node] : uint32_t(node);
+            dma16<kStreamPolicy>(src, off < U ? (row * uint32_t(U) + uint32_t(off)) * 16u : 0xfffffff0u,
+                                 lds + c * 64);
         }
     }
 }
-__device__ __forceinline__ f3v q9_lds_row(const float* urows, uint32_t p, int q) {
-    const float* r = urows + p * 9u + uint32_t(q) * 3u;
-    return f3v{r[0], r[1], r[2]};
+
+// NG groups of four records, every gather issued before the first use.
+template <int NG>
+__device__ __forceinline__ void stencil_groups_q9(const float4* rp, uint32_t lane_off,
+                                                  __amdgpu_buffer_rsrc_t fin, float4& acc) {
+    float4 wx[NG], wy[NG], gv[4 * NG];
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+        const float4 j = rp[3 * g];
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            gv[4 * g + e] = ld4(fin, __float_as_uint(get(j, e)) * 32u + lane_off);
+        wx[g] = rp[3 * g + 1];
+        wy[g] = rp[3 * g + 2];
+    }
+#pragma unroll
+    for (int g = 0; g < NG; ++g)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {  // velocities of alpha 1 .. 4
+            const float x = get(wx[g], e), y = get(wy[g], e);
+            acc.x += (y - x) * gv[4 * g + e].x;
+            acc.y -= x * gv[4 * g + e].y;
+            acc.z -= (x + y) * gv[4 * g + e].z;
+            acc.w -= y * gv[4 * g + e].w;
+        }
 }
 
-template <int STAGE, int BATCH, bool TU = false>
-__global__ __launch_bounds__(kBlock) void k_stage3(StepGeom G, StepBuffers S, BatchArgs B) {
-    extern __shared__ float srec3[];
+// sum_s (c_a . W_s) fin(idx_s)_a of the lane's four distributions over the
+// node's staged records.
+template <int BATCH>
+__device__ __forceinline__ float4 stencil_sum_q9(const float4* rp, int K, int q,
+                                                 __amdgpu_buffer_rsrc_t fin) {
+    constexpr int NG = BATCH / 4;
+    const uint32_t lane_off = uint32_t(q) * 16u;
+    const int G = (K + 3) / 4;
+    float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
+    int g = 0;
+    for (; g + NG <= G; g += NG) stencil_groups_q9<NG>(rp + 3 * g, lane_off, fin, a);
+    for (; g < G; ++g) stencil_groups_q9<1>(rp + 3 * g, lane_off, fin, a);
+    const float sign = q ? -1.0f : 1.0f;
+    return make_float4(sign * a.x, sign * a.y, sign * a.z, sign * a.w);
+}
+
+template <int STAGE, int BATCH>
+__global__ __launch_bounds__(kBlock) void k_stage_q9(StepGeom G, StepBuffers S, BatchArgs B) {
+    extern __shared__ float4 recs9[];
     const BlockCtx bc = locate(B, G, S);
-    const int K = G.k, RW = 3 * K;
-    const int64_t tile = xcd_tile(bc.b, bc.nb);
-    const int64_t node0 = tile * kQ9Npb;
-    const Q9Lane ln;
-    const int64_t i = node0 + ln.slot;
-    const uint64_t rows = uint64_t(G.N) * 36u;
-    const uint32_t own = uint32_t(i) * 36u + uint32_t(ln.q) * 12u;
-    const __amdgpu_buffer_rsrc_t rg = rsrc(S.g, rows);
+    const int K = G.k, U = q9_units(K, 2);
+    const int64_t node0 = xcd_tile(bc.b, bc.nb) * kQ9Npb;
+    const int slot = threadIdx.x >> 1, q = threadIdx.x & 1;
+    const int64_t i = node0 + slot;
+    const uint64_t rows = uint64_t(G.N) * 32u;
+    const uint32_t own = uint32_t(i) * 32u + uint32_t(q) * 16u;
     const __amdgpu_buffer_rsrc_t gin = rsrc(stage_in(S, STAGE), rows);
     // own rows first: their latency overlaps the record staging
     const bool fluid = i < G.nfluid;
-    const f3v g0 = ld3(rg, own);  // past N: zero
-    f3v y1 = {0.f, 0.f, 0.f}, y2 = y1, y3 = y1;
+    const float4 g0 = ld4(rsrc(S.g, rows), own);  // past N: zero
+    float4 y1 = make_float4(0.f, 0.f, 0.f, 0.f), y2 = y1, y3 = y1;
     if (STAGE == 4 && fluid) {
-        y1 = ld3(rsrc(S.A, rows), own);
-        y2 = ld3(rsrc(S.B, rows), own);
-        y3 = ld3(rsrc(S.acc, rows), own);
+        y1 = ld4(rsrc(S.A, rows), own);
+        y2 = ld4(rsrc(S.B, rows), own);
+        y3 = ld4(rsrc(S.acc, rows), own);
     }
     const int64_t nf = G.nfluid - node0;
     const int cnt = nf <= 0 ? 0 : (nf < kQ9Npb ? int(nf) : kQ9Npb);
-    // with tile unions: the tile's union range (tiles of fluid nodes only)
-    int64_t u0 = 0;
-    int U = 0;
-    if (TU && cnt > 0) union_range(S.uoff, tile, u0, U);
-    const int Uc = U < S.ucap ? U : S.ucap;
-    float* urows = srec3 + kQ9Npb * (RW + 1);
-    Q9UnionIdx ux;
-    if (TU) ux = q9_union_indices(S.ulist + u0, Uc);
-    stage_padded(TU ? S.uslab : S.slab, node0, cnt, RW, srec3);
-    if (TU) q9_union_rows(urows, ux, Uc, gin);
+    stage_units(rsrc(S.slab + node0 * U * 4, uint64_t(cnt) * U * 16u), nullptr, cnt, U, recs9);
     dma_fence();
-    if (!ln.active || i >= G.N) return;
+    if (i >= G.N) return;
     if (STAGE == 1 && !fluid) {
-        st3(rsrc(S.A, rows), own, g0);
-        st3(rsrc(S.B, rows), own, g0);
-        st3(rsrc(S.acc, rows), own, g0);
+        stb4(rsrc(S.A, rows), own, g0);
+        stb4(rsrc(S.B, rows), own, g0);
+        stb4(rsrc(S.acc, rows), own, g0);
         return;
     }
     if (!fluid) return;
-    // stage 4: the part without the rate, formed before the gather (three
-    // live values instead of twelve; the arithmetic of rk4_out<4>)
-    f3v pre = g0;
-    if (STAGE == 4) {
-        pre.x = rk4_pre(g0.x, y1.x, y2.x, y3.x);
-        pre.y = rk4_pre(g0.y, y1.y, y2.y, y3.y);
-        pre.z = rk4_pre(g0.z, y1.z, y2.z, y3.z);
-        asm volatile("" : "+v"(pre.x), "+v"(pre.y), "+v"(pre.z));
-    }
-    const float* rp = srec3 + ln.slot * (RW + 1);
-    const uint32_t lane_off = uint32_t(ln.q) * 12u;
-    f3v acc;
-    if (!TU) {
-        acc = stencil_sum3<BATCH>(rp, K, ln.q,
-                                  [&](uint32_t j) { return ld3(gin, j * 36u + lane_off); });
-    } else if (U <= S.ucap) {
-        acc = stencil_sum3<BATCH>(rp, K, ln.q,
-                                  [&](uint32_t p) { return q9_lds_row(urows, p, ln.q); });
-    } else {  // union over the cap: rows read from HBM through the list
-        const uint32_t* ul = S.ulist + u0;
-        acc = stencil_sum3<BATCH>(rp, K, ln.q,
-                                  [&](uint32_t p) { return ld3(gin, ul[p] * 36u + lane_off); });
-    }
-    f3v out;
-    if (STAGE == 4) {
-        const float c = G.dt * (1.0f / 6.0f);
-        out.x = pre.x + c * -acc.x;
-        out.y = pre.y + c * -acc.y;
-        out.z = pre.z + c * -acc.z;
-    } else {
-        out.x = rk4_out<STAGE>(g0.x, -acc.x, G.dt, y1.x, y2.x, y3.x);
-        out.y = rk4_out<STAGE>(g0.y, -acc.y, G.dt, y1.y, y2.y, y3.y);
-        out.z = rk4_out<STAGE>(g0.z, -acc.z, G.dt, y1.z, y2.z, y3.z);
-    }
-    st3(rsrc(stage_out(S, STAGE), rows), own, out);
+    // stage 4: the part without the rate, formed before the gather (four
+    // live values instead of sixteen; the arithmetic of rk4_out<4>)
+    float4 pre = STAGE == 4 ? rk4_pre4(g0, y1, y2, y3) : g0;
+    if (STAGE == 4) asm volatile("" : "+v"(pre.x), "+v"(pre.y), "+v"(pre.z), "+v"(pre.w));
+    const float4 acc = stencil_sum_q9<BATCH>(recs9 + slot * q9_pitch(U), K, q, gin);
+    const float4 r = make_float4(-acc.x, -acc.y, -acc.z, -acc.w);
+    stb4(rsrc(stage_out(S, STAGE), rows), own,
+         STAGE == 4 ? rk4_post4(pre, r, G.dt) : rk4_out4<STAGE>(g0, r, G.dt, y1, y2, y3));
 }
 
-// p2 for D2Q9, three per lane: the PML divergence over the listed nodes
-// (the arithmetic of k_p2), each node's records staged by its three lanes.
-__global__ __launch_bounds__(kBlock) void k_p2_3(StepGeom G, StepBuffers S, BatchArgs B) {
-    extern __shared__ float srec3[];
+// p2 for D2Q9, two lanes per node: the PML divergence over the listed nodes
+// (the arithmetic of k_p2), the listed nodes' records staged like a tile's.
+__global__ __launch_bounds__(kBlock) void k_p2_q9(StepGeom G, StepBuffers S, BatchArgs B) {
+    extern __shared__ float4 recs9[];
+    __shared__ uint32_t rows_of[kQ9Npb];
     const BlockCtx bc = locate(B, G, S);
-    const int K = G.k, RW = 3 * K;
-    const Q9Lane ln;
-    const int64_t item0 = xcd_tile(bc.b, bc.nb) * kQ9Npb, item = item0 + ln.slot;
-    const bool valid = ln.active && item < S.n_pml;
-    const int64_t i = valid ? S.pml_list[item] : 0;
-    float* rp = srec3 + ln.slot * (RW + 1);
+    const int K = G.k, U = q9_units(K, 2), UP = q9_pitch(U);
+    const int slot = threadIdx.x >> 1, q = threadIdx.x & 1;
+    const int64_t item0 = xcd_tile(bc.b, bc.nb) * kQ9Npb;
     const int64_t left = S.n_pml - item0;
     const int cnt = left < kQ9Npb ? int(left) : kQ9Npb;
-    if (uint64_t(G.nfluid) * uint64_t(RW) * 4u < (uint64_t(1) << 32)) {
-        // the listed nodes' records by LDS DMA (32-bit offsets into the slab)
-        __shared__ uint32_t rows_of[kQ9Npb];
-        if (int(threadIdx.x) < cnt) rows_of[threadIdx.x] = uint32_t(S.pml_list[item0 + threadIdx.x]);
-        __syncthreads();
-        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-        const int RP = RW + 1, tot = cnt * RP;
-        const __amdgpu_buffer_rsrc_t src = rsrc(S.slab, uint64_t(G.nfluid) * RW * 4u);
-        const float rinv = 1.0f / float(RP);  // as in stage_padded
-        for (int c = wave; c < (tot + 63) / 64; c += kBlock / 64) {
-            const int t = c * 64 + lane;
-            const int node = int((float(t) + 0.5f) * rinv), off = t - node * RP;
-            const uint32_t e =
-                (t < tot && off < RW) ? rows_of[node < cnt ? node : 0] * uint32_t(RW) + uint32_t(off)
-                                      : 0u;
-            if (t < tot)
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(src, (lds_void_t*)(srec3 + c * 64), 4,
-                                                         e * 4u, 0, 0, kStreamPolicy);
-        }
+    if (int(threadIdx.x) < cnt) rows_of[threadIdx.x] = uint32_t(S.pml_list[item0 + threadIdx.x]);
+    __syncthreads();
+    const bool valid = slot < cnt;
+    const uint32_t i = valid ? rows_of[slot] : 0u;
+    const uint64_t bytes = uint64_t(G.nfluid) * U * 16u;
+    if (bytes < 0xfffffff0ull) {  // 32-bit offsets into the slab
+        stage_units(rsrc(S.slab, bytes), rows_of, cnt, U, recs9);
         dma_fence();
     } else {
         if (valid) {
-            const float* src = S.slab + i * int64_t(RW);
-            for (int t = ln.q; t < RW; t += kQ9Lanes) rp[t] = src[t];
+            const float4* src = reinterpret_cast<const float4*>(S.slab) + int64_t(i) * U;
+            for (int t = q; t < U; t += 2) recs9[slot * UP + t] = src[t];
         }
         __syncthreads();
     }
     if (!valid) return;
-    const uint64_t rows = uint64_t(G.N) * 36u;
-    const __amdgpu_buffer_rsrc_t gf = rsrc(S.Gf, rows);
-    const uint32_t lane_off = uint32_t(ln.q) * 12u;
-    const f3v acc =
-        stencil_sum3<8>(rp, K, ln.q, [&](uint32_t j) { return ld3(gf, j * 36u + lane_off); });
+    const uint64_t rows = uint64_t(G.N) * 32u;
+    const float4 acc = stencil_sum_q9<8>(recs9 + slot * UP, K, q, rsrc(S.Gf, rows));
     const __amdgpu_buffer_rsrc_t ra = rsrc(S.A, rows);
-    const uint32_t own = uint32_t(i) * 36u + uint32_t(ln.q) * 12u;
-    f3v a = ld3(ra, own);
-    a.x += acc.x;
-    a.y += acc.y;
-    a.z += acc.z;
-    st3(ra, own, a);
+    const uint32_t own = i * 32u + uint32_t(q) * 16u;
+    const float4 a = ld4(ra, own);
+    stb4(ra, own, make_float4(a.x + acc.x, a.y + acc.y, a.z + acc.z, a.w + acc.w));
 }
 
-// Boundary interpolation for D2Q9, three per lane (the arithmetic of
-// k_binterp): accumulate = true (p3) interpolates s1 minus the sources'
-// collision increments onto the row's own increment, false (p5) overwrites.
+// Boundary interpolation for D2Q9, eight lanes per node (two pieces of the
+// row by four interleaved quarters of the stencil, summed at the end): the
+// pass has few nodes and is bound by the latency of its two dependent loads,
+// so each lane issues its quarter's at once.  accumulate = true (p3)
+// interpolates s1 minus the sources' collision increments onto the row's own
+// increment, false (p5) overwrites.
 template <bool ACCUMULATE>
-__global__ __launch_bounds__(kBlock) void k_binterp3(StepGeom G, StepBuffers S, BatchArgs B) {
+__global__ __launch_bounds__(kBlock) void k_binterp_q9(StepGeom G, StepBuffers S, BatchArgs B) {
     const BlockCtx bc = locate(B, G, S);
-    const Q9Lane ln;
-    const int64_t nbnd = G.N - G.nfluid;
-    const int64_t m = xcd_tile(bc.b, bc.nb) * kQ9Npb + ln.slot;
-    if (!ln.active || m >= nbnd) return;
+    const int q = threadIdx.x & 1, part = (threadIdx.x >> 1) & 3;
+    const int64_t m = xcd_tile(bc.b, bc.nb) * kQ9BndNpb + (threadIdx.x >> 3);
+    if (m >= G.N - G.nfluid) return;  // the node's eight lanes together
     float* field = ACCUMULATE ? S.A : S.g;
-    const uint64_t rows = uint64_t(G.N) * 36u;
-    const __amdgpu_buffer_rsrc_t f = rsrc(field, rows), cl = rsrc(S.coll, rows);
-    const float* rec = S.bslab + m * int64_t(G.kb) * 2;
-    const uint32_t lane_off = uint32_t(ln.q) * 12u;
-    const uint32_t own = uint32_t(G.nfluid + m) * 36u + lane_off;
-    const f3v b = ACCUMULATE ? ld3(f, own) : f3v{0.0f, 0.0f, 0.0f};
-    f3v acc = {0.0f, 0.0f, 0.0f};
-    for (int s0 = 0; s0 < G.kb; s0 += 8) {
-        float w[8];
-        f3v v[8];
+    const uint64_t rows = uint64_t(G.N) * 32u, rest = uint64_t(G.N) * 4u;
+    const __amdgpu_buffer_rsrc_t f = rsrc(field, rows), f0 = rsrc(field + 8 * G.N, rest);
+    const __amdgpu_buffer_rsrc_t cl = rsrc(S.coll, rows), cl0 = rsrc(S.coll + 8 * G.N, rest);
+    const float2* rec = reinterpret_cast<const float2*>(S.bslab) + m * int64_t(G.kb);
+    const uint32_t lane_off = uint32_t(q) * 16u;
+    const uint32_t own = uint32_t(G.nfluid + m);
+    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+    float acc0 = 0.0f;  // rest: the even lanes' sum
+    constexpr int BT = 4;
+    for (int s0 = part; s0 < G.kb; s0 += 4 * BT) {
+        float2 r[BT];
+        float4 v[BT];
+        float v0[BT];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const int s = s0 + u;
-            const bool in = s < G.kb;
-            const uint32_t j = __float_as_uint(rec[2 * (in ? s : 0)]);
-            w[u] = in ? rec[2 * s + 1] : 0.0f;
-            v[u] = ld3(f, j * 36u + lane_off);
+        for (int u = 0; u < BT; ++u)
+            r[u] = s0 + 4 * u < G.kb ? rec[s0 + 4 * u] : make_float2(__uint_as_float(own), 0.0f);
+#pragma unroll
+        for (int u = 0; u < BT; ++u) {
+            const uint32_t j = __float_as_uint(r[u].x);
+            v[u] = ld4(f, j * 32u + lane_off);
+            v0[u] = q == 0 ? ld1(f0, j * 4u) : 0.0f;
             if (ACCUMULATE) {
-                const f3v c = ld3(cl, j * 36u + lane_off);
-                v[u].x = v[u].x - c.x;
-                v[u].y = v[u].y - c.y;
-                v[u].z = v[u].z - c.z;
+                const float4 c = ld4(cl, j * 32u + lane_off);
+                v[u] = make_float4(v[u].x - c.x, v[u].y - c.y, v[u].z - c.z, v[u].w - c.w);
+                if (q == 0) v0[u] -= ld1(cl0, j * 4u);
             }
         }
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            acc.x += w[u] * v[u].x;
-            acc.y += w[u] * v[u].y;
-            acc.z += w[u] * v[u].z;
+        for (int u = 0; u < BT; ++u) {
+            const bool in = s0 + 4 * u < G.kb;  // the row of a missing record is not used
+            acc.x += in ? r[u].y * v[u].x : 0.0f;
+            acc.y += in ? r[u].y * v[u].y : 0.0f;
+            acc.z += in ? r[u].y * v[u].z : 0.0f;
+            acc.w += in ? r[u].y * v[u].w : 0.0f;
+            acc0 += in ? r[u].y * v0[u] : 0.0f;
         }
     }
-    f3v out = acc;
-    if (ACCUMULATE) {
-        out.x = b.x + acc.x;
-        out.y = b.y + acc.y;
-        out.z = b.z + acc.z;
+#pragma unroll
+    for (int o = 2; o <= 4; o <<= 1) {
+        acc.x += __shfl_xor(acc.x, o);
+        acc.y += __shfl_xor(acc.y, o);
+        acc.z += __shfl_xor(acc.z, o);
+        acc.w += __shfl_xor(acc.w, o);
+        acc0 += __shfl_xor(acc0, o);
     }
-    st3(f, own, out);
+    if (part != 0) return;
+    if (ACCUMULATE) {
+        const float4 b = ld4(f, own * 32u + lane_off);
+        acc = make_float4(b.x + acc.x, b.y + acc.y, b.z + acc.z, b.w + acc.w);
+        if (q == 0) acc0 += field[8 * G.N + own];
+    }
+    stb4(f, own * 32u + lane_off, acc);
+    if (q == 0) field[8 * G.N + own] = acc0;
 }
 
-// p4 for D2Q9, three per lane: selective filter on fluid nodes, bounce-back
-// on boundary nodes (the arithmetic of k_p4).
-template <bool TU = false>
-__global__ __launch_bounds__(kBlock) void k_p4_3(StepGeom G, StepBuffers S, BatchArgs B) {
-    extern __shared__ float srec3[];
+// NG groups of four filter records ({indices}, {weights}), every gather
+// issued before the first use; the rest values of a node's neighbours are
+// taken by its two lanes in turns.
+template <int NG>
+__device__ __forceinline__ void filter_groups_q9(const float4* rp, int q, __amdgpu_buffer_rsrc_t r1,
+                                                 __amdgpu_buffer_rsrc_t r0, const float4& si,
+                                                 float si0, float4& sum, float& sum0) {
+    const uint32_t lane_off = uint32_t(q) * 16u;
+    float4 w[NG], gv[4 * NG];
+    float g0[2 * NG];
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+        const float4 j = rp[2 * g];
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            gv[4 * g + e] = ld4(r1, __float_as_uint(get(j, e)) * 32u + lane_off);
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+            g0[2 * g + e] = ld1(r0, __float_as_uint(q ? get(j, 2 * e + 1) : get(j, 2 * e)) * 4u);
+        w[g] = rp[2 * g + 1];
+    }
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float4& v = gv[4 * g + e];
+            sum.x += get(w[g], e) * (v.x - si.x);
+            sum.y += get(w[g], e) * (v.y - si.y);
+            sum.z += get(w[g], e) * (v.z - si.z);
+            sum.w += get(w[g], e) * (v.w - si.w);
+        }
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+            sum0 += (q ? get(w[g], 2 * e + 1) : get(w[g], 2 * e)) * (g0[2 * g + e] - si0);
+    }
+}
+
+// p4 for D2Q9, two lanes per node: selective filter on fluid nodes,
+// bounce-back on boundary nodes (the arithmetic of k_p4).
+__global__ __launch_bounds__(kBlock) void k_p4_q9(StepGeom G, StepBuffers S, BatchArgs B) {
+    extern __shared__ float4 recs9[];
     const BlockCtx bc = locate(B, G, S);
-    const int K = G.k, RW = 2 * K;
-    const int64_t tile = xcd_tile(bc.b, bc.nb);
-    const int64_t node0 = tile * kQ9Npb;
-    const Q9Lane ln;
-    const int64_t i = node0 + ln.slot;
-    const uint64_t rows = uint64_t(G.N) * 36u;
-    const uint32_t own = uint32_t(i) * 36u + uint32_t(ln.q) * 12u;
-    const __amdgpu_buffer_rsrc_t r1 = rsrc(S.A, rows);
-    const f3v si = ld3(r1, own);
+    const int U = q9_units(G.k, 1);
+    const int64_t node0 = xcd_tile(bc.b, bc.nb) * kQ9Npb;
+    const int slot = threadIdx.x >> 1, q = threadIdx.x & 1;
+    const int64_t i = node0 + slot;
+    const uint64_t rows = uint64_t(G.N) * 32u;
+    const uint32_t own = uint32_t(i) * 32u + uint32_t(q) * 16u;
+    const __amdgpu_buffer_rsrc_t r1 = rsrc(S.A, rows), r0 = rsrc(S.A + 8 * G.N, uint64_t(G.N) * 4u);
+    const float4 si = ld4(r1, own);  // past N: zero
+    const float si0 = ld1(r0, uint32_t(i) * 4u);
     const int64_t nf = G.nfluid - node0;
     const int cnt = nf <= 0 ? 0 : (nf < kQ9Npb ? int(nf) : kQ9Npb);
-    int64_t u0 = 0;
-    int U = 0;
-    if (TU && cnt > 0) union_range(S.uoff, tile, u0, U);
-    const int Uc = U < S.ucap ? U : S.ucap;
-    float* urows = srec3 + kQ9Npb * (RW + 1);
-    Q9UnionIdx ux;
-    if (TU) ux = q9_union_indices(S.ulist + u0, Uc);
-    stage_padded(TU ? S.ufslab : S.fslab, node0, cnt, RW, srec3);
-    if (TU) q9_union_rows(urows, ux, Uc, r1);
+    stage_units(rsrc(S.fslab + node0 * U * 4, uint64_t(cnt) * U * 16u), nullptr, cnt, U, recs9);
     dma_fence();
-    if (!ln.active || i >= G.N) return;
-    f3v out;
+    if (i >= G.N) return;
+    float4 out;
+    float out0 = si0;
     if (i < G.nfluid) {
-        const float* rp = srec3 + ln.slot * (RW + 1);
-        const uint32_t lane_off = uint32_t(ln.q) * 12u;
-        const uint32_t* ul = S.ulist + u0;
-        const bool lds = TU && U <= S.ucap;
-        f3v sum = {0.0f, 0.0f, 0.0f};
-        for (int s0 = 0; s0 < K; s0 += 8) {
-            float w[8];
-            f3v gv[8];
-#pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const int s = s0 + u;
-                const bool in = s < K;
-                const uint32_t j = __float_as_uint(rp[(in ? s : 0) * 2]);
-                w[u] = in ? rp[s * 2 + 1] : 0.0f;
-                if (!TU) gv[u] = ld3(r1, j * 36u + lane_off);
-                else if (lds) gv[u] = q9_lds_row(urows, j, ln.q);
-                else gv[u] = ld3(r1, ul[j] * 36u + lane_off);  // over the cap: through the list
-            }
-#pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                sum.x += w[u] * (gv[u].x - si.x);
-                sum.y += w[u] * (gv[u].y - si.y);
-                sum.z += w[u] * (gv[u].z - si.z);
-            }
-        }
+        const float4* rp = recs9 + slot * q9_pitch(U);
+        const int ng = (G.k + 3) / 4;
+        float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
+        float sum0 = 0.0f;
+        int g = 0;
+        for (; g + 2 <= ng; g += 2) filter_groups_q9<2>(rp + 2 * g, q, r1, r0, si, si0, sum, sum0);
+        if (g < ng) filter_groups_q9<1>(rp + 2 * g, q, r1, r0, si, si0, sum, sum0);
+        sum0 += __shfl_xor(sum0, 1);
         out.x = si.x + G.filter * sum.x;
         out.y = si.y + G.filter * sum.y;
         out.z = si.z + G.filter * sum.z;
+        out.w = si.w + G.filter * sum.w;
+        out0 = si0 + G.filter * sum0;
     } else {
         const int64_t b = i - G.nfluid;
         const float n0 = S.normals[b * 2], n1 = S.normals[b * 2 + 1];
-        const float* row = S.A + i * 9;
-        float o3[3];
+        float o[4];
 #pragma unroll
-        for (int e = 0; e < 3; ++e) {
-            const int a = 3 * ln.q + e;
+        for (int e = 0; e < 4; ++e) {
+            const int a = 4 * q + 1 + e;
             float cn = 0.0f;
-            cn += c9(a, 0) * n0;
-            cn += c9(a, 1) * n1;
-            const int src = cn > 0.0f ? Lattice<9>::bb(a) : a;
-            o3[e] = row[src];
+            cn += lane_c<9>(a, 0) * n0;
+            cn += lane_c<9>(a, 1) * n1;
+            const int src = cn > 0.0f ? (a > 4 ? a - 4 : a + 4) : a;  // opposite: four on
+            o[e] = S.A[row_at<9>(i, src, G.N)];
         }
-        out.x = o3[0];
-        out.y = o3[1];
-        out.z = o3[2];
+        out = make_float4(o[0], o[1], o[2], o[3]);
     }
-    st3(rsrc(S.g, rows), own, out);
+    stb4(rsrc(S.g, rows), own, out);
+    if (q == 0) S.g[8 * G.N + i] = out0;
 }
 
 // sum_s w_s (g_s - g_i) over the staged filter records rp ({index field, w}),
@@ -2073,8 +2017,8 @@ __global__ __launch_bounds__(kBlock) void k_source_field(const int32_t* nodes,
 template <int Q>
 __global__ __launch_bounds__(kBlock) void k_probe(int64_t n, int k, const uint32_t* idx,
                                                   const float* w, const float* held,
-                                                  const float* g, double rho0, double* out) {
-    using L = Lattice<Q>;
+                                                  const float* g, int64_t N, double rho0,
+                                                  double* out) {
     const int64_t p = int64_t(blockIdx.x) * kBlock + threadIdx.x;
     if (p >= n) return;
     double acc = 0.0;
@@ -2086,7 +2030,7 @@ __global__ __launch_bounds__(kBlock) void k_probe(int64_t n, int k, const uint32
         } else {
             double t = 0.0;
 #pragma unroll
-            for (int a = 0; a < Q; ++a) t += double(g[j * L::RS + a]);
+            for (int a = 0; a < Q; ++a) t += double(g[row_at<Q>(j, a, N)]);
             d = rho0 * t;
         }
         acc += double(w[p * k + s]) * d;
@@ -2099,13 +2043,13 @@ __global__ __launch_bounds__(kBlock) void k_macro(StepGeom G, const float* g,
                                                   float* rho, double* drho,
                                                   float* u) {
     using L = Lattice<Q>;
-    constexpr int D = L::D, RS = L::RS;
+    constexpr int D = L::D;
     const int64_t i = int64_t(blockIdx.x) * kBlock + threadIdx.x;
     if (i >= G.N) return;
     double rt = 0.0, mom[3] = {0.0, 0.0, 0.0};
 #pragma unroll
     for (int a = 0; a < Q; ++a) {
-        const double v = double(g[i * RS + a]);
+        const double v = double(g[row_at<Q>(i, a, G.N)]);
         rt += v;
 #pragma unroll
         for (int d = 0; d < D; ++d) mom[d] += v * double(L::c(a, d));
@@ -2149,15 +2093,16 @@ bool step_uses_unions(int Q, int k, int64_t N) {
     return Q == 27 && on && (k == 48 || k == 32 || k == 16) && N < (int64_t(1) << 25);
 }
 
-// D2Q9 scenes run the three-per-lane stencil kernels (12-byte pieces with
-// 32-bit buffer offsets: fewer than 2^26 nodes) unless NAGA_Q9_THREE=0.
-bool q9_three_fits(int64_t N) { return N < (int64_t(1) << 26); }
-bool q9_three(int Q, int64_t N) {
+// D2Q9 scenes run the stencil kernels with two lanes per node (16-byte
+// pieces with 32-bit buffer offsets: fewer than 2^26 nodes) unless
+// NAGA_Q9_THREE=0.
+bool q9_pair_fits(int64_t N) { return N < (int64_t(1) << 26); }
+bool q9_pair(int Q, int64_t N) {
     static const bool on = [] {
         const char* e = std::getenv("NAGA_Q9_THREE");
         return !(e && e[0] == '0');
     }();
-    return on && Q == 9 && q9_three_fits(N);
+    return on && Q == 9 && q9_pair_fits(N);
 }
 
 // Nodes per block of the D3Q27 stencil kernels: the union tile size with
@@ -2205,7 +2150,7 @@ struct PassCfg {
     bool tiles;    // tile unions built (slab index fields are union positions)
     int kmax;      // largest stencil width of the launch's scenes (LDS of the D2Q9 kernels)
     bool ragged;   // per-tile record widths (StepBuffers::tile_ng)
-    bool three;    // D2Q9 stencil passes with three distributions per lane
+    bool pair;     // D2Q9 stencil passes with two lanes per node
 };
 
 template <int Q, int STAGE, int KT>
@@ -2295,36 +2240,25 @@ void launch_pass(int pass, int64_t nb, const StepGeom& G, const StepBuffers& S,
         check_launch("step pass");
         return;
     }
-    if (Q == 9 && c.three &&
+    if (Q == 9 && c.pair &&
         (pass == kP2 || pass == kP3 || pass == kP4 || pass == kP5 ||
          (pass >= kS1 && pass <= kS4))) {
-        // records of the block's nodes (one pad float per node row), then
-        // with tile unions the union rows (36 bytes each)
-        const size_t recs = size_t(kQ9Npb) * ((pass == kP4 ? 2 : 3) * c.kmax + 1) * 4u;
-        const size_t lds = recs + (c.tiles ? size_t(c.ucap) * 36u : 0u);
+        // records of the block's nodes
+        const size_t lds = size_t(kQ9Npb) * q9_pitch(q9_units(c.kmax, pass == kP4 ? 1 : 2)) * 16u;
         const int b = c.gbatch > 0 ? c.gbatch : 8;
         switch (pass) {
-            case kP2: k_p2_3<<<nb, kBlock, recs, st>>>(G, S, c.B); break;
-            case kP3: k_binterp3<true><<<nb, kBlock, 0, st>>>(G, S, c.B); break;
-            case kP5: k_binterp3<false><<<nb, kBlock, 0, st>>>(G, S, c.B); break;
-            case kP4:
-                if (c.tiles) k_p4_3<true><<<nb, kBlock, lds, st>>>(G, S, c.B);
-                else k_p4_3<false><<<nb, kBlock, lds, st>>>(G, S, c.B);
-                break;
-#define NAGA_S3(STG)                                                                          \
-    case kS##STG:                                                                             \
-        if (c.tiles) {                                                                        \
-            if (b == 32) k_stage3<STG, 32, true><<<nb, kBlock, lds, st>>>(G, S, c.B);         \
-            else if (b == 16) k_stage3<STG, 16, true><<<nb, kBlock, lds, st>>>(G, S, c.B);    \
-            else k_stage3<STG, 8, true><<<nb, kBlock, lds, st>>>(G, S, c.B);                  \
-        } else {                                                                              \
-            if (b == 32) k_stage3<STG, 32><<<nb, kBlock, lds, st>>>(G, S, c.B);               \
-            else if (b == 16) k_stage3<STG, 16><<<nb, kBlock, lds, st>>>(G, S, c.B);          \
-            else k_stage3<STG, 8><<<nb, kBlock, lds, st>>>(G, S, c.B);                        \
-        }                                                                                     \
+            case kP2: k_p2_q9<<<nb, kBlock, lds, st>>>(G, S, c.B); break;
+            case kP3: k_binterp_q9<true><<<nb, kBlock, 0, st>>>(G, S, c.B); break;
+            case kP5: k_binterp_q9<false><<<nb, kBlock, 0, st>>>(G, S, c.B); break;
+            case kP4: k_p4_q9<<<nb, kBlock, lds, st>>>(G, S, c.B); break;
+#define NAGA_S9(STG)                                                                 \
+    case kS##STG:                                                                    \
+        if (b == 32) k_stage_q9<STG, 32><<<nb, kBlock, lds, st>>>(G, S, c.B);        \
+        else if (b == 16) k_stage_q9<STG, 16><<<nb, kBlock, lds, st>>>(G, S, c.B);   \
+        else k_stage_q9<STG, 8><<<nb, kBlock, lds, st>>>(G, S, c.B);                 \
         break;
-            NAGA_S3(1) NAGA_S3(2) NAGA_S3(3) NAGA_S3(4)
-#undef NAGA_S3
+            NAGA_S9(1) NAGA_S9(2) NAGA_S9(3) NAGA_S9(4)
+#undef NAGA_S9
             default: break;
         }
         check_launch("step pass");
@@ -2337,7 +2271,8 @@ void launch_pass(int pass, int64_t nb, const StepGeom& G, const StepBuffers& S,
             } else if (p1_uses_dma(Q, c.unions)) {
                 k_p1_dma<<<nb, kP1Chunk, 0, st>>>(G, S, cp, c.B);
             } else {
-                k_p1<Q><<<nb, kP1Block, 0, st>>>(G, S, cp, c.B);
+                if (Q == 9) k_p1_9<<<nb, kP1Block, 0, st>>>(G, S, cp, c.B);
+                else k_p1_27<<<nb, kP1Block, 0, st>>>(G, S, cp, c.B);
             }
             break;
         case kPl:
@@ -2396,7 +2331,7 @@ int64_t pml_part_lo(int Q, int k, int64_t N, int64_t nbulk) {
     return p1_fuses_pml(Q, step_uses_unions(Q, k, N)) ? nbulk / kP1Fused : 0;
 }
 
-void step_block_counts(int Q, const StepGeom& G, const StepBuffers& S, int64_t* nb, int three) {
+void step_block_counts(int Q, const StepGeom& G, const StepBuffers& S, int64_t* nb, int pair) {
     const bool un = step_uses_unions(Q, G.k, G.N);
     const int npb = kBlock / 64 * (Q == 27 ? Lattice<27>::NPW : Lattice<9>::NPW);
     auto lanes = [&](int64_t n) { return (n + npb - 1) / npb; };
@@ -2421,22 +2356,26 @@ void step_block_counts(int Q, const StepGeom& G, const StepBuffers& S, int64_t* 
     nb[kP4] = un ? tiles(G.N) + ns : lanes(G.N);
     nb[kS1] = un ? tiles(G.N) + ns : lanes(G.N);
     nb[kS2] = nb[kS3] = nb[kS4] = un ? tiles(G.nfluid) + ns : lanes(G.nfluid);
-    if (three < 0 ? q9_three(Q, G.N) : (Q == 9 && three > 0)) {
-        auto t84 = [](int64_t n) { return (n + kQ9Npb - 1) / kQ9Npb; };
-        nb[kP4] = nb[kS1] = t84(G.N);
-        nb[kS2] = nb[kS3] = nb[kS4] = t84(G.nfluid);
-        nb[kP2] = (pml && S.n_pml > 0) ? t84(S.n_pml) : 0;
-        nb[kP3] = nb[kP5] = nbnd > 0 ? t84(nbnd) : 0;
+    if (pair < 0 ? q9_pair(Q, G.N) : (Q == 9 && pair > 0)) {
+        auto per = [](int64_t n, int64_t nodes) { return (n + nodes - 1) / nodes; };
+        nb[kP4] = nb[kS1] = per(G.N, kQ9Npb);
+        nb[kS2] = nb[kS3] = nb[kS4] = per(G.nfluid, kQ9Npb);
+        nb[kP2] = (pml && S.n_pml > 0) ? per(S.n_pml, kQ9Npb) : 0;
+        nb[kP3] = per(nbnd, kQ9BndNpb);
     }
     nb[kP5] = nb[kP3];
 }
 
 template <int Q>
 void launch_rk4_stage(int stage, const StepGeom& G, const StepBuffers& S, hipStream_t st) {
+    // a caller's stage 4 may hand in stage outputs whose rest values differ
+    // from y's; within a step they are equal and the two-lane kernel leaves
+    // the rest value alone
+    const bool pair = q9_pair(Q, G.N) && stage != 4;
     int64_t nb[kStepKernels];
-    step_block_counts(Q, G, S, nb);
+    step_block_counts(Q, G, S, nb, pair ? 1 : 0);
     const PassCfg c{ktemplate(G.k), step_uses_unions(Q, G.k, G.N), S.ucap, S.ucap_f, BatchArgs{}, 0,
-                    S.ulist != nullptr, G.k, S.tile_ng != nullptr, q9_three(Q, G.N)};
+                    S.ulist != nullptr, G.k, S.tile_ng != nullptr, pair};
     launch_pass<Q>(kS1 + stage - 1, nb[kS1 + stage - 1], G, S, CollisionParams{}, c, st);
 }
 
@@ -2446,7 +2385,7 @@ void launch_step(const StepGeom& G, const StepBuffers& S, const CollisionParams&
     int64_t nb[kStepKernels];
     step_block_counts(Q, G, S, nb);
     const PassCfg c{ktemplate(G.k), step_uses_unions(Q, G.k, G.N), S.ucap, S.ucap_f, BatchArgs{}, 0,
-                    S.ulist != nullptr, G.k, S.tile_ng != nullptr, q9_three(Q, G.N)};
+                    S.ulist != nullptr, G.k, S.tile_ng != nullptr, q9_pair(Q, G.N)};
     for (int p = 0; p < kStepKernels; ++p) {
         if (ev) hip_check(hipEventRecord(ev[p], st), "event");
         launch_pass<Q>(p, nb[p], G, S, cp, c, st);
@@ -2462,20 +2401,20 @@ void launch_step_batch(const BatchPlan& plan, hipStream_t st) {
         const PassCfg c{plan.k_template, plan.unions, plan.ucap, plan.ucap_f,
                         BatchArgs{plan.dev_scenes, plan.dev_bstart + p * (plan.nscenes + 1),
                                   plan.nscenes},
-                        plan.gather_batch, plan.tiles, plan.kmax, plan.ragged, plan.three};
+                        plan.gather_batch, plan.tiles, plan.kmax, plan.ragged, plan.pair};
         launch_pass<Q>(p, plan.blocks[p], G, S, CollisionParams{}, c, st);
     }
 }
 
 void launch_probe(int Q, int64_t n, int k, const uint32_t* idx, const float* w,
-                  const float* held, const float* g, double rho0, double* out,
+                  const float* held, const float* g, int64_t N, double rho0, double* out,
                   hipStream_t st) {
     if (n == 0) return;
     const int64_t nb = (n + kBlock - 1) / kBlock;
     if (Q == 27)
-        k_probe<27><<<nb, kBlock, 0, st>>>(n, k, idx, w, held, g, rho0, out);
+        k_probe<27><<<nb, kBlock, 0, st>>>(n, k, idx, w, held, g, N, rho0, out);
     else
-        k_probe<9><<<nb, kBlock, 0, st>>>(n, k, idx, w, held, g, rho0, out);
+        k_probe<9><<<nb, kBlock, 0, st>>>(n, k, idx, w, held, g, N, rho0, out);
     check_launch("probe");
 }
 

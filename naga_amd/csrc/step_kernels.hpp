@@ -1,8 +1,11 @@
 // Stepping kernels of the nonlocal LBM on CDNA4 (gfx950).
 //
-// State layout in HBM: each node owns one row of RS floats holding the
-// deviation g_alpha = f_alpha - w_alpha of its Q distributions (AoS).  Rows
-// are ordered [bulk | layer | boundary].  The divergence stencil of fluid
+// State layout in HBM: the deviations g_alpha = f_alpha - w_alpha of a node's
+// Q distributions lie in one row (AoS), rows ordered [bulk | layer |
+// boundary].  D3Q27 rows are padded to 32 floats (one 128-byte line).  D2Q9
+// rows hold the eight moving distributions (32 bytes, four to a line, two
+// 16-byte pieces); the N rest values, which streaming never moves, follow the
+// rows (row_at).  The divergence stencil of fluid
 // node i is a slab of k records {neighbour index, W_x, W_y(, W_z)}.
 //
 // Kernels that gather neighbours map one node to LPN consecutive lanes with
@@ -31,6 +34,17 @@
 #include "naga_common.hpp"
 
 namespace naga_amd {
+
+// Offset of distribution a of node i in a row buffer of N nodes, and the
+// distance between the a-values of consecutive nodes.
+template <int Q>
+NAGA_HD constexpr int64_t row_at(int64_t i, int a, int64_t N) {
+    return Q == 27 ? i * Lattice<27>::RS + a : a == 0 ? 8 * N + i : 8 * i + a - 1;
+}
+template <int Q>
+NAGA_HD constexpr int64_t row_pitch(int a) {
+    return Q == 27 ? Lattice<27>::RS : a == 0 ? 1 : 8;
+}
 
 struct StepGeom {
     int64_t N;        // all nodes
@@ -62,10 +76,6 @@ struct StepBuffers {
     float* Q2v;      // [N][RS] current Q2 value
     const float* slab;    // [nfluid][k][1+D] stencil records
     const float* fslab;   // [nfluid][k][2] filter records {idx, weight}
-    // D2Q9 tile unions: the same records with the index fields holding
-    // positions in the node's tile union (null without unions)
-    const float* uslab;
-    const float* ufslab;
     const float* bslab;   // [nbnd][kb][2] boundary interpolation records
     const float* sigma;   // [nlayer] absorption
     const float* normals; // [nbnd][D] inward normals
@@ -185,13 +195,13 @@ struct BatchPlan {
     bool tiles = false;                 // tile unions built for every scene
     int kmax = 0;                       // largest stencil width over the scenes
     bool ragged = false;                // per-tile record widths in every scene
-    bool three = false;                 // D2Q9: three distributions per lane (else one)
+    bool pair = false;                  // D2Q9: two lanes per node (else one per distribution)
 };
 // Block counts of each pass for one scene (the same counts launch_step
-// uses).  three: D2Q9 lanes per node, 1 for three distributions per lane,
-// 0 for one, -1 for the default (q9_three).
+// uses).  pair: D2Q9 kernels, 1 for two lanes per node, 0 for one lane per
+// distribution, -1 for the default (q9_pair).
 void step_block_counts(int Q, const StepGeom& G, const StepBuffers& S, int64_t* blocks,
-                       int three = -1);
+                       int pair = -1);
 template <int Q>
 void launch_step_batch(const BatchPlan& plan, hipStream_t stream);
 
@@ -199,11 +209,11 @@ void launch_step_batch(const BatchPlan& plan, hipStream_t stream);
 // the tile unions (StepBuffers::ulist/uoff/ucap) and slabs holding union
 // positions: D3Q27, k in {16, 32, 48}, fewer than 2^25 nodes.
 bool step_uses_unions(int Q, int k, int64_t N);
-// Whether the D2Q9 stencil passes run three distributions per lane by
-// default (NAGA_Q9_THREE=0: one), and whether they can (fewer than 2^26
-// nodes: 32-bit buffer offsets of 36-byte rows).
-bool q9_three(int Q, int64_t N);
-bool q9_three_fits(int64_t N);
+// Whether the D2Q9 stencil passes run two lanes per node by default
+// (NAGA_Q9_THREE=0: one lane per distribution), and whether they can (fewer
+// than 2^26 nodes: 32-bit buffer offsets of 32-byte rows).
+bool q9_pair(int Q, int64_t N);
+bool q9_pair_fits(int64_t N);
 // Nodes per union tile (= per block of the union kernels) for stencil width
 // k: 64 for k <= 32 (5.4 union rows per node against 7.0 with 32-node
 // tiles, two blocks per CU; 1.40 against 1.44 ms per step on the 1M-node
@@ -220,11 +230,6 @@ constexpr int means_stride(int Q) { return Q == 27 ? 32 : Q; }
 constexpr int kBUnionCap = 256;   // LDS rows per boundary-interpolation tile
 constexpr int kBTileNodes = 32;   // boundary nodes per boundary-interpolation tile
 constexpr int kUnionRowsMax = 512;  // LDS union rows per block, upper bound
-// D2Q9 tile unions: fluid nodes per tile (the block of the three-per-lane
-// kernels: 21 nodes per wavefront, four wavefronts) and LDS union rows per
-// tile, upper bound (36-byte rows).
-constexpr int kQ9TileNodes = 84;
-constexpr int kQ9UnionRowsMax = 512;
 
 // Per-kernel entry points (used by the profiler and the standalone C-ABI).
 template <int Q>
@@ -233,9 +238,9 @@ void launch_rk4_stage(int stage, const StepGeom& geo, const StepBuffers& buf,
 
 // Density probes (density_observer.cuh:62-113): out[p] = rho0 +
 // sum_s w[p][s] (rho(idx[p][s]) - rho0), with rho the held FP32 density
-// (held != null) or computed fresh from the deviation rows g.
+// (held != null) or computed fresh from the deviation rows g of N nodes.
 void launch_probe(int Q, int64_t n, int k, const uint32_t* idx, const float* w,
-                  const float* held, const float* g, double rho0, double* out,
+                  const float* held, const float* g, int64_t N, double rho0, double* out,
                   hipStream_t stream);
 
 // Fresh macroscopic values from the current state: rho (FP32, reference
