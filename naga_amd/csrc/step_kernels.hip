@@ -170,18 +170,6 @@ __device__ __forceinline__ void store_row9(float* p, int64_t i, int64_t N, const
     p[8 * N + i] = v[0];
 }
 
-__global__ __launch_bounds__(kP1Block) void k_p1_9(StepGeom G, StepBuffers S, CollisionParams cp,
-                                                   BatchArgs B) {
-    const BlockCtx bc = locate(B, G, S);
-    if (B.scenes) cp = B.scenes[bc.scene].cp;
-    const int64_t i = bc.b * kP1Block + threadIdx.x;
-    if (i >= G.N) return;
-    float v[9];
-    load_row9(S.g, i, G.N, v);
-    S.ru[i] = p1_node<9>(G, S, cp, i, FlatRow{v});
-    store_row9(S.A, i, G.N, v);
-}
-
 // ---------------------------------------------------------------------------
 // PML local terms (pml_absorption.inl:551-631) over the nodes whose Q values
 // are used (the layer, plus nodes [0, num_layer) when the layer field reads
@@ -225,6 +213,95 @@ __device__ __forceinline__ float feq_dev32(const float4& ru, int a) {
     const float uu = L::D == 3 ? ru.w * ru.w + (ru.z * ru.z + ru.y * ru.y)
                                : ru.z * ru.z + ru.y * ru.y;
     return float(L::w(a)) * (rt + rho * (uc * inv_cs2 + (uc * uc) * inv_2cs4 - uu));
+}
+
+// Sum over the wavefront (every lane), in a fixed order.
+__device__ __forceinline__ double wave_sum(double v) {
+#define NAGA_DPP_ADD(ctrl)                                                                     \
+    {                                                                                          \
+        const uint64_t b = uint64_t(__double_as_longlong(v));                                  \
+        const uint32_t lo = uint32_t(__builtin_amdgcn_update_dpp(0, int(uint32_t(b)), ctrl,    \
+                                                                 0xf, 0xf, false));            \
+        const uint32_t hi = uint32_t(__builtin_amdgcn_update_dpp(0, int(uint32_t(b >> 32)),    \
+                                                                 ctrl, 0xf, 0xf, false));      \
+        v += __longlong_as_double((long long)((uint64_t(hi) << 32) | lo));                     \
+    }
+    NAGA_DPP_ADD(0xb1)   // quad_perm [1, 0, 3, 2]
+    NAGA_DPP_ADD(0x4e)   // quad_perm [2, 3, 0, 1]
+    NAGA_DPP_ADD(0x141)  // row_half_mirror
+    NAGA_DPP_ADD(0x140)  // row_mirror: each row of 16 lanes holds its sum
+#undef NAGA_DPP_ADD
+    const uint64_t b = uint64_t(__double_as_longlong(v));
+    double t = 0.0;
+#pragma unroll
+    for (int r = 0; r < 64; r += 16) {
+        const uint32_t lo = __builtin_amdgcn_readlane(int(uint32_t(b)), r);
+        const uint32_t hi = __builtin_amdgcn_readlane(int(uint32_t(b >> 32)), r);
+        t += __longlong_as_double((long long)((uint64_t(hi) << 32) | lo));
+    }
+    return t;
+}
+
+// Collision and PML local terms for D2Q9, one node per thread: the collided
+// row stays in registers while the terms of k_pml_local (FP64) are applied to
+// the nodes whose Q values are maintained.  Wavefronts that hold layer nodes
+// write their partial layer sums (part = wavefront).  As a pass of its own,
+// eight dependent rounds of 28 nodes a block, the PML terms took 13 us of a
+// 10k-node scene's 53 us step; here the same loads are one round.
+__global__ __launch_bounds__(kP1Block) void k_p1_9(StepGeom G, StepBuffers S, CollisionParams cp,
+                                                   BatchArgs B) {
+    const BlockCtx bc = locate(B, G, S);
+    if (B.scenes) cp = B.scenes[bc.scene].cp;
+    const int64_t i = bc.b * kP1Block + threadIdx.x;
+    const int64_t w0 = bc.b * kP1Block + (threadIdx.x & ~63u);  // the wavefront's first node
+    const bool layer = i >= G.nbulk && i < G.nfluid;
+    const bool keep = G.nlayer > 0 && (layer || (G.pml_ref && i < G.nlayer && i < G.nfluid));
+    float v[9], p[9];
+    float4 prev = make_float4(0.f, 0.f, 0.f, 0.f);
+    float sigma = 0.0f;
+    if (keep) {  // issued with the row's loads
+        load_row9(S.Qp, i, G.N, p);
+        prev = reinterpret_cast<const float4*>(S.E)[i];
+        sigma = layer ? S.sigma[i - G.nbulk] : 0.0f;
+    }
+    float4 ru = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (i < G.N) {
+        load_row9(S.g, i, G.N, v);
+        ru = p1_node<9>(G, S, cp, i, FlatRow{v});
+        S.ru[i] = ru;
+    }
+    double q1[9], q2[9];
+#pragma unroll
+    for (int a = 0; a < 9; ++a) q1[a] = q2[a] = 0.0;
+    if (keep) {
+        const double hdt = double(G.dt) / 2.0, sig = double(sigma);
+        float o1[9], o2[9];
+#pragma unroll
+        for (int a = 0; a < 9; ++a) {
+            // feq - w now and at the previous step's macroscopic values
+            const double fte = feq_dev<9>(ru, a);
+            q1[a] = (fte + feq_dev<9>(prev, a)) * hdt;
+            q2[a] = (q1[a] + double(p[a])) * hdt;
+            o1[a] = float(q1[a]);
+            o2[a] = float(q2[a]);
+            if (layer)
+                v[a] = float(double(v[a]) -
+                             sig * (3.0 * fte + 3.0 * sig * q1[a] + sig * sig * q2[a]));
+        }
+        reinterpret_cast<float4*>(S.E)[i] = ru;
+        store_row9(S.Qp, i, G.N, o1);
+        if (G.pml_ref ? i < G.nlayer : layer) store_row9(S.Q2v, i, G.N, o2);  // read by the field
+    }
+    if (i < G.N) store_row9(S.A, i, G.N, v);
+    if (G.nlayer == 0 || w0 >= G.nfluid || w0 + 64 <= G.nbulk) return;
+    double mine = 0.0;  // lane c: the wavefront's sum of column c
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int a = 0; a < 9; ++a) {
+        const double s1 = wave_sum(layer ? q1[a] : 0.0), s2 = wave_sum(layer ? q2[a] : 0.0);
+        mine = lane == a ? s1 : lane == 9 + a ? s2 : mine;
+    }
+    if (lane < 18) S.partial[int64_t(lane) * S.nparts + w0 / 64] = mine;
 }
 
 template <int Q>
@@ -319,6 +396,48 @@ __global__ __launch_bounds__(kBlock) void k_pml_field(StepGeom G, StepBuffers S,
     const float q1 = S.Qp[o], q2 = S.Q2v[o];
     S.Gf[row_at<Q>(j, a, G.N)] =
         -2.0f * sig * (q1 - S.means[a]) + sig * sig * (q2 - S.means[means_stride(Q) + a]);
+}
+
+// The same for D2Q9, two lanes per node, with the layer means formed by each
+// block from the partial sums (16 columns; the rest distribution's field is
+// not read): the launch of its own that k_means needs costs more than reading
+// the sums (8 bytes per column and 64 layer nodes) once per 128 rows.
+__global__ __launch_bounds__(kBlock) void k_pml_field_q9(StepGeom G, StepBuffers S, BatchArgs B) {
+    __shared__ double part[kBlock / 16][16];
+    __shared__ float means[16];
+    const BlockCtx bc = locate(B, G, S);
+    const int64_t m = xcd_tile(bc.b, bc.nb) * (kBlock / 2) + (threadIdx.x >> 1);
+    const int q = threadIdx.x & 1;
+    const bool in = m < G.nlayer;
+    const int64_t j = G.nbulk + m, p = G.pml_ref ? m : j;
+    float sig = 0.0f;
+    float4 q1 = make_float4(0.f, 0.f, 0.f, 0.f), q2 = q1;
+    if (in) {  // in flight while the means are formed
+        sig = S.sigma[m];
+        q1 = reinterpret_cast<const float4*>(S.Qp)[2 * p + q];
+        q2 = reinterpret_cast<const float4*>(S.Q2v)[2 * p + q];
+    }
+    const int c = threadIdx.x & 15, r = threadIdx.x >> 4;  // column: Q1 of alpha 1 .. 8, then Q2
+    const double* col = S.partial + int64_t((c >> 3) * 9 + 1 + (c & 7)) * S.nparts;
+    double s = 0.0;
+#pragma unroll 4
+    for (int t = S.part_lo + r; t < S.nparts; t += kBlock / 16) s += col[t];
+    part[r][c] = s;
+    __syncthreads();
+    if (threadIdx.x < 16) {
+        double t = 0.0;
+        for (int e = 0; e < kBlock / 16; ++e) t += part[e][threadIdx.x];
+        means[threadIdx.x] = float(t / double(G.nlayer));
+    }
+    __syncthreads();
+    if (!in) return;
+    const float* m1 = means + 4 * q;
+    const float* m2 = means + 8 + 4 * q;
+    auto field = [&](float a, float b, int e) {
+        return -2.0f * sig * (a - m1[e]) + sig * sig * (b - m2[e]);
+    };
+    reinterpret_cast<float4*>(S.Gf)[2 * j + q] = make_float4(
+        field(q1.x, q2.x, 0), field(q1.y, q2.y, 1), field(q1.z, q2.z, 2), field(q1.w, q2.w, 3));
 }
 
 // ---------------------------------------------------------------------------
@@ -2277,12 +2396,13 @@ void launch_pass(int pass, int64_t nb, const StepGeom& G, const StepBuffers& S,
             break;
         case kPl:
             if (v4) k_pml_local_v4<<<nb, kBlock, 0, st>>>(G, S, c.B);
-            else k_pml_local<Q><<<nb, kBlock, 0, st>>>(G, S, c.B);
+            else k_pml_local<27><<<nb, kBlock, 0, st>>>(G, S, c.B);
             break;
-        case kPm: k_means<Q><<<nb, 256, 0, st>>>(G, S, c.B); break;
+        case kPm: k_means<27><<<nb, 256, 0, st>>>(G, S, c.B); break;
         case kPf:
             if (v4) k_pml_field_v4<<<nb, kBlock, 0, st>>>(G, S, c.B);
-            else k_pml_field<Q><<<nb, kBlock, 0, st>>>(G, S, c.B);
+            else if (Q == 27) k_pml_field<27><<<nb, kBlock, 0, st>>>(G, S, c.B);
+            else k_pml_field_q9<<<nb, kBlock, 0, st>>>(G, S, c.B);
             break;
         case kP2:
             if (c.ktmpl == 32) k_p2<Q, 32><<<nb, kBlock, 0, st>>>(G, S, c.B);
@@ -2319,15 +2439,16 @@ int ktemplate(int k) { return (k == 48 || k == 32 || k == 16) ? k : 0; }
 }  // namespace
 
 int64_t pml_parts(int Q, int k, int64_t N, int64_t nfluid, int64_t n_rq) {
+    if (Q == 9) return (nfluid + 63) / 64;  // a wavefront of k_p1_9
     if (p1_fuses_pml(Q, step_uses_unions(Q, k, N))) return (nfluid + kP1Fused - 1) / kP1Fused;
     const int64_t per = step_uses_unions(Q, k, N)
                             ? int64_t(kV4Nodes) * kPmlRounds
-                            : int64_t(kBlock / 64) * (Q == 27 ? Lattice<27>::NPW : Lattice<9>::NPW) *
-                                  kPmlRounds;
+                            : int64_t(kBlock / 64) * Lattice<27>::NPW * kPmlRounds;
     return (n_rq + per - 1) / per;
 }
 
 int64_t pml_part_lo(int Q, int k, int64_t N, int64_t nbulk) {
+    if (Q == 9) return nbulk / 64;
     return p1_fuses_pml(Q, step_uses_unions(Q, k, N)) ? nbulk / kP1Fused : 0;
 }
 
@@ -2340,13 +2461,16 @@ void step_block_counts(int Q, const StepGeom& G, const StepBuffers& S, int64_t* 
     auto tiles32 = [&](int64_t n) { return (n + kV4Nodes - 1) / kV4Nodes; };
     const bool pml = G.nlayer > 0 && S.n_rq > 0;
     const int64_t nbnd = G.N - G.nfluid;
-    const bool fused = p1_fuses_pml(Q, un);
-    nb[kP1] = fused ? (G.N + kP1Fused - 1) / kP1Fused
+    const bool fused = Q == 9 || p1_fuses_pml(Q, un);
+    nb[kP1] = Q == 27 && fused ? (G.N + kP1Fused - 1) / kP1Fused
                     : p1_uses_dma(Q, un) ? (G.N + kP1Chunk - 1) / kP1Chunk
                                          : (G.N + kP1Block - 1) / kP1Block;
     nb[kPl] = (pml && !fused) ? S.nparts : 0;
-    nb[kPm] = pml ? 2 * Q : 0;
-    nb[kPf] = pml ? (un ? tiles32(G.nlayer) : lanes(G.nlayer)) : 0;
+    // (D2Q9: the means are formed in the field pass)
+    nb[kPm] = pml && Q == 27 ? 2 * Q : 0;
+    nb[kPf] = !pml ? 0
+              : Q == 9 ? (G.nlayer + kBlock / 2 - 1) / (kBlock / 2)
+                       : un ? tiles32(G.nlayer) : lanes(G.nlayer);
     nb[kP2] = (pml && S.n_pml > 0)
                   ? (un ? (S.ulist ? S.n_ptiles : tiles(S.n_pml)) : lanes(S.n_pml))
                   : 0;
