@@ -232,16 +232,34 @@ void Engine::init_domain(const float* pts, int64_t nbulk, int64_t nlayer, int64_
     filt_.allocate(N * k);
     launch_filter_weights(D, pts_.get(), N, idx_.get(), k, cfg_.h, filt_.get(), st, kvar_.get());
     if (kvar_.size() == size_t(N)) launch_self_past_k(N, k, kvar_.get(), idx_.get(), st);
+    // the step's records: the stencils, padded to the kernels' width
+    const int ks = step_width(Q, k, N);
+    geo_.k = ks;
+    geo_.pml64 = k != 16 && k != 32 && k != 48;
+    const uint32_t* sidx = idx_.get();
+    const float *sW = W_.get(), *sfilt = filt_.get();
+    DeviceBuffer<uint32_t> idx_pad;
+    DeviceBuffer<float> W_pad, filt_pad;
+    if (ks != k) {
+        idx_pad.allocate(nfluid * ks);
+        W_pad.allocate(nfluid * ks * D);
+        filt_pad.allocate(nfluid * ks);
+        launch_pad_entries(nfluid, k, ks, D, sidx, sW, idx_pad.get(), W_pad.get(), st);
+        launch_pad_entries(nfluid, k, ks, 1, sidx, sfilt, idx_pad.get(), filt_pad.get(), st);
+        sidx = idx_pad.get();
+        sW = W_pad.get();
+        sfilt = filt_pad.get();
+    }
     if (Q == 9) {
         slab_.allocate(nfluid * q9_units(k, 2) * 4);
         launch_make_slab_q9(nfluid, k, 2, idx_.get(), W_.get(), slab_.get(), st);
         fslab_.allocate(nfluid * q9_units(k, 1) * 4);
         launch_make_slab_q9(nfluid, k, 1, idx_.get(), filt_.get(), fslab_.get(), st);
     } else {
-        slab_.allocate(nfluid * k * (1 + D));
-        launch_make_slab(nfluid, k, D, idx_.get(), W_.get(), slab_.get(), st);
-        fslab_.allocate(nfluid * k * 2);
-        launch_make_slab(nfluid, k, 1, idx_.get(), filt_.get(), fslab_.get(), st);
+        slab_.allocate(nfluid * ks * (1 + D));
+        launch_make_slab(nfluid, ks, D, sidx, sW, slab_.get(), st);
+        fslab_.allocate(nfluid * ks * 2);
+        launch_make_slab(nfluid, ks, 1, sidx, sfilt, fslab_.get(), st);
     }
     ucap_ = 0;
     ucap_f_ = 0;
@@ -273,12 +291,12 @@ void Engine::init_domain(const float* pts, int64_t nbulk, int64_t nlayer, int64_
     if (!(un_env && un_env[0] == '0') && step_uses_unions(Q, k, N) && nfluid > 0) {
         // tile unions; slab index fields become union positions
         std::vector<int32_t> last_counts;  // union rows per tile of the last set built
-        const int T = union_tile_nodes(k);
+        const int T = union_tile_nodes(ks);
         tile_nodes_ = T;
         const int64_t ntiles = (nfluid + T - 1) / T;
         const char* env = std::getenv("NAGA_UCAP");
         const int cap = env ? std::max(0, std::min(std::atoi(env), kUnionRowsMax))
-                            : union_cap_default(k);
+                            : union_cap_default(ks);
         // tiles over the cap are split into two half-tile unions when
         // those fit (NAGA_SPLIT=0: never)
         const char* sp_env = std::getenv("NAGA_SPLIT");
@@ -292,7 +310,7 @@ void Engine::init_domain(const float* pts, int64_t nbulk, int64_t nlayer, int64_
             DeviceBuffer<int32_t> counts(ntiles);
             last_counts.clear();
             usplit.allocate(ntiles);
-            launch_tile_unions(nfluid, k, T, idx_in, split ? cap : 0, counts.get(), usplit.get(),
+            launch_tile_unions(nfluid, ks, T, idx_in, split ? cap : 0, counts.get(), usplit.get(),
                                nullptr, nullptr, nullptr, 0, nullptr, 0, st);
             std::vector<int32_t> hc(ntiles), hs(ntiles), splits;
             counts.download(hc.data(), ntiles, st);
@@ -312,7 +330,7 @@ void Engine::init_domain(const float* pts, int64_t nbulk, int64_t nlayer, int64_
             }
             uoff = to_device(off, st);
             ulist.allocate(std::max<int64_t>(off[ntiles], 1));
-            launch_tile_unions(nfluid, k, T, idx_in, split ? cap : 0, nullptr, usplit.get(),
+            launch_tile_unions(nfluid, ks, T, idx_in, split ? cap : 0, nullptr, usplit.get(),
                                uoff.get(), ulist.get(), slab_a, nca, slab_b, ncb, st);
             n_split = int64_t(splits.size());
             split_tiles = to_device(splits.empty() ? std::vector<int32_t>{0} : splits, st);
@@ -323,27 +341,27 @@ void Engine::init_domain(const float* pts, int64_t nbulk, int64_t nlayer, int64_
         // mapped to a node outside the layer), about 60% of the full union.
         DeviceBuffer<float> slab2;
         if (nlayer > 0) {
-            DeviceBuffer<uint32_t> idx2(nfluid * k);
+            DeviceBuffer<uint32_t> idx2(nfluid * ks);
             const uint32_t zero_row = nbnd > 0 ? uint32_t(nfluid) : 0u;
-            launch_layer_only(nfluid * k, idx_.get(), uint32_t(nbulk), uint32_t(nfluid), zero_row,
+            launch_layer_only(nfluid * ks, sidx, uint32_t(nbulk), uint32_t(nfluid), zero_row,
                               idx2.get(), st);
-            slab2.allocate(nfluid * k * (1 + D));
-            launch_make_slab(nfluid, k, D, idx_.get(), W_.get(), slab2.get(), st);
+            slab2.allocate(nfluid * ks * (1 + D));
+            launch_make_slab(nfluid, ks, D, sidx, sW, slab2.get(), st);
             build(idx2.get(), slab2.get(), D, nullptr, 0, p2ulist_, p2uoff_, p2usplit_,
                   p2split_tiles_, p2split_of_, p2n_split_);
-            p2slab_.allocate(nfluid * packed_div_units(k) * 4);
-            launch_pack_div_records(nfluid, k, slab2.get(), p2slab_.get(), st);
+            p2slab_.allocate(nfluid * packed_div_units(ks) * 4);
+            launch_pack_div_records(nfluid, ks, slab2.get(), p2slab_.get(), st);
             NAGA_HIP(hipStreamSynchronize(st));
         }
-        const int maxu = build(idx_.get(), slab_.get(), D, fslab_.get(), 1, ulist_, uoff_,
+        const int maxu = build(sidx, slab_.get(), D, fslab_.get(), 1, ulist_, uoff_,
                                usplit_, split_tiles_, split_of_, n_split_);
         // the union kernels copy records into LDS as they lie: packed rows
         // (16-bit union positions, an odd number of 16-byte units per node)
         // keep the records of consecutive nodes in distinct LDS banks
-        DeviceBuffer<float> ps(nfluid * packed_div_units(k) * 4),
-            pf(nfluid * packed_filter_units(k) * 4);
-        launch_pack_div_records(nfluid, k, slab_.get(), ps.get(), st);
-        launch_pack_filter_records(nfluid, k, fslab_.get(), pf.get(), st);
+        DeviceBuffer<float> ps(nfluid * packed_div_units(ks) * 4),
+            pf(nfluid * packed_filter_units(ks) * 4);
+        launch_pack_div_records(nfluid, ks, slab_.get(), ps.get(), st);
+        launch_pack_filter_records(nfluid, ks, fslab_.get(), pf.get(), st);
         NAGA_HIP(hipStreamSynchronize(st));
         slab_ = std::move(ps);
         fslab_ = std::move(pf);
@@ -388,7 +406,7 @@ void Engine::init_domain(const float* pts, int64_t nbulk, int64_t nlayer, int64_
                 const int64_t a = t * T, b = std::min<int64_t>(a + T, nfluid);
                 int m = 1;
                 for (int64_t i = a; i < b; ++i) m = std::max(m, (int(hk[size_t(i)]) + 7) / 8);
-                ng[size_t(t)] = std::min(m, k / 8);
+                ng[size_t(t)] = std::min(m, ks / 8);
                 ro[size_t(t) + 1] = ro[size_t(t)] + (b - a) * ragged_div_units(ng[size_t(t)]);
                 fo[size_t(t) + 1] = fo[size_t(t)] + (b - a) * ragged_filter_units(ng[size_t(t)]);
             }
@@ -397,13 +415,13 @@ void Engine::init_domain(const float* pts, int64_t nbulk, int64_t nlayer, int64_
             frec_off_ = to_device(fo, st);
             DeviceBuffer<float> rs(size_t(ro[size_t(ntiles)]) * 4),
                 rf(size_t(fo[size_t(ntiles)]) * 4);
-            launch_ragged_records(nfluid, T, packed_div_units(k), 7, tile_ng_.get(),
+            launch_ragged_records(nfluid, T, packed_div_units(ks), 7, tile_ng_.get(),
                                   rec_off_.get(), slab_.get(), rs.get(), st);
-            launch_ragged_records(nfluid, T, packed_filter_units(k), 3, tile_ng_.get(),
+            launch_ragged_records(nfluid, T, packed_filter_units(ks), 3, tile_ng_.get(),
                                   frec_off_.get(), fslab_.get(), rf.get(), st);
             if (p2slab_.size() > 0) {
                 DeviceBuffer<float> r2(size_t(ro[size_t(ntiles)]) * 4);
-                launch_ragged_records(nfluid, T, packed_div_units(k), 7, tile_ng_.get(),
+                launch_ragged_records(nfluid, T, packed_div_units(ks), 7, tile_ng_.get(),
                                       rec_off_.get(), p2slab_.get(), r2.get(), st);
                 NAGA_HIP(hipStreamSynchronize(st));
                 p2slab_ = std::move(r2);
@@ -1085,7 +1103,8 @@ void Batch::rebuild() {
         const bool tiles = tiles_of(e);
         const bool pair = pair_of(e);
         const bool ragged = e->scene_desc().S.tile_ng != nullptr;
-        return Q * 1000 + (un ? e->stencil_k() : 0) + (tiles ? 500 : 0) + (pair ? 250 : 0) +
+        const bool pml64 = Q == 27 && e->scene_desc().G.pml64 != 0;
+        return Q * 1000 + (pml64 ? 100000 : 0) + (un ? e->stencil_k() : 0) + (tiles ? 500 : 0) + (pair ? 250 : 0) +
                (ragged ? 125 : 0);
     };
     std::vector<int> keys;
@@ -1132,10 +1151,11 @@ void Batch::rebuild() {
         }
         for (int p = 0; p < kStepKernels; ++p) P.blocks[p] = bstart[size_t(p) * (n + 1) + n];
         P.unions = step_uses_unions(g.Q, g.members[0]->stencil_k(), g.members[0]->nodes());
-        P.k_template = (kcommon == 48 || kcommon == 32 || kcommon == 16) ? kcommon : 0;
+        P.k_template = step_k_template(kcommon);
         P.gather_batch = gather_batch_;
         P.tiles = g.tiles;
         P.ragged = descs[0].S.tile_ng != nullptr;
+        P.pml64 = descs[0].G.pml64 != 0;
         for (const SceneDesc& d : descs)
             require((d.S.ulist != nullptr) == P.tiles, "scenes with and without tile unions");
         require(!P.unions || P.k_template != 0, "four-per-lane scenes need a common k");

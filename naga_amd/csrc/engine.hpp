@@ -88,7 +88,7 @@ class Engine {
     void finish_batched_step();
     bool has_domain() const { return ready_; }
     Batch* batch = nullptr;  // the batch holding this scene, if any
-    int stencil_k() const { return cfg_.k; }
+    int stencil_k() const { return geo_.k; }  // of the step's records
     int64_t fluid_nodes() const { return nfluid_; }
 
     int64_t nodes() const { return N_; }

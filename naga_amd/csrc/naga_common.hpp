@@ -46,26 +46,22 @@ inline void require(bool ok, const std::string& msg) {
 // Divergence records of a node with tile unions, packed: per group of 8
 // records, six 16-byte units of weights (record r's x, y, z at floats 3r ..
 // 3r + 2) and one unit of eight 16-bit union positions (record 2m in the
-// low half of dword m, 2m + 1 in the high half); then one zero unit, which
-// makes the row length odd in units so the records of consecutive nodes
+// low half of dword m, 2m + 1 in the high half); then one or two zero units,
+// which make the row length odd in units so the records of consecutive nodes
 // fall in distinct LDS banks.  k must be a multiple of 8.
-constexpr int packed_div_units(int k) { return 7 * (k / 8) + 1; }
+constexpr int ragged_div_units(int ng) { return 7 * ng + ((ng & 1) ? 2 : 1); }
+constexpr int packed_div_units(int k) { return ragged_div_units(k / 8); }
 // 16-byte units of one D2Q9 node's records (launch_make_slab_q9): per group of
 // four records one unit of indices and one per weight; and the LDS row that
 // holds them, an odd number of units (distinct banks for consecutive nodes).
 NAGA_HD constexpr int q9_units(int k, int ncomp) { return (1 + ncomp) * ((k + 3) / 4); }
 NAGA_HD constexpr int q9_pitch(int units) { return units | 1; }
 // Filter records of a node with tile unions, packed like the divergence
-// records: per group of 8 records two units of weights and one unit of 16-bit positions, then
-// one zero unit.
-constexpr int packed_filter_units(int k) { return 3 * (k / 8) + 1; }
-// Record rows of a tile whose nodes use ng groups of 8 records (per-tile
-// stencil widths): the groups' units plus one or two zero units, an odd
-// number of 16-byte units per node (distinct LDS banks for the nodes of a
-// wavefront); equal to the fixed-width rows for ng = k / 8 with k in
-// {16, 32, 48}.
-constexpr int ragged_div_units(int ng) { return 7 * ng + ((ng & 1) ? 2 : 1); }
+// records: per group of 8 records two units of weights and one unit of
+// 16-bit positions, then the zero units.  (ragged_*: rows of a tile whose
+// nodes use ng groups, per-tile stencil widths.)
 constexpr int ragged_filter_units(int ng) { return 3 * ng + ((ng & 1) ? 2 : 1); }
+constexpr int packed_filter_units(int k) { return ragged_filter_units(k / 8); }
 
 #if defined(__HIPCC__)
 inline void hip_check(hipError_t e, const char* what) {

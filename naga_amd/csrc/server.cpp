@@ -84,7 +84,8 @@ size_t Server::footprint(int Q, int k, int64_t n) {
     const int D = Q == 9 ? 2 : 3, RS = Q == 9 ? Lattice<9>::RS : Lattice<27>::RS;
     // nine [N][RS] state buffers, stencil products (idx, W, filter, slabs),
     // setup transients, per-node scalars; 25% margin
-    const double per = 36.0 * RS + double(k) * (4.0 + 4.0 * D + 4.0 + 4.0 * (1 + D) + 8.0 + 8.0) +
+    const int ks = step_width(Q, k, n);  // of the step's records
+    const double per = 36.0 * RS + double(ks) * (4.0 + 4.0 * D + 4.0 + 4.0 * (1 + D) + 8.0 + 8.0) +
                        96.0;
     return size_t(1.25 * per * double(n)) + (size_t(8) << 20);
 }

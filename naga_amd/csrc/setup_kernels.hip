@@ -857,6 +857,16 @@ __global__ void k_filter(int D, const float* pts, int64_t n, const uint32_t* idx
     }
 }
 
+__global__ void k_pad_entries(int64_t n, int k, int ks, int nc, const uint32_t* idx,
+                              const float* w, uint32_t* idx_out, float* w_out) {
+    const int64_t e = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (e >= n * ks) return;
+    const int64_t i = e / ks;
+    const int s = int(e - i * ks);
+    idx_out[e] = s < k ? idx[i * k + s] : uint32_t(i);
+    for (int c = 0; c < nc; ++c) w_out[e * nc + c] = s < k ? w[(i * k + s) * nc + c] : 0.0f;
+}
+
 __global__ void k_make_slab(int64_t n, int k, int nc, const uint32_t* idx,
                             const float* w, float* slab) {
     const int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -890,8 +900,8 @@ __global__ void k_pack_div_records(int64_t n, int k, const float* src, uint32_t*
     const int u = word / 4, g = u / 7, w = u % 7;
     const float* rec = src + (i * k + 8 * g) * 4;  // the group's 8 records
     uint32_t v = 0;
-    if (u == units - 1) {
-        v = 0;  // padding unit
+    if (u >= 7 * (k / 8)) {
+        v = 0;  // padding units
     } else if (w < 6) {
         const int f = 4 * w + word % 4;  // float f of the group's 24 weights
         v = __float_as_uint(rec[(f / 3) * 4 + 1 + f % 3]);
@@ -914,8 +924,8 @@ __global__ void k_pack_filter_records(int64_t n, int k, const float* src, uint32
     const int u = word / 4, g = u / 3, w = u % 3;
     const float* rec = src + (i * k + 8 * g) * 2;  // the group's 8 {position, weight}
     uint32_t v = 0;
-    if (u == units - 1) {
-        v = 0;  // padding unit
+    if (u >= 3 * (k / 8)) {
+        v = 0;  // padding units
     } else if (w < 2) {
         v = __float_as_uint(rec[(4 * w + word % 4) * 2 + 1]);
     } else {
@@ -1542,6 +1552,13 @@ void launch_filter_weights(int D, const float* pts, int64_t n, const uint32_t* i
     if (n == 0) return;
     k_filter<<<(n + 255) / 256, 256, 0, st>>>(D, pts, n, idx, k, h / 2.5, kvar, wf);
     hip_check(hipGetLastError(), "filter weights");
+}
+
+void launch_pad_entries(int64_t n, int k, int ks, int nc, const uint32_t* idx, const float* w,
+                        uint32_t* idx_out, float* w_out, hipStream_t st) {
+    if (n == 0) return;
+    k_pad_entries<<<(n * ks + 255) / 256, 256, 0, st>>>(n, k, ks, nc, idx, w, idx_out, w_out);
+    hip_check(hipGetLastError(), "stencil padding");
 }
 
 void launch_make_slab(int64_t n, int k, int nc, const uint32_t* idx, const float* w,

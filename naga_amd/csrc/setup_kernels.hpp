@@ -146,6 +146,11 @@ void launch_filter_weights(int D, const float* pts, int64_t n,
                            const uint32_t* idx, int k, double h, float* wf,
                            hipStream_t stream, const uint8_t* kvar = nullptr);
 
+// Rows of ks >= k entries from rows of k: entry s < k of node i is copied, the
+// others point at i with zero weights (ncomp weights per entry).
+void launch_pad_entries(int64_t n, int k, int ks, int ncomp, const uint32_t* idx, const float* w,
+                        uint32_t* idx_out, float* w_out, hipStream_t stream);
+
 // Interleave indices and weights into slab records:
 // rec[(i*k + s)*(1+ncomp) + 0] = idx bits, then ncomp weights.
 void launch_make_slab(int64_t n, int k, int ncomp, const uint32_t* idx,

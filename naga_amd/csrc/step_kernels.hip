@@ -182,37 +182,20 @@ __device__ __forceinline__ void store_row9(float* p, int64_t i, int64_t N, const
 constexpr int kPmlRounds = 8;
 
 // feq_a - w_a (equilibrium_distribution.cuh:52-63, cancellation-free) at
-// rho = 1 + rt and velocity u, ru = (rt, u).
-template <int Q>
-__device__ __forceinline__ double feq_dev(const float4& ru, int a) {
+// rho = 1 + rt and velocity u, ru = (rt, u), in precision P (FP32: the terms
+// are deviations of order 1e-3 whose rounding is that of the rows they
+// update).
+template <int Q, class P = double>
+__device__ __forceinline__ P feq_dev(const float4& ru, int a) {
     using L = Lattice<Q>;
     constexpr double cs2 = kCsLat * kCsLat;
-    constexpr double inv_cs2 = 1.0 / cs2, inv_2cs4 = 1.0 / (2.0 * cs2 * cs2);
-    const double rt = double(ru.x), rho = 1.0 + rt;
-    const double u0 = ru.y, u1 = ru.z, u2 = ru.w;
-    const double uc = L::D == 3 ? u0 * double(L::c(a, 0)) + u1 * double(L::c(a, 1)) +
-                                      u2 * double(L::c(a, 2))
-                                : u0 * double(L::c(a, 0)) + u1 * double(L::c(a, 1));
-    const double uu = L::D == 3 ? u2 * u2 + (u1 * u1 + u0 * u0) : u1 * u1 + u0 * u0;
-    return L::w(a) * (rt + rho * (uc * inv_cs2 + (uc * uc) * inv_2cs4 - uu));
-}
-
-// The same in FP32 (the fused collision pass): the terms are deviations of
-// order 1e-3 whose FP32 rounding is that of the FP32 rows they update.
-template <int Q>
-__device__ __forceinline__ float feq_dev32(const float4& ru, int a) {
-    using L = Lattice<Q>;
-    constexpr float cs2 = float(kCsLat * kCsLat);
-    constexpr float inv_cs2 = float(1.0 / (kCsLat * kCsLat));
-    constexpr float inv_2cs4 = float(1.0 / (2.0 * kCsLat * kCsLat * kCsLat * kCsLat));
-    (void)cs2;
-    const float rt = ru.x, rho = 1.0f + rt;
-    const float uc = L::D == 3 ? ru.y * float(L::c(a, 0)) + ru.z * float(L::c(a, 1)) +
-                                     ru.w * float(L::c(a, 2))
-                               : ru.y * float(L::c(a, 0)) + ru.z * float(L::c(a, 1));
-    const float uu = L::D == 3 ? ru.w * ru.w + (ru.z * ru.z + ru.y * ru.y)
-                               : ru.z * ru.z + ru.y * ru.y;
-    return float(L::w(a)) * (rt + rho * (uc * inv_cs2 + (uc * uc) * inv_2cs4 - uu));
+    constexpr P inv_cs2 = P(1.0 / cs2), inv_2cs4 = P(1.0 / (2.0 * cs2 * cs2));
+    const P rt = P(ru.x), rho = P(1) + rt;
+    const P u0 = ru.y, u1 = ru.z, u2 = ru.w;
+    const P uc = L::D == 3 ? u0 * P(L::c(a, 0)) + u1 * P(L::c(a, 1)) + u2 * P(L::c(a, 2))
+                           : u0 * P(L::c(a, 0)) + u1 * P(L::c(a, 1));
+    const P uu = L::D == 3 ? u2 * u2 + (u1 * u1 + u0 * u0) : u1 * u1 + u0 * u0;
+    return P(L::w(a)) * (rt + rho * (uc * inv_cs2 + (uc * uc) * inv_2cs4 - uu));
 }
 
 // Sum over the wavefront (every lane), in a fixed order.
@@ -1105,7 +1088,7 @@ __global__ __launch_bounds__(kP1Chunk) __attribute__((amdgpu_waves_per_eu(3))) v
 // per block of 64 nodes (as k_p1_dma, whose independent one-wave blocks
 // overlap each other's memory and FP64 work): the wave collides its rows in
 // LDS, then its 64 lanes, eight per node (four distributions each), apply
-// the PML local terms of k_pml_local_v4 in FP32 to the block's nodes whose
+// the PML local terms of k_pml_local_v4 (in precision P, pml64) to the nodes whose
 // Q values are maintained, subtracting the layer damping from the collided
 // rows before they are stored.  Blocks that hold layer nodes write their
 // partial layer sums (column-major, part = block).  Saves the PML pass's
@@ -1120,6 +1103,7 @@ __device__ __forceinline__ bool pml_maintained(const StepGeom& G, int64_t i) {
     return (i >= G.nbulk && i < G.nfluid) || (G.pml_ref && i < G.nlayer && i < G.nfluid);
 }
 
+template <class P>
 __global__ __launch_bounds__(kP1Fused) __attribute__((amdgpu_waves_per_eu(3))) void k_p1_pml(
     StepGeom G, StepBuffers S, CollisionParams cp, BatchArgs B) {
     __shared__ float4 buf[8 * kP1Chunk];  // collided rows, XorRow layout
@@ -1146,7 +1130,7 @@ __global__ __launch_bounds__(kP1Fused) __attribute__((amdgpu_waves_per_eu(3))) v
     const int slot = t / kV4Lanes, q = t % kV4Lanes;
     double s1[4] = {0.0, 0.0, 0.0, 0.0}, s2[4] = {0.0, 0.0, 0.0, 0.0};
     if (any_pml) {
-        const float hdt = G.dt * 0.5f;
+        const P hdt = P(G.dt) * P(0.5);
         const __amdgpu_buffer_rsrc_t rQp = rsrc(S.Qp, rows);
         constexpr int kRounds = kP1Chunk / 8;
 #if NAGA_P1_PREFETCH
@@ -1173,10 +1157,10 @@ __global__ __launch_bounds__(kP1Fused) __attribute__((amdgpu_waves_per_eu(3))) v
             const bool layer = i >= G.nbulk && i < G.nfluid;
 #if NAGA_P1_PREFETCH
             const float4 p4 = qp[rd];
-            const float sig = sg[rd];
+            const P sig = sg[rd];
 #else
             const float4 p4 = ld4(rQp, own);
-            const float sig = layer ? S.sigma[i - G.nbulk] : 0.0f;
+            const P sig = layer ? S.sigma[i - G.nbulk] : 0.0f;
 #endif
             const float4 ru = rul[n];
             float4& a4 = buf[q * kP1Chunk + (n ^ q)];
@@ -1190,13 +1174,14 @@ __global__ __launch_bounds__(kP1Fused) __attribute__((amdgpu_waves_per_eu(3))) v
                     set(qo, e, 0.0f);
                     continue;
                 }
-                const float fte = feq_dev32<27>(ru, a);
-                const float q1 = (fte + feq_dev32<27>(prv, a)) * hdt;
-                const float q2 = (q1 + get(p4, e)) * hdt;
-                set(po, e, q1);
-                set(qo, e, q2);
+                const P fte = feq_dev<27, P>(ru, a);
+                const P q1 = (fte + feq_dev<27, P>(prv, a)) * hdt;
+                const P q2 = (q1 + P(get(p4, e))) * hdt;
+                set(po, e, float(q1));
+                set(qo, e, float(q2));
                 if (layer) {
-                    set(av, e, get(av, e) - sig * (3.0f * fte + 3.0f * sig * q1 + sig * sig * q2));
+                    set(av, e, float(P(get(av, e)) -
+                                     sig * (P(3) * fte + P(3) * sig * q1 + sig * sig * q2)));
                     s1[e] += double(q1);
                     s2[e] += double(q2);
                 }
@@ -2202,14 +2187,20 @@ int stage_batch() {
     return b;
 }
 
-// The four-per-lane D3Q27 kernels need k in {16, 32, 48} and 32-bit row offsets.
-// NAGA_V4=0 selects the one-per-lane kernels.
+// The four-per-lane D3Q27 kernels serve stencil widths of 12 to 48 (padded to
+// a multiple of 8, see step_width) and 32-bit row offsets.  NAGA_V4=0 selects
+// the one-per-lane kernels.
 bool step_uses_unions(int Q, int k, int64_t N) {
     static const bool on = [] {
         const char* e = std::getenv("NAGA_V4");
         return !(e && e[0] == '0');
     }();
-    return Q == 27 && on && (k == 48 || k == 32 || k == 16) && N < (int64_t(1) << 25);
+    return Q == 27 && on && k >= 12 && k <= 48 && N < (int64_t(1) << 25);
+}
+
+int step_width(int Q, int k, int64_t N) {
+    if (!step_uses_unions(Q, k, N)) return k;
+    return k <= 16 ? 16 : (k + 7) / 8 * 8;
 }
 
 // D2Q9 scenes run the stencil kernels with two lanes per node (16-byte
@@ -2260,7 +2251,7 @@ enum Pass { kP1, kPl, kPm, kPf, kP2, kP3, kP4, kS1, kS2, kS3, kS4, kP5 };
 // How a pass is launched: kernel template choices shared by every scene of
 // the launch, and the batch table (or none).
 struct PassCfg {
-    int ktmpl;     // K template: 32, 16 or 0 (runtime k)
+    int ktmpl;     // K template: a multiple of 8 from 16 to 48, or 0 (runtime k)
     bool unions;   // D3Q27 four-per-lane kernels with tile unions
     int ucap;      // LDS union rows (dynamic shared memory / 128 B)
     int ucap_f;    // the same for the filter pass
@@ -2270,6 +2261,7 @@ struct PassCfg {
     int kmax;      // largest stencil width of the launch's scenes (LDS of the D2Q9 kernels)
     bool ragged;   // per-tile record widths (StepBuffers::tile_ng)
     bool pair;     // D2Q9 stencil passes with two lanes per node
+    bool pml64;    // StepGeom::pml64
 };
 
 template <int Q, int STAGE, int KT>
@@ -2285,7 +2277,7 @@ void launch_stage_scalar(int64_t nb, const StepGeom& G, const StepBuffers& S, Ba
 }
 
 // The D3Q27 four-per-lane kernels of the stencil passes for one stencil
-// width K (16, 32 or 48) and NPB nodes per block.
+// width K (a multiple of 8, 16 to 48) and NPB nodes per block.
 template <int K, int NPB>
 void launch_v4_npb(int pass, int64_t nb, const StepGeom& G, const StepBuffers& S,
                    const PassCfg& c, hipStream_t st) {
@@ -2354,7 +2346,9 @@ void launch_pass(int pass, int64_t nb, const StepGeom& G, const StepBuffers& S,
     const bool v4 = Q == 27 && c.unions;
     if (v4 && (pass == kP2 || pass == kP4 || (pass >= kS1 && pass <= kS4))) {
         if (c.ktmpl == 48) launch_v4<48>(pass, nb, G, S, c, st);
+        else if (c.ktmpl == 40) launch_v4<40>(pass, nb, G, S, c, st);
         else if (c.ktmpl == 32) launch_v4<32>(pass, nb, G, S, c, st);
+        else if (c.ktmpl == 24) launch_v4<24>(pass, nb, G, S, c, st);
         else launch_v4<16>(pass, nb, G, S, c, st);
         check_launch("step pass");
         return;
@@ -2386,7 +2380,8 @@ void launch_pass(int pass, int64_t nb, const StepGeom& G, const StepBuffers& S,
     switch (pass) {
         case kP1:
             if (p1_fuses_pml(Q, c.unions)) {
-                k_p1_pml<<<nb, kP1Fused, 0, st>>>(G, S, cp, c.B);
+                if (c.pml64) k_p1_pml<double><<<nb, kP1Fused, 0, st>>>(G, S, cp, c.B);
+                else k_p1_pml<float><<<nb, kP1Fused, 0, st>>>(G, S, cp, c.B);
             } else if (p1_uses_dma(Q, c.unions)) {
                 k_p1_dma<<<nb, kP1Chunk, 0, st>>>(G, S, cp, c.B);
             } else {
@@ -2434,7 +2429,7 @@ void launch_pass(int pass, int64_t nb, const StepGeom& G, const StepBuffers& S,
     check_launch("step pass");
 }
 
-int ktemplate(int k) { return (k == 48 || k == 32 || k == 16) ? k : 0; }
+int ktemplate(int k) { return step_k_template(k); }
 
 }  // namespace
 
@@ -2499,7 +2494,7 @@ void launch_rk4_stage(int stage, const StepGeom& G, const StepBuffers& S, hipStr
     int64_t nb[kStepKernels];
     step_block_counts(Q, G, S, nb, pair ? 1 : 0);
     const PassCfg c{ktemplate(G.k), step_uses_unions(Q, G.k, G.N), S.ucap, S.ucap_f, BatchArgs{}, 0,
-                    S.ulist != nullptr, G.k, S.tile_ng != nullptr, pair};
+                    S.ulist != nullptr, G.k, S.tile_ng != nullptr, pair, G.pml64 != 0};
     launch_pass<Q>(kS1 + stage - 1, nb[kS1 + stage - 1], G, S, CollisionParams{}, c, st);
 }
 
@@ -2509,7 +2504,7 @@ void launch_step(const StepGeom& G, const StepBuffers& S, const CollisionParams&
     int64_t nb[kStepKernels];
     step_block_counts(Q, G, S, nb);
     const PassCfg c{ktemplate(G.k), step_uses_unions(Q, G.k, G.N), S.ucap, S.ucap_f, BatchArgs{}, 0,
-                    S.ulist != nullptr, G.k, S.tile_ng != nullptr, q9_pair(Q, G.N)};
+                    S.ulist != nullptr, G.k, S.tile_ng != nullptr, q9_pair(Q, G.N), G.pml64 != 0};
     for (int p = 0; p < kStepKernels; ++p) {
         if (ev) hip_check(hipEventRecord(ev[p], st), "event");
         launch_pass<Q>(p, nb[p], G, S, cp, c, st);
@@ -2525,7 +2520,7 @@ void launch_step_batch(const BatchPlan& plan, hipStream_t st) {
         const PassCfg c{plan.k_template, plan.unions, plan.ucap, plan.ucap_f,
                         BatchArgs{plan.dev_scenes, plan.dev_bstart + p * (plan.nscenes + 1),
                                   plan.nscenes},
-                        plan.gather_batch, plan.tiles, plan.kmax, plan.ragged, plan.pair};
+                        plan.gather_batch, plan.tiles, plan.kmax, plan.ragged, plan.pair, plan.pml64};
         launch_pass<Q>(p, plan.blocks[p], G, S, CollisionParams{}, c, st);
     }
 }

@@ -51,8 +51,11 @@ struct StepGeom {
     int64_t nbulk;    // [0, nbulk) bulk
     int64_t nlayer;   // [nbulk, nfluid) absorbing layer
     int64_t nfluid;   // nbulk + nlayer; [nfluid, N) boundary
-    int k;            // divergence stencil width
+    int k;            // divergence stencil width of the records (step_width)
     int kb;           // boundary interpolation stencil width
+    int pml64;        // fused D3Q27 collision: PML local terms in FP64 (stencil widths other
+                      // than 16, 32 and 48; in FP32 the pass is 2 to 3 us shorter at
+                      // 10k to 130k nodes, which these three widths rely on)
     int pml_ref;      // layer field reads Q at (j - nbulk) as the reference
     float dt;         // lattice time step
     float rho0;       // nominal density
@@ -195,6 +198,7 @@ struct BatchPlan {
     bool tiles = false;                 // tile unions built for every scene
     int kmax = 0;                       // largest stencil width over the scenes
     bool ragged = false;                // per-tile record widths in every scene
+    bool pml64 = false;                 // StepGeom::pml64 of every scene
     bool pair = false;                  // D2Q9: two lanes per node (else one per distribution)
 };
 // Block counts of each pass for one scene (the same counts launch_step
@@ -207,8 +211,16 @@ void launch_step_batch(const BatchPlan& plan, hipStream_t stream);
 
 // Whether the step runs the D3Q27 four-per-lane kernels, which may use
 // the tile unions (StepBuffers::ulist/uoff/ucap) and slabs holding union
-// positions: D3Q27, k in {16, 32, 48}, fewer than 2^25 nodes.
+// positions: D3Q27, 12 <= k <= 48, fewer than 2^25 nodes.
 bool step_uses_unions(int Q, int k, int64_t N);
+// Stencil width of the step's records: k, or for the four-per-lane kernels
+// the next multiple of 8 (at least 16), the added records pointing at the node
+// itself with zero weights.  A padded record costs less than the
+// one-distribution-per-lane kernels do on all of them (h = 0.02 cube, k = 24:
+// 254 us per step against 205 at k = 32); below k = 12 the padding would be a
+// third of the records.
+int step_width(int Q, int k, int64_t N);
+constexpr int step_k_template(int k) { return k >= 16 && k <= 48 && k % 8 == 0 ? k : 0; }
 // Whether the D2Q9 stencil passes run two lanes per node by default
 // (NAGA_Q9_THREE=0: one lane per distribution), and whether they can (fewer
 // than 2^26 nodes: 32-bit buffer offsets of 32-byte rows).
