@@ -1261,8 +1261,10 @@ void Engine::get_distributions(double* f, double* g) {
     NAGA_HIP(hipStreamSynchronize(stream_));
     for (int a = 0; a < Q; ++a) {
         const double w = weight(Q, a);
+        const float* col = rows.data() + row_of(0, a);
+        const size_t pitch = row_of(1, a) - row_of(0, a);
         for (int64_t i = 0; i < N_; ++i) {
-            const double v = double(rows[row_of(i, a)]);
+            const double v = double(col[size_t(i) * pitch]);
             if (g) g[a * N_ + i] = v;
             if (f) f[a * N_ + i] = w + v;
         }
@@ -1275,7 +1277,9 @@ void Engine::set_distributions(const double* f) {
     std::vector<float> rows(size_t(N_) * RS_, 0.0f);
     for (int a = 0; a < Q; ++a) {
         const double w = weight(Q, a);
-        for (int64_t i = 0; i < N_; ++i) rows[row_of(i, a)] = float(f[a * N_ + i] - w);
+        float* col = rows.data() + row_of(0, a);
+        const size_t pitch = row_of(1, a) - row_of(0, a);
+        for (int64_t i = 0; i < N_; ++i) col[size_t(i) * pitch] = float(f[a * N_ + i] - w);
     }
     g_.upload(rows.data(), rows.size(), stream_);
     refresh_macroscopic_state();
@@ -1285,21 +1289,10 @@ void Engine::set_distributions(const double* f) {
 void Engine::set_pulse(const double* center, double amp, double width) {
     require_domain();
     require(width > 0, "pulse width must be positive");
-    const int Q = cfg_.Q, D = D_;
-    std::vector<float> hp(size_t(N_) * D);
-    pts_.download(hp.data(), hp.size(), stream_);
-    NAGA_HIP(hipStreamSynchronize(stream_));
-    std::vector<float> rows(size_t(N_) * RS_, 0.0f);
-    for (int64_t i = 0; i < N_; ++i) {
-        double r2 = 0.0;
-        for (int d = 0; d < D; ++d) {
-            const double t = double(hp[i * D + d]) - center[d];
-            r2 += t * t;
-        }
-        const double p = amp * std::exp(-r2 / (2.0 * width * width));
-        for (int a = 0; a < Q; ++a) rows[row_of(i, a)] = float(weight(Q, a) * p);
-    }
-    g_.upload(rows.data(), rows.size(), stream_);
+    if (cfg_.Q == 27)
+        launch_pulse<27>(N_, pts_.get(), center, amp, width, g_.get(), stream_);
+    else
+        launch_pulse<9>(N_, pts_.get(), center, amp, width, g_.get(), stream_);
     refresh_macroscopic_state();
     NAGA_HIP(hipStreamSynchronize(stream_));
     time_ = 0.0;

@@ -255,6 +255,12 @@ void launch_probe(int Q, int64_t n, int k, const uint32_t* idx, const float* w,
                   const float* held, const float* g, int64_t N, double rho0, double* out,
                   hipStream_t stream);
 
+// A Gaussian density pulse at rest as deviation rows: g_alpha = w_alpha amp
+// exp(-|x - center|^2 / (2 width^2)) in FP64, rounded once; pts [N][D].
+template <int Q>
+void launch_pulse(int64_t N, const float* pts, const double* center, double amp, double width,
+                  float* g, hipStream_t stream);
+
 // Fresh macroscopic values from the current state: rho (FP32, reference
 // units), drho = rho - rho0 in FP64 without cancellation, u (FP32).
 template <int Q>
