@@ -1,4 +1,4 @@
-// Owning device allocation (hipMalloc/hipFree) with typed access.
+// Owning device allocation with typed access.
 #pragma once
 
 #include <utility>
@@ -7,6 +7,13 @@
 #include "naga_common.hpp"
 
 namespace naga_amd {
+
+// Device memory of at least `bytes` (> 0) on the current device, from blocks
+// released before or from hipMalloc; contents undefined.  Any thread.
+void* device_allocate(size_t bytes);
+// Gives a block back.  Work on any stream may still use it: it is handed out
+// again only after the device has been synchronised.
+void device_release(void* p) noexcept;
 
 template <class T>
 class DeviceBuffer {
@@ -26,13 +33,11 @@ class DeviceBuffer {
     void allocate(size_t n) {
         release();
         if (n == 0) return;
-        void* p = nullptr;
-        NAGA_HIP(hipMalloc(&p, n * sizeof(T)));
-        ptr_ = static_cast<T*>(p);
+        ptr_ = static_cast<T*>(device_allocate(n * sizeof(T)));
         n_ = n;
     }
     void release() {
-        if (ptr_) (void)hipFree(ptr_);
+        if (ptr_) device_release(ptr_);
         ptr_ = nullptr;
         n_ = 0;
     }

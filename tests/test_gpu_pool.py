@@ -1,0 +1,50 @@
+"""Device blocks kept between allocations: scenes rebuilt in memory that other
+scenes used, one after another and from several threads at once, give the
+results of their first build bit for bit."""
+import threading
+
+import numpy as np
+import pytest
+
+import naga_amd
+from tests.scenes import gpu_engine, grid_nodes
+
+pytestmark = pytest.mark.gpu
+
+SCENES = [(27, 0.1, 32), (9, 0.04, 16), (27, 0.125, 20), (9, 0.03, 13), (27, 0.11, 32)]
+
+
+def _solve(nodes, Q, k, h):
+    eng = gpu_engine(nodes, Q, k, h, kb=16)
+    eng.set_initial_pulse([0.4] * (2 if Q == 9 else 3), 1e-3, 0.15)
+    eng.step_forward(12)
+    out = eng.macroscopic(fresh=True)
+    eng.close()
+    return out
+
+
+def _same(a, b):
+    return all(np.array_equal(a[f], b[f]) for f in ("rho", "drho", "u"))
+
+
+def test_rebuilt_scenes_and_threads(oracle64):
+    nodes = [grid_nodes(oracle64, 2 if Q == 9 else 3, h, 2 * h) for Q, h, _ in SCENES]
+    first = [_solve(n, Q, k, h) for n, (Q, h, k) in zip(nodes, SCENES)]
+    for _ in range(2):  # now in blocks of the scenes before
+        for n, (Q, h, k), want in reversed(list(zip(nodes, SCENES, first))):
+            assert _same(_solve(n, Q, k, h), want)
+    bad = []
+
+    def work(t):
+        for r in range(4):
+            i = (t + r) % len(SCENES)
+            Q, h, k = SCENES[i]
+            if not _same(_solve(nodes[i], Q, k, h), first[i]):
+                bad.append((t, r, i))
+
+    threads = [threading.Thread(target=work, args=(t,)) for t in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
