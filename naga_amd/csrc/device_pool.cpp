@@ -7,8 +7,10 @@
 // Released blocks of up to kPoolBytes in all are kept for later allocations
 // of about their size; the rest is freed at once, and all of it when the
 // device runs out of memory.  A block is handed out again only after the
-// device has been synchronised since its release (one hipDeviceSynchronize
-// covers every block released before it), which is what hipFree waited for.
+// device has been synchronised since its release (one wait covers every block
+// released before it), which is what freeing it waited for.  The wait is the
+// one that hipFree performs, on a small block of its own: hipDeviceSynchronize
+// would invalidate a stream capture in progress on another thread.
 #include <mutex>
 #include <unordered_map>
 #include <vector>
@@ -81,7 +83,9 @@ void* device_allocate(size_t bytes) {
         if (P.find(bytes, device, false) >= 0) {
             const uint64_t upto = P.releases;
             lk.unlock();  // other threads go on while this one waits
-            const bool ok = hipDeviceSynchronize() == hipSuccess;
+            void* token = nullptr;
+            const bool ok =
+                hipMalloc(&token, 256) == hipSuccess && hipFree(token) == hipSuccess;
             if (!ok) (void)hipGetLastError();
             lk.lock();
             if (ok && P.synced[device] < upto) P.synced[device] = upto;

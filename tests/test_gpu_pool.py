@@ -39,8 +39,11 @@ def test_rebuilt_scenes_and_threads(oracle64):
         for r in range(4):
             i = (t + r) % len(SCENES)
             Q, h, k = SCENES[i]
-            if not _same(_solve(nodes[i], Q, k, h), first[i]):
-                bad.append((t, r, i))
+            try:
+                if not _same(_solve(nodes[i], Q, k, h), first[i]):
+                    bad.append((t, r, i))
+            except Exception as e:  # a thread's error is the test's
+                bad.append((t, r, i, str(e)))
 
     threads = [threading.Thread(target=work, args=(t,)) for t in range(4)]
     for t in threads:
