@@ -1139,6 +1139,7 @@ void Batch::rebuild() {
             P.ucap = std::max(P.ucap, descs[s].S.ucap);
             P.ucap_f = std::max(P.ucap_f, descs[s].S.ucap_f);
             P.kmax = std::max(P.kmax, e->stencil_k());
+            P.kb = std::max(P.kb, descs[s].G.kb);
             any_sources_ = any_sources_ || descs[s].S.src != nullptr;
             int64_t nb[kStepKernels];
             step_block_counts(g.Q, descs[s].G, descs[s].S, nb, g.pair ? 1 : 0);

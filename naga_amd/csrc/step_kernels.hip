@@ -2020,23 +2020,23 @@ __global__ __launch_bounds__(kBlock) void k_binterp_v4(StepGeom G, StepBuffers S
 }
 
 // Boundary interpolation for D3Q27 with the sources of each 32-node tile
-// staged in LDS (the field rows, and for the first pass the collision
-// increments too) by LDS DMA: about 6 rows per node instead of 32 (64)
-// gathers.  Same records, products and order as k_binterp_v4.
+// staged in LDS: about 6 rows per node instead of 32 (64) gathers.  The last
+// pass copies the field rows by LDS DMA; the first subtracts the sources'
+// collision increments on the way, so both hold one row per source.  LDS per
+// block is the tile's sources (bunion_cap) and records: with both rows staged
+// and room for 63 records per node it was 82 KB, one block per CU.  Same
+// records, products and order as k_binterp_v4.
 static_assert(kBTileNodes == kV4Nodes, "one boundary tile per block");
-// LDS of k_binterp_u: the tile's records (kb <= 63: 32 x 63 {position, w})
-// after the field rows and, for the first pass, the increments.
-constexpr int kBRecUnits = (kBTileNodes * 63 * 8 + 15) / 16;
-template <bool ACCUMULATE>
-constexpr size_t binterp_lds() {
-    return size_t((ACCUMULATE ? 2 : 1) * kBUnionCap * kV4Lanes + kBRecUnits) * 16u;
+constexpr size_t binterp_lds(int kb) {
+    return (size_t(bunion_cap(kb)) * kV4Lanes + (size_t(kBTileNodes) * kb * 8 + 15) / 16) * 16u;
 }
 
 template <bool ACCUMULATE>
 __global__ __launch_bounds__(kBlock) void k_binterp_u(StepGeom G, StepBuffers S, BatchArgs B) {
-    extern __shared__ float4 urows[];  // field rows, (ACCUMULATE) increments, records
-    float4* recs = urows + (ACCUMULATE ? 2 : 1) * kBUnionCap * kV4Lanes;
+    extern __shared__ float4 urows[];  // source rows, then records
     const BlockCtx bc = locate(B, G, S);
+    const int cap = bunion_cap(G.kb);
+    float4* recs = urows + cap * kV4Lanes;
     const int slot = threadIdx.x / kV4Lanes, q = threadIdx.x % kV4Lanes;
     const int64_t nbnd = G.N - G.nfluid;
     const int64_t tile = xcd_tile(bc.b, bc.nb);
@@ -2048,20 +2048,36 @@ __global__ __launch_bounds__(kBlock) void k_binterp_u(StepGeom G, StepBuffers S,
     int U;
     union_range(S.buoff, tile, u0, U);
     const uint32_t* ul = S.bulist + u0;
-    const bool lds = U <= kBUnionCap;
+    const bool lds = U <= cap;
     const UnionIdx<kBlock> ux = union_indices<kBlock>(ul, lds ? U : 0);
     __builtin_amdgcn_sched_barrier(0);
     // the tile's records: cnt * kb pairs from the tile's start (the last
     // tile's piece past the slab reads as zero)
     const int64_t left = nbnd - m0;
     const int cnt = left < kV4Nodes ? int(left) : kV4Nodes;
-    dma_contiguous<kBRecUnits, kBlock>(
+    dma_contiguous<(kBTileNodes * 63 * 8 + 15) / 16, kBlock>(
         rsrc(S.bslab + m0 * G.kb * 2, uint64_t(nbnd - m0) * G.kb * 8u), recs,
         (cnt * G.kb * 8 + 15) / 16);
     __builtin_amdgcn_sched_barrier(0);
-    if (lds) {
-        union_copy<kBlock>(urows, ux, U, f);
-        if (ACCUMULATE) union_copy<kBlock>(urows + kBUnionCap * kV4Lanes, ux, U, cl);
+    if (lds && !ACCUMULATE) union_copy<kBlock>(urows, ux, U, f);
+    if (lds && ACCUMULATE) {
+        constexpr int kChunks = bunion_cap(64) / (8 * (kBlock / 64));  // 8-row chunks per wave
+        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+        float4 v[kChunks], c[kChunks];
+#pragma unroll
+        for (int t = 0; t < kChunks; ++t)
+            if ((wave + t * (kBlock / 64)) * 8 < U) {  // every load first
+                const uint32_t off = ux.j[t] * 128u + uint32_t(lane & 7) * 16u;
+                v[t] = ld4(f, off);
+                c[t] = ld4(cl, off);
+            }
+#pragma unroll
+        for (int t = 0; t < kChunks; ++t) {
+            const int r = (wave + t * (kBlock / 64)) * 8 + (lane >> 3);
+            if (r < U)
+                urows[r * kV4Lanes + (lane & 7)] = make_float4(v[t].x - c[t].x, v[t].y - c[t].y,
+                                                               v[t].z - c[t].z, v[t].w - c[t].w);
+        }
     }
     const uint32_t own = uint32_t(G.nfluid + m) * 128u + uint32_t(q) * 16u;
     // the node's own row (the collision increment it accumulates onto),
@@ -2084,10 +2100,6 @@ __global__ __launch_bounds__(kBlock) void k_binterp_u(StepGeom G, StepBuffers S,
             const uint32_t j = __float_as_uint(rec[u].x);
             if (lds) {
                 v[u] = urows[j * kV4Lanes + q];
-                if (ACCUMULATE) {
-                    const float4 c = urows[(kBUnionCap + j) * kV4Lanes + q];
-                    v[u] = make_float4(v[u].x - c.x, v[u].y - c.y, v[u].z - c.z, v[u].w - c.w);
-                }
             } else {  // sources over the cap: rows read from HBM through the list
                 const uint32_t off = ul[j] * 128u + lane_off;
                 v[u] = ld4(f, off);
@@ -2298,6 +2310,7 @@ struct PassCfg {
     bool ragged;   // per-tile record widths (StepBuffers::tile_ng)
     bool pair;     // D2Q9 stencil passes with two lanes per node
     bool pml64;    // StepGeom::pml64
+    int kb;        // largest boundary stencil width (LDS of the boundary tiles)
 };
 
 template <int Q, int STAGE, int KT>
@@ -2442,7 +2455,7 @@ void launch_pass(int pass, int64_t nb, const StepGeom& G, const StepBuffers& S,
             break;
         case kP3:
             if (v4 && c.tiles)
-                k_binterp_u<true><<<nb, kBlock, binterp_lds<true>(), st>>>(G, S, c.B);
+                k_binterp_u<true><<<nb, kBlock, binterp_lds(c.kb), st>>>(G, S, c.B);
             else if (v4) k_binterp_v4<true><<<nb, kBlock, 0, st>>>(G, S, c.B);
             else k_binterp<Q, true><<<nb, kBlock, 0, st>>>(G, S, c.B);
             break;
@@ -2457,7 +2470,7 @@ void launch_pass(int pass, int64_t nb, const StepGeom& G, const StepBuffers& S,
         case kS4: launch_stage_pass<Q, 4>(nb, G, S, c, st); break;
         default:
             if (Q == 27 && c.unions && c.tiles)
-                k_binterp_u<false><<<nb, kBlock, binterp_lds<false>(), st>>>(G, S, c.B);
+                k_binterp_u<false><<<nb, kBlock, binterp_lds(c.kb), st>>>(G, S, c.B);
             else if (Q == 27 && c.unions) k_binterp_v4<false><<<nb, kBlock, 0, st>>>(G, S, c.B);
             else k_binterp<Q, false><<<nb, kBlock, 0, st>>>(G, S, c.B);
             break;
@@ -2530,7 +2543,7 @@ void launch_rk4_stage(int stage, const StepGeom& G, const StepBuffers& S, hipStr
     int64_t nb[kStepKernels];
     step_block_counts(Q, G, S, nb, pair ? 1 : 0);
     const PassCfg c{ktemplate(G.k), step_uses_unions(Q, G.k, G.N), S.ucap, S.ucap_f, BatchArgs{}, 0,
-                    S.ulist != nullptr, G.k, S.tile_ng != nullptr, pair, G.pml64 != 0};
+                    S.ulist != nullptr, G.k, S.tile_ng != nullptr, pair, G.pml64 != 0, G.kb};
     launch_pass<Q>(kS1 + stage - 1, nb[kS1 + stage - 1], G, S, CollisionParams{}, c, st);
 }
 
@@ -2540,7 +2553,7 @@ void launch_step(const StepGeom& G, const StepBuffers& S, const CollisionParams&
     int64_t nb[kStepKernels];
     step_block_counts(Q, G, S, nb);
     const PassCfg c{ktemplate(G.k), step_uses_unions(Q, G.k, G.N), S.ucap, S.ucap_f, BatchArgs{}, 0,
-                    S.ulist != nullptr, G.k, S.tile_ng != nullptr, q9_pair(Q, G.N), G.pml64 != 0};
+                    S.ulist != nullptr, G.k, S.tile_ng != nullptr, q9_pair(Q, G.N), G.pml64 != 0, G.kb};
     for (int p = 0; p < kStepKernels; ++p) {
         if (ev) hip_check(hipEventRecord(ev[p], st), "event");
         launch_pass<Q>(p, nb[p], G, S, cp, c, st);
@@ -2556,7 +2569,8 @@ void launch_step_batch(const BatchPlan& plan, hipStream_t st) {
         const PassCfg c{plan.k_template, plan.unions, plan.ucap, plan.ucap_f,
                         BatchArgs{plan.dev_scenes, plan.dev_bstart + p * (plan.nscenes + 1),
                                   plan.nscenes},
-                        plan.gather_batch, plan.tiles, plan.kmax, plan.ragged, plan.pair, plan.pml64};
+                        plan.gather_batch, plan.tiles, plan.kmax, plan.ragged, plan.pair, plan.pml64,
+                        plan.kb};
         launch_pass<Q>(p, plan.blocks[p], G, S, CollisionParams{}, c, st);
     }
 }

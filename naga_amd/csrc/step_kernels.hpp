@@ -137,7 +137,7 @@ struct StepBuffers {
     // Boundary interpolation tiles (32 boundary nodes): the distinct source
     // nodes of each tile, bulist[buoff[t] .. buoff[t+1]), and bslab index
     // fields holding positions in that list (null: no boundary unions).
-    // Tiles of at most kBUnionCap sources are staged in LDS.
+    // Tiles of at most bunion_cap(kb) sources are staged in LDS.
     const uint32_t* bulist;
     const int64_t* buoff;
 };
@@ -197,6 +197,7 @@ struct BatchPlan {
     int gather_batch = 0;               // neighbours gathered per unrolled step (0: default)
     bool tiles = false;                 // tile unions built for every scene
     int kmax = 0;                       // largest stencil width over the scenes
+    int kb = 0;                         // largest boundary stencil width
     bool ragged = false;                // per-tile record widths in every scene
     bool pml64 = false;                 // StepGeom::pml64 of every scene
     bool pair = false;                  // D2Q9: two lanes per node (else one per distribution)
@@ -239,7 +240,10 @@ int union_cap_default(int k);
 // Stride of the two rows of layer means (D3Q27: 32, so each row's
 // quarters load as 16-byte vectors; padding entries stay zero).
 constexpr int means_stride(int Q) { return Q == 27 ? 32 : Q; }
-constexpr int kBUnionCap = 256;   // LDS rows per boundary-interpolation tile
+// LDS rows per boundary-interpolation tile: 32-node tiles of a cube's faces
+// have 183 sources on average, at most 253, with kb = 32, and about 255 with
+// kb = 48 (half of them over 256).
+NAGA_HD constexpr int bunion_cap(int kb) { return kb <= 32 ? 256 : 320; }
 constexpr int kBTileNodes = 32;   // boundary nodes per boundary-interpolation tile
 constexpr int kUnionRowsMax = 512;  // LDS union rows per block, upper bound
 
