@@ -1878,22 +1878,55 @@ __global__ __launch_bounds__(NPB * kV4Lanes) void k_p2_t(StepGeom G, StepBuffers
     st4(S.A, own, make_float4(s.x - r.x, s.y - r.y, s.z - r.z, s.w - r.w));
 }
 
+// Few enough partial layer sums for each field block to read them all (54
+// columns) in about the time of k_means' launch: 128 parts are 64-node blocks
+// of at most 8,192 layer nodes (the 9,261-node cube has about 100).
+__host__ __device__ __forceinline__ bool means_in_field(const StepBuffers& S) {
+    return S.nparts - S.part_lo <= 128;
+}
+
 // PML auxiliary field rows for D3Q27, four distributions per lane (the
 // arithmetic of k_pml_field; padding slots stay zero).
+// Where the layer's partial sums are few (means_in_field) each block forms the
+// means from them, else they are read from k_means.
 __global__ __launch_bounds__(kBlock) void k_pml_field_v4(StepGeom G, StepBuffers S, BatchArgs B) {
+    __shared__ double part[4][64];
+    __shared__ float4 means[2][kV4Lanes];
     const BlockCtx bc = locate(B, G, S);
     const int slot = threadIdx.x / kV4Lanes, q = threadIdx.x % kV4Lanes;
     const int64_t m = xcd_tile(bc.b, bc.nb) * kV4Nodes + slot;
-    if (m >= G.nlayer) return;
+    const bool in = m < G.nlayer;
     const int64_t j = G.nbulk + m;
     const int64_t p = G.pml_ref ? j - G.nbulk : j;
     const uint64_t rows = uint64_t(G.N) * 128u;
     const uint32_t lane_off = uint32_t(q) * 16u;
-    const float sig = S.sigma[m];
-    const float4 q1 = ld4(rsrc(S.Qp, rows), uint32_t(p) * 128u + lane_off);
+    const float sig = in ? S.sigma[m] : 0.0f;
+    const float4 q1 = ld4(rsrc(S.Qp, rows), uint32_t(p) * 128u + lane_off);  // past N: zero
     const float4 q2 = ld4(rsrc(S.Q2v, rows), uint32_t(p) * 128u + lane_off);
-    const float4 m1 = reinterpret_cast<const float4*>(S.means)[q];
-    const float4 m2 = reinterpret_cast<const float4*>(S.means + means_stride(27))[q];
+    float4 m1, m2;
+    if (means_in_field(S)) {
+        // thread t: column t % 64 (27 of Q1 from 0, 27 of Q2 from 32), every
+        // fourth part
+        const int c = threadIdx.x & 63, r = threadIdx.x >> 6, a = c & 31;
+        double s = 0.0;
+        if (a < 27) {
+            const double* col = S.partial + int64_t((c >> 5) * 27 + a) * S.nparts;
+#pragma unroll 8
+            for (int t = S.part_lo + r; t < S.nparts; t += 4) s += col[t];
+        }
+        part[r][c] = s;
+        __syncthreads();
+        if (threadIdx.x < 64)
+            reinterpret_cast<float*>(means)[threadIdx.x] =
+                float(((part[0][c] + part[1][c]) + (part[2][c] + part[3][c])) / double(G.nlayer));
+        __syncthreads();
+        m1 = means[0][q];
+        m2 = means[1][q];
+    } else {
+        m1 = reinterpret_cast<const float4*>(S.means)[q];
+        m2 = reinterpret_cast<const float4*>(S.means + means_stride(27))[q];
+    }
+    if (!in) return;
     float4 out;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -2511,7 +2544,7 @@ void step_block_counts(int Q, const StepGeom& G, const StepBuffers& S, int64_t* 
                                          : (G.N + kP1Block - 1) / kP1Block;
     nb[kPl] = (pml && !fused) ? S.nparts : 0;
     // (D2Q9: the means are formed in the field pass)
-    nb[kPm] = pml && Q == 27 ? 2 * Q : 0;
+    nb[kPm] = pml && Q == 27 && !(un && means_in_field(S)) ? 2 * Q : 0;
     nb[kPf] = !pml ? 0
               : Q == 9 ? (G.nlayer + kBlock / 2 - 1) / (kBlock / 2)
                        : un ? tiles32(G.nlayer) : lanes(G.nlayer);
