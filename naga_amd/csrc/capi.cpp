@@ -1135,20 +1135,29 @@ int naga_rk4_stage(int32_t q, int64_t n, int64_t n_fluid, int32_t k, const uint3
             }
             DeviceBuffer<uint32_t> didx(std::max<int64_t>(n_fluid * k, 1));
             DeviceBuffer<float> dW(std::max<int64_t>(n_fluid * k * D, 1));
+            const int ks = step_width(q, k, n);  // of the records
             DeviceBuffer<float> slab(std::max<int64_t>(
-                n_fluid * (q == 9 ? 4 * q9_units(k, 2) : k * (1 + D)), 1));
+                n_fluid * (q == 9 ? 4 * q9_units(k, 2) : ks * (1 + D)), 1));
             if (n_fluid) {
                 didx.upload(idx, size_t(n_fluid) * k, s);
                 dW.upload(W, size_t(n_fluid) * k * D, s);
+                if (ks != k) {
+                    DeviceBuffer<uint32_t> pi(n_fluid * ks);
+                    DeviceBuffer<float> pW(n_fluid * ks * D);
+                    launch_pad_entries(n_fluid, k, ks, D, didx.get(), dW.get(), pi.get(), pW.get(),
+                                       s);
+                    didx = std::move(pi);
+                    dW = std::move(pW);
+                }
                 if (q == 9) launch_make_slab_q9(n_fluid, k, D, didx.get(), dW.get(), slab.get(), s);
-                else launch_make_slab(n_fluid, k, D, didx.get(), dW.get(), slab.get(), s);
+                else launch_make_slab(n_fluid, ks, D, didx.get(), dW.get(), slab.get(), s);
             }
             StepGeom G{};
             G.N = n;
             G.nbulk = n_fluid;
             G.nlayer = 0;
             G.nfluid = n_fluid;
-            G.k = k;
+            G.k = ks;
             G.kb = 1;
             G.dt = float(dt);
             G.rho0 = 1.0f;

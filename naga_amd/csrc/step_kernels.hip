@@ -2281,12 +2281,11 @@ bool step_uses_unions(int Q, int k, int64_t N) {
         const char* e = std::getenv("NAGA_V4");
         return !(e && e[0] == '0');
     }();
-    return Q == 27 && on && k >= 12 && k <= 48 && N < (int64_t(1) << 25);
+    return Q == 27 && on && k >= kUnionKMin && k <= kUnionKMax && N < (int64_t(1) << 25);
 }
 
 int step_width(int Q, int k, int64_t N) {
-    if (!step_uses_unions(Q, k, N)) return k;
-    return k <= 16 ? 16 : (k + 7) / 8 * 8;
+    return step_uses_unions(Q, k, N) ? union_width(k) : k;
 }
 
 // D2Q9 scenes run the stencil kernels with two lanes per node (16-byte
@@ -2432,11 +2431,14 @@ void launch_pass(int pass, int64_t nb, const StepGeom& G, const StepBuffers& S,
     if (nb <= 0) return;
     const bool v4 = Q == 27 && c.unions;
     if (v4 && (pass == kP2 || pass == kP4 || (pass >= kS1 && pass <= kS4))) {
-        if (c.ktmpl == 48) launch_v4<48>(pass, nb, G, S, c, st);
-        else if (c.ktmpl == 40) launch_v4<40>(pass, nb, G, S, c, st);
-        else if (c.ktmpl == 32) launch_v4<32>(pass, nb, G, S, c, st);
-        else if (c.ktmpl == 24) launch_v4<24>(pass, nb, G, S, c, st);
-        else launch_v4<16>(pass, nb, G, S, c, st);
+        switch (c.ktmpl) {
+            case 48: launch_v4<48>(pass, nb, G, S, c, st); break;
+            case 40: launch_v4<40>(pass, nb, G, S, c, st); break;
+            case 32: launch_v4<32>(pass, nb, G, S, c, st); break;
+            case 24: launch_v4<24>(pass, nb, G, S, c, st); break;
+            case 16: launch_v4<16>(pass, nb, G, S, c, st); break;
+            default: fail(kInvalidArgument, "records are not padded to a kernel's stencil width");
+        }
         check_launch("step pass");
         return;
     }

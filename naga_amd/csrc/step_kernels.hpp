@@ -213,15 +213,25 @@ void launch_step_batch(const BatchPlan& plan, hipStream_t stream);
 // Whether the step runs the D3Q27 four-per-lane kernels, which may use
 // the tile unions (StepBuffers::ulist/uoff/ucap) and slabs holding union
 // positions: D3Q27, 12 <= k <= 48, fewer than 2^25 nodes.
+constexpr int kUnionKMin = 12, kUnionKMax = 48;
 bool step_uses_unions(int Q, int k, int64_t N);
-// Stencil width of the step's records: k, or for the four-per-lane kernels
+// Stencil width of the step's records, which every caller that builds them
+// gives them and puts in StepGeom::k: k, or for the four-per-lane kernels
 // the next multiple of 8 (at least 16), the added records pointing at the node
 // itself with zero weights.  A padded record costs less than the
 // one-distribution-per-lane kernels do on all of them (h = 0.02 cube, k = 24:
 // 254 us per step against 205 at k = 32); below k = 12 the padding would be a
 // third of the records.
 int step_width(int Q, int k, int64_t N);
+constexpr int union_width(int k) { return k <= 16 ? 16 : (k + 7) / 8 * 8; }
+// The width that the kernels are instantiated for, or 0.
 constexpr int step_k_template(int k) { return k >= 16 && k <= 48 && k % 8 == 0 ? k : 0; }
+constexpr bool union_widths_instantiated() {
+    for (int k = kUnionKMin; k <= kUnionKMax; ++k)
+        if (union_width(k) < k || step_k_template(union_width(k)) != union_width(k)) return false;
+    return true;
+}
+static_assert(union_widths_instantiated(), "a stencil width pads to one without kernels");
 // Whether the D2Q9 stencil passes run two lanes per node by default
 // (NAGA_Q9_THREE=0: one lane per distribution), and whether they can (fewer
 // than 2^26 nodes: 32-bit buffer offsets of 32-byte rows).

@@ -1,6 +1,7 @@
 """D3Q27 stencil widths between the kernels' own (padded to the next multiple
-of 8): whole steps against the FP64 oracle with and without tile unions, per
-node widths, and a batch that mixes widths sharing a padded one."""
+of 8): whole steps against the FP64 oracle with and without tile unions, single
+RK4 stages against FP64 numpy, and a batch that mixes widths sharing a padded
+one."""
 import numpy as np
 import pytest
 
@@ -41,3 +42,32 @@ def test_batch_of_widths_sharing_a_padded_one(oracle64):
     for a, b in zip(alone, scenes):
         assert np.array_equal(a.macroscopic()["drho"], b.macroscopic()["drho"])
     batch.close()
+
+
+@pytest.mark.parametrize("n,n_fluid,k", [(1, 1, 12), (33, 31, 11), (65, 64, 12), (97, 95, 13),
+                                         (301, 257, 15), (129, 127, 17), (333, 300, 20),
+                                         (95, 95, 31), (257, 201, 33), (63, 61, 41),
+                                         (131, 130, 47), (99, 77, 49)])
+@pytest.mark.parametrize("stage", [1, 2, 3, 4])
+def test_single_stages_of_any_width(n, n_fluid, k, stage):
+    rng = np.random.default_rng(n + k + stage)
+    c, _, _, _ = naga_amd.lattice_tables(27)
+    idx = rng.integers(0, n, (n_fluid, k)).astype(np.uint32)
+    W = rng.standard_normal((n_fluid, k, 3)).astype(np.float32)
+    y, f, y1, y2 = (rng.standard_normal((n, 27)).astype(np.float32) for _ in range(4))
+    dt = 0.01
+    got = naga_amd.rk4_stage(stage, y, idx, W, dt, n_fluid=n_fluid, stage_input=f, y1=y1, y2=y2)
+    g = (y if stage == 1 else f).astype(np.float64)
+    r = -np.einsum("ikd,ad,ika->ia", W.astype(np.float64), c, g[idx])
+    want = y.astype(np.float64)
+    Y = want[:n_fluid]
+    if stage < 4:
+        want[:n_fluid] = Y + (dt if stage == 3 else dt / 2) * r
+    else:
+        want[:n_fluid] = Y + ((y1[:n_fluid] - Y) + 2 * (y2[:n_fluid] - Y) +
+                              (g[:n_fluid] - Y)) / 3 + dt / 6 * r
+    # FP32 rounding of a sum of k products (three terms each) scaled by dt,
+    # and of the sums of the four rows
+    size = np.einsum("ikd,ad,ika->ia", np.abs(W).astype(np.float64), np.abs(c), np.abs(g)[idx])
+    most = max(np.abs(v).max() for v in (y, f, y1, y2))
+    assert np.abs(got - want).max() < 2.0 ** -24 * ((k + 6) * dt * size.max() + 16 * most)
