@@ -863,7 +863,7 @@ __global__ void k_pad_entries(int64_t n, int k, int ks, int nc, const uint32_t* 
     if (e >= n * ks) return;
     const int64_t i = e / ks;
     const int s = int(e - i * ks);
-    idx_out[e] = s < k ? idx[i * k + s] : uint32_t(i);
+    idx_out[e] = idx[i * k + (s < k ? s : 0)];
     for (int c = 0; c < nc; ++c) w_out[e * nc + c] = s < k ? w[(i * k + s) * nc + c] : 0.0f;
 }
 
@@ -885,8 +885,9 @@ __global__ void k_make_slab_q9(int64_t n, int k, int nc, const uint32_t* idx, co
     const int64_t i = t / words;
     const int u = int(t - i * words) / 4, f = u % (1 + nc);  // field: index, weights
     const int s = u / (1 + nc) * 4 + int(t % 4);             // record (words is a multiple of 4)
-    uint32_t v = f == 0 ? uint32_t(i) : 0u;
-    if (s < k) v = f == 0 ? idx[i * k + s] : __float_as_uint(w[(i * k + s) * nc + f - 1]);
+    uint32_t v = 0u;
+    if (f == 0) v = idx[i * k + (s < k ? s : 0)];
+    else if (s < k) v = __float_as_uint(w[(i * k + s) * nc + f - 1]);
     slab[t] = v;
 }
 

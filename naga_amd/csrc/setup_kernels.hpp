@@ -147,7 +147,9 @@ void launch_filter_weights(int D, const float* pts, int64_t n,
                            hipStream_t stream, const uint8_t* kvar = nullptr);
 
 // Rows of ks >= k entries from rows of k: entry s < k of node i is copied, the
-// others point at i with zero weights (ncomp weights per entry).
+// others name its first entry again with zero weights (ncomp weights per
+// entry).  Not node i: a zero weight times a row that the stencil does not name
+// would bring that row's infinities and NaN in.
 void launch_pad_entries(int64_t n, int k, int ks, int ncomp, const uint32_t* idx, const float* w,
                         uint32_t* idx_out, float* w_out, hipStream_t stream);
 
@@ -158,7 +160,7 @@ void launch_make_slab(int64_t n, int k, int ncomp, const uint32_t* idx,
 
 // D2Q9 records: per node ceil(k / 4) groups of four records, each group four
 // indices and then the four values of each of the ncomp weights (q9_units
-// 16-byte units per node); entries past k hold the node itself, weights zero.
+// 16-byte units per node); entries past k name the first again, weights zero.
 void launch_make_slab_q9(int64_t n, int k, int ncomp, const uint32_t* idx, const float* w,
                          float* slab, hipStream_t stream);
 

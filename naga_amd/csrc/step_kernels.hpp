@@ -217,8 +217,8 @@ constexpr int kUnionKMin = 12, kUnionKMax = 48;
 bool step_uses_unions(int Q, int k, int64_t N);
 // Stencil width of the step's records, which every caller that builds them
 // gives them and puts in StepGeom::k: k, or for the four-per-lane kernels
-// the next multiple of 8 (at least 16), the added records pointing at the node
-// itself with zero weights.  A padded record costs less than the
+// the next multiple of 8 (at least 16), the added records naming the first
+// one's node again with zero weights.  A padded record costs less than the
 // one-distribution-per-lane kernels do on all of them (h = 0.02 cube, k = 24:
 // 254 us per step against 205 at k = 32); below k = 12 the padding would be a
 // third of the records.

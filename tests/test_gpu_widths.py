@@ -1,7 +1,7 @@
 """D3Q27 stencil widths between the kernels' own (padded to the next multiple
 of 8): whole steps against the FP64 oracle with and without tile unions, single
-RK4 stages against FP64 numpy, and a batch that mixes widths sharing a padded
-one."""
+RK4 stages against FP64 numpy, rows that no stencil names, and a batch that
+mixes widths sharing a padded one."""
 import numpy as np
 import pytest
 
@@ -71,3 +71,19 @@ def test_single_stages_of_any_width(n, n_fluid, k, stage):
     size = np.einsum("ikd,ad,ika->ia", np.abs(W).astype(np.float64), np.abs(c), np.abs(g)[idx])
     most = max(np.abs(v).max() for v in (y, f, y1, y2))
     assert np.abs(got - want).max() < 2.0 ** -24 * ((k + 6) * dt * size.max() + 16 * most)
+
+
+@pytest.mark.parametrize("Q,k", [(9, 5), (9, 16), (27, 11), (27, 13), (27, 32)])
+@pytest.mark.parametrize("stage", [2, 3])
+def test_rows_outside_a_stencil_are_not_read(Q, k, stage):
+    """Infinities in rows that no stencil entry names change nothing, also for
+    those rows' own nodes (padding records must name entries of the stencil)."""
+    rng = np.random.default_rng(k)
+    n, D = 100, 2 if Q == 9 else 3
+    idx = rng.integers(0, 90, (n, k)).astype(np.uint32)
+    W = rng.standard_normal((n, k, D)).astype(np.float32)
+    y = rng.standard_normal((n, Q)).astype(np.float32)
+    f = y.copy()
+    f[95:] = np.inf
+    a, b = (naga_amd.rk4_stage(stage, y, idx, W, 0.01, stage_input=v) for v in (f, y))
+    assert np.array_equal(a, b)
