@@ -2220,7 +2220,7 @@ __global__ __launch_bounds__(kBlock) void k_macro(StepGeom G, const float* g,
 // their padding).  On the host the exponentials and the upload of the rows
 // took 1.8 ms of a 132,651-node solve, the pulse's kernel 0.02.
 struct PulseArgs {
-    double center[3], amp, inv;  // inv = 1 / (2 width^2)
+    double center[3], amp, two_w2;  // 2 width^2 (its reciprocal overflows for the smallest)
 };
 template <int Q>
 __global__ __launch_bounds__(kBlock) void k_pulse(int64_t N, const float* pts, PulseArgs P,
@@ -2234,7 +2234,7 @@ __global__ __launch_bounds__(kBlock) void k_pulse(int64_t N, const float* pts, P
         const double t = double(pts[i * L::D + d]) - P.center[d];
         r2 += t * t;
     }
-    const double p = P.amp * exp(-(r2 * P.inv));
+    const double p = P.amp * exp(-r2 / P.two_w2);
     if constexpr (Q == 9) {
         float v[9];
 #pragma unroll
@@ -2644,7 +2644,7 @@ void launch_pulse(int64_t N, const float* pts, const double* center, double amp,
     PulseArgs P{};
     for (int d = 0; d < Lattice<Q>::D; ++d) P.center[d] = center[d];
     P.amp = amp;
-    P.inv = 1.0 / (2.0 * width * width);
+    P.two_w2 = 2.0 * width * width;
     k_pulse<Q><<<(N + kBlock - 1) / kBlock, kBlock, 0, st>>>(N, pts, P, g);
     check_launch("pulse");
 }
