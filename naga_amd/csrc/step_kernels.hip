@@ -381,10 +381,26 @@ __global__ __launch_bounds__(kBlock) void k_pml_field(StepGeom G, StepBuffers S,
         -2.0f * sig * (q1 - S.means[a]) + sig * sig * (q2 - S.means[means_stride(Q) + a]);
 }
 
-// The same for D2Q9, two lanes per node, with the layer means formed by each
-// block from the partial sums (16 columns; the rest distribution's field is
-// not read): the launch of its own that k_means needs costs more than reading
-// the sums (8 bytes per column and 64 layer nodes) once per 128 rows.
+// Few enough partial layer sums for each field block to read them all in
+// about the time of k_means' launch.  Every block reads every part, so the
+// reads grow with the square of the layer: past the bound k_means forms the
+// means once.  D3Q27 (54 columns): 128 parts are 64-node blocks of at most
+// 8,192 layer nodes (the 9,261-node cube has about 100).  D2Q9 (16 columns):
+// a step with the means in the field takes 45.5 us against 46.5 at 260 parts,
+// 46.5 against 46.3 at 306, 48.2 against 47.4 at 462 and 106 against 82 at
+// 1,550; without a bound a million nodes with 358,000 in the layer took 612 us
+// against 333.
+constexpr int kFieldParts27 = 128, kFieldParts9 = 300;
+template <int Q>
+__host__ __device__ __forceinline__ bool means_in_field(const StepBuffers& S) {
+    return S.nparts - S.part_lo <= (Q == 27 ? kFieldParts27 : kFieldParts9);
+}
+
+// The rows of k_pml_field for D2Q9, two lanes per node; the rest
+// distribution's field is not read.  Where the partial sums are few (means_in_field) each block forms the
+// layer means from them (8 bytes per column and 64 layer nodes), else they are
+// read from k_means.  IN_FIELD false: a launch whose scenes all read them.
+template <bool IN_FIELD>
 __global__ __launch_bounds__(kBlock) void k_pml_field_q9(StepGeom G, StepBuffers S, BatchArgs B) {
     __shared__ double part[kBlock / 16][16];
     __shared__ float means[16];
@@ -400,22 +416,34 @@ __global__ __launch_bounds__(kBlock) void k_pml_field_q9(StepGeom G, StepBuffers
         q1 = reinterpret_cast<const float4*>(S.Qp)[2 * p + q];
         q2 = reinterpret_cast<const float4*>(S.Q2v)[2 * p + q];
     }
-    const int c = threadIdx.x & 15, r = threadIdx.x >> 4;  // column: Q1 of alpha 1 .. 8, then Q2
-    const double* col = S.partial + int64_t((c >> 3) * 9 + 1 + (c & 7)) * S.nparts;
-    double s = 0.0;
+    float m1[4], m2[4];
+    if (IN_FIELD && means_in_field<9>(S)) {
+        const int c = threadIdx.x & 15, r = threadIdx.x >> 4;  // Q1 of alpha 1 .. 8, then Q2
+        const double* col = S.partial + int64_t((c >> 3) * 9 + 1 + (c & 7)) * S.nparts;
+        double s = 0.0;
 #pragma unroll 4
-    for (int t = S.part_lo + r; t < S.nparts; t += kBlock / 16) s += col[t];
-    part[r][c] = s;
-    __syncthreads();
-    if (threadIdx.x < 16) {
-        double t = 0.0;
-        for (int e = 0; e < kBlock / 16; ++e) t += part[e][threadIdx.x];
-        means[threadIdx.x] = float(t / double(G.nlayer));
+        for (int t = S.part_lo + r; t < S.nparts; t += kBlock / 16) s += col[t];
+        part[r][c] = s;
+        __syncthreads();
+        if (threadIdx.x < 16) {
+            double t = 0.0;
+            for (int e = 0; e < kBlock / 16; ++e) t += part[e][threadIdx.x];
+            means[threadIdx.x] = float(t / double(G.nlayer));
+        }
+        __syncthreads();
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            m1[e] = means[4 * q + e];
+            m2[e] = means[8 + 4 * q + e];
+        }
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            m1[e] = S.means[1 + 4 * q + e];
+            m2[e] = S.means[means_stride(9) + 1 + 4 * q + e];
+        }
     }
-    __syncthreads();
     if (!in) return;
-    const float* m1 = means + 4 * q;
-    const float* m2 = means + 8 + 4 * q;
     auto field = [&](float a, float b, int e) {
         return -2.0f * sig * (a - m1[e]) + sig * sig * (b - m2[e]);
     };
@@ -1878,13 +1906,6 @@ __global__ __launch_bounds__(NPB * kV4Lanes) void k_p2_t(StepGeom G, StepBuffers
     st4(S.A, own, make_float4(s.x - r.x, s.y - r.y, s.z - r.z, s.w - r.w));
 }
 
-// Few enough partial layer sums for each field block to read them all (54
-// columns) in about the time of k_means' launch: 128 parts are 64-node blocks
-// of at most 8,192 layer nodes (the 9,261-node cube has about 100).
-__host__ __device__ __forceinline__ bool means_in_field(const StepBuffers& S) {
-    return S.nparts - S.part_lo <= 128;
-}
-
 // PML auxiliary field rows for D3Q27, four distributions per lane (the
 // arithmetic of k_pml_field; padding slots stay zero).
 // Where the layer's partial sums are few (means_in_field) each block forms the
@@ -1907,7 +1928,7 @@ __global__ __launch_bounds__(kBlock) void k_pml_field_v4(StepGeom G, StepBuffers
     const float4 q1 = ld4(rsrc(S.Qp, rows), uint32_t(p) * 128u + lane_off);  // past N: zero
     const float4 q2 = ld4(rsrc(S.Q2v, rows), uint32_t(p) * 128u + lane_off);
     float4 m1, m2;
-    if (IN_FIELD && means_in_field(S)) {
+    if (IN_FIELD && means_in_field<27>(S)) {
         // thread t: column t % 64 (27 of Q1 from 0, 27 of Q2 from 32), every
         // fourth part
         const int c = threadIdx.x & 63, r = threadIdx.x >> 6, a = c & 31;
@@ -2482,13 +2503,17 @@ void launch_pass(int pass, int64_t nb, const StepGeom& G, const StepBuffers& S,
             if (v4) k_pml_local_v4<<<nb, kBlock, 0, st>>>(G, S, c.B);
             else k_pml_local<27><<<nb, kBlock, 0, st>>>(G, S, c.B);
             break;
-        case kPm: k_means<27><<<nb, 256, 0, st>>>(G, S, c.B); break;
+        case kPm: k_means<Q><<<nb, 256, 0, st>>>(G, S, c.B); break;
         case kPf:
-            if (v4 && (c.B.scenes || means_in_field(S)))
-                k_pml_field_v4<true><<<nb, kBlock, 0, st>>>(G, S, c.B);
-            else if (v4) k_pml_field_v4<false><<<nb, kBlock, 0, st>>>(G, S, c.B);
-            else if (Q == 27) k_pml_field<27><<<nb, kBlock, 0, st>>>(G, S, c.B);
-            else k_pml_field_q9<<<nb, kBlock, 0, st>>>(G, S, c.B);
+            if (Q == 27 && !v4) {
+                k_pml_field<27><<<nb, kBlock, 0, st>>>(G, S, c.B);
+            } else if (c.B.scenes || means_in_field<Q>(S)) {
+                if (Q == 27) k_pml_field_v4<true><<<nb, kBlock, 0, st>>>(G, S, c.B);
+                else k_pml_field_q9<true><<<nb, kBlock, 0, st>>>(G, S, c.B);
+            } else {
+                if (Q == 27) k_pml_field_v4<false><<<nb, kBlock, 0, st>>>(G, S, c.B);
+                else k_pml_field_q9<false><<<nb, kBlock, 0, st>>>(G, S, c.B);
+            }
             break;
         case kP2:
             if (c.ktmpl == 32) k_p2<Q, 32><<<nb, kBlock, 0, st>>>(G, S, c.B);
@@ -2552,8 +2577,8 @@ void step_block_counts(int Q, const StepGeom& G, const StepBuffers& S, int64_t* 
                     : p1_uses_dma(Q, un) ? (G.N + kP1Chunk - 1) / kP1Chunk
                                          : (G.N + kP1Block - 1) / kP1Block;
     nb[kPl] = (pml && !fused) ? S.nparts : 0;
-    // (D2Q9: the means are formed in the field pass)
-    nb[kPm] = pml && Q == 27 && !(un && means_in_field(S)) ? 2 * Q : 0;
+    const bool field_means = Q == 27 ? un && means_in_field<27>(S) : means_in_field<9>(S);
+    nb[kPm] = pml && !field_means ? 2 * Q : 0;
     nb[kPf] = !pml ? 0
               : Q == 9 ? (G.nlayer + kBlock / 2 - 1) / (kBlock / 2)
                        : un ? tiles32(G.nlayer) : lanes(G.nlayer);

@@ -1,7 +1,8 @@
 """D2Q9 stencil passes at the edges of their blocks (128 nodes) and record
 groups (four records): single RK4 stages against FP64 numpy, whole steps of
 odd widths against the FP64 oracle and against the one-lane-per-distribution
-kernels, and the saved state's rows."""
+kernels, layers on both sides of the number of partial sums that the field
+pass reads itself, and the saved state's rows."""
 import struct
 
 import numpy as np
@@ -78,3 +79,54 @@ def test_saved_state_rows(oracle64):
     assert np.array_equal(eng.distributions()["g"], g)
     eng.step_forward(2)
     assert np.array_equal(eng.distributions()["g"], want)
+
+
+# nodes per side with a layer over nearly the whole square: 96, 294 and
+# 307 partial sums of 64 layer nodes (the field pass reads up to 300 itself)
+LAYERS = (80, 139, 142)
+
+
+def _wide_layer(oracle, side):
+    h = 1.0 / (side - 1)
+    return h, grid_nodes(oracle, 2, h, 0.49)
+
+
+def test_wide_layers_against_the_oracle(oracle64):
+    scenes = [_wide_layer(oracle64, side) for side in LAYERS]
+    parts = [-(-(n["n_bulk"] + n["n_layer"]) // 64) - n["n_bulk"] // 64 for _, n in scenes]
+    assert parts[0] < parts[1] <= 300 < parts[2]
+    alone, batched = ([gpu_engine(n, 9, 16, h) for h, n in scenes] for _ in range(2))
+    for e in alone + batched:
+        e.set_initial_pulse([0.4, 0.6], 1e-3, 0.1)
+    batch = naga_amd.SceneBatch(batched)
+    batch.step_forward(10)
+    for (h, nodes), e, b in zip(scenes, alone, batched):
+        ref = oracle_engine(oracle64, nodes, 9, 16, h)
+        ref.set_pulse([0.4, 0.6], 1e-3, 0.1)
+        ref.step(10)
+        e.step_forward(10)
+        got, want = e.macroscopic(fresh=True), ref.get(fresh=True)
+        assert rel_l2(got["drho"], want["drho"]) < 1e-5 and rel_l2(got["u"], want["u"]) < 1e-5
+        assert np.array_equal(got["drho"], b.macroscopic(fresh=True)["drho"])
+    batch.close()
+
+
+def test_layer_means_are_linear_in_the_layer():
+    """The field pass and the means, which move a fraction of the bytes that the
+    collision and its PML terms do, take no longer than it does, whatever the
+    layer's width (a million nodes)."""
+    h = 0.001
+    for layer in (0.03, 0.3):
+        nodes = naga_amd.UniformGridProvider([0, 0], [1, 1], h, layer, 0.5, jitter=0.25,
+                                             seed=5).get()
+        eng = naga_amd.SimulationEngine(lattice=9, k=16)
+        p = naga_amd.problem_parameters(9, 0.6, 0.4 * h)
+        eng.set_problem_parameters(p["nu"], 1.0, p["dt"], p["c"])
+        eng.init_domain(nodes)
+        eng.set_initial_pulse([0.4, 0.6], 1e-3, 0.1)
+        eng.step_forward(2)
+        ms = [eng.profile_step() for _ in range(7)]
+        t = {name: float(np.median([m[name] for m in ms])) for name in ms[0]}
+        print(layer, t, flush=True)
+        assert t["pm_layer_means"] + t["pf_pml_field"] < t["p1_collide"] + t["pl_pml_local"]
+        eng.close()
