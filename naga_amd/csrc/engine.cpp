@@ -823,17 +823,10 @@ void Engine::save_state(void* buf, int64_t capacity) {
     char* p = static_cast<char*>(buf);
     std::memcpy(p, &h, sizeof(h));
     p += sizeof(h);
-    for (DeviceBuffer<float>* b : {&g_, &E_, &Qp_}) {
-        if (cfg_.Q == 9 && b != &E_) {
-            std::vector<float> rows(b->size());
-            b->download(rows.data(), rows.size(), stream_);
-            NAGA_HIP(hipStreamSynchronize(stream_));
-            float* out = reinterpret_cast<float*>(p);
-            for (int64_t i = 0; i < N_; ++i)
-                for (int a = 0; a < 9; ++a) std::memcpy(out + i * 9 + a, &rows[row_of(i, a)], 4);
-        } else {
-            b->download(reinterpret_cast<float*>(p), b->size(), stream_);
-        }
+    const bool q9 = cfg_.Q == 9;  // rows as saved in B_ and acc_: a step writes both before it reads them
+    if (q9) launch_plain_rows_q9(N_, g_.get(), Qp_.get(), B_.get(), acc_.get(), true, stream_);
+    for (DeviceBuffer<float>* b : {q9 ? &B_ : &g_, &E_, q9 ? &acc_ : &Qp_}) {
+        b->download(reinterpret_cast<float*>(p), b->size(), stream_);
         p += b->size() * sizeof(float);
     }
     rho_.download(reinterpret_cast<float*>(p), size_t(N_), stream_);
@@ -851,22 +844,15 @@ void Engine::load_state(const void* buf, int64_t bytes) {
             "state was saved from a different scene");
     require(bytes >= state_bytes(), "state buffer truncated");
     const char* p = static_cast<const char*>(buf) + sizeof(h);
-    for (DeviceBuffer<float>* b : {&g_, &E_, &Qp_}) {
-        if (cfg_.Q == 9 && b != &E_) {
-            std::vector<float> rows(b->size());
-            const float* in = reinterpret_cast<const float*>(p);
-            for (int64_t i = 0; i < N_; ++i)
-                for (int a = 0; a < 9; ++a) std::memcpy(&rows[row_of(i, a)], in + i * 9 + a, 4);
-            b->upload(rows.data(), rows.size(), stream_);
-            NAGA_HIP(hipStreamSynchronize(stream_));
-        } else {
-            b->upload(reinterpret_cast<const float*>(p), b->size(), stream_);
-        }
+    const bool q9 = cfg_.Q == 9;  // as in save_state
+    for (DeviceBuffer<float>* b : {q9 ? &B_ : &g_, &E_, q9 ? &acc_ : &Qp_}) {
+        b->upload(reinterpret_cast<const float*>(p), b->size(), stream_);
         p += b->size() * sizeof(float);
     }
     rho_.upload(reinterpret_cast<const float*>(p), size_t(N_), stream_);
     p += size_t(N_) * sizeof(float);
     u_.upload(reinterpret_cast<const float*>(p), size_t(N_) * D_, stream_);
+    if (q9) launch_plain_rows_q9(N_, B_.get(), acc_.get(), g_.get(), Qp_.get(), false, stream_);
     NAGA_HIP(hipStreamSynchronize(stream_));
     time_ = h.time;
     frame_ = h.frame;

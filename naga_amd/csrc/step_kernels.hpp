@@ -275,6 +275,11 @@ template <int Q>
 void launch_pulse(int64_t N, const float* pts, const double* center, double amp, double width,
                   float* g, hipStream_t stream);
 
+// Two D2Q9 row buffers (row_at) to or from plain rows [N][9], the form of saved
+// states: pack copies the row buffers to plain rows, else the reverse.
+void launch_plain_rows_q9(int64_t N, const float* src0, const float* src1, float* dst0, float* dst1,
+                          bool pack, hipStream_t stream);
+
 // Fresh macroscopic values from the current state: rho (FP32, reference
 // units), drho = rho - rho0 in FP64 without cancellation, u (FP32).
 template <int Q>

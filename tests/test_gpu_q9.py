@@ -4,6 +4,7 @@ odd widths against the FP64 oracle and against the one-lane-per-distribution
 kernels, layers on both sides of the number of partial sums that the field
 pass reads itself, and the saved state's rows."""
 import struct
+import time
 
 import numpy as np
 import pytest
@@ -79,6 +80,29 @@ def test_saved_state_rows(oracle64):
     assert np.array_equal(eng.distributions()["g"], g)
     eng.step_forward(2)
     assert np.array_equal(eng.distributions()["g"], want)
+
+
+def test_states_load_at_the_link_rate():
+    """Loading a D2Q9 state takes about as long per byte as a D3Q27 one, whose
+    rows lie on the device as they are saved."""
+    per_byte = []
+    for Q, h in ((27, 0.02), (9, 0.001)):
+        D = 2 if Q == 9 else 3
+        nodes = naga_amd.UniformGridProvider([0] * D, [1] * D, h, 8 * h, 0.5, jitter=0.25,
+                                             seed=5).get()
+        eng = naga_amd.SimulationEngine(lattice=Q, k=16)
+        p = naga_amd.problem_parameters(Q, 0.6, 0.4 * h)
+        eng.set_problem_parameters(p["nu"], 1.0, p["dt"], p["c"])
+        eng.init_domain(nodes)
+        state, t = eng.save_state(), []
+        for _ in range(9):
+            t0 = time.perf_counter()
+            eng.load_state(state)
+            t.append(time.perf_counter() - t0)
+        per_byte.append(float(np.median(t)) / len(state))
+        eng.close()
+    print(per_byte, flush=True)
+    assert per_byte[1] < 2.5 * per_byte[0]
 
 
 # nodes per side with a layer over nearly the whole square: 96, 294 and
