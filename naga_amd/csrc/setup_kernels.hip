@@ -174,18 +174,20 @@ __device__ void knn_rings(const CellGrid& G, const float4* cpts, const uint32_t*
 // One query by the box of cells within R of its own: the points closer than
 // a filter radius (the radius expected to hold about 1.75 k + 8 of them at
 // the box's density, at most the distance to the box's nearest open side)
-// are compacted into LDS, the threshold that leaves k to 64 of them is
-// bisected by ballots, and those are ranked by counting.  Returns false,
-// having written nothing, where the box cannot decide (too few points inside
-// up to R = 3, more than kKnnKeep inside the radius after its retries, more
-// than 64 tied at the threshold): the caller then searches by rings.
+// are compacted into LDS, a bound that leaves k to 64 of them is found by
+// ballots, and those are ranked by counting.  More points than fit are
+// filtered again, below a bound taken from those kept.  Returns false, having
+// written nothing, where the box cannot decide (too few points inside up to
+// R = 3, more than kKnnKeep left after the retries): the caller then searches
+// by rings.
 //
 // Bound by VALU issue, not bytes (1M points: 0.28 GB in and out, 0.05 ms at
 // the card's copy rate).  Merging every cell row into a sorted list of 64-bit
 // keys took 11 wavefront sorts per query; here a candidate costs about 20
 // instructions once and only 64 keys are ordered, by counting smaller ones
 // (broadcast LDS reads, no shuffles).  1,030,301 cube nodes, k = 32: 14.4 ->
-// 1.4 ms; 1M random points 1.7 ms; 1M square nodes, k = 16: 0.8 ms.
+// 1.4 ms; 1M random points 1.7 ms; 1M square nodes, k = 16: 0.8 ms.  200,000
+// points that repeat 300-fold, k = 16: 0.55 ms in 2D (by rings 1.9).
 constexpr int kKnnKeep = 256;   // points kept of one query (four per lane)
 constexpr int kKnnMaxBox = 4096;  // points of a box visited by one wavefront
 constexpr int kKnnBlockQueries = 16;  // queries per block: four per wavefront
@@ -259,8 +261,13 @@ __device__ bool knn_box(const CellGrid& G, double inv_w, const float4* __restric
                           (1.75f * float(k) + 8.0f) / float(T);
         float f2 = D == 3 ? exp2f(log2f(vol * 0.238732f) * (2.0f / 3.0f)) : vol * 0.318310f;
         if (!(f2 < b2)) f2 = b2;
-        for (int attempt = 0; attempt < 4; ++attempt) {
-            // keys of the box's points closer than f2, compacted
+        // points are kept whose key is below lim (their distance below f2, or
+        // past a key known to have at least k below it); none above `most`
+        uint64_t most = uint64_t(__float_as_uint(b2)) << 32;
+        uint64_t lim = uint64_t(__float_as_uint(f2)) << 32;
+        bool shrink = true;  // the radius may still be guessed from the count
+        for (int attempt = 0; attempt < 6; ++attempt) {
+            // keys of the box's points below lim, compacted
             int M = 0;
             for (int r0 = 0; r0 < nrows; r0 += 3) {
                 uint32_t a[3], e[3];
@@ -276,8 +283,7 @@ __device__ bool knn_box(const CellGrid& G, double inv_w, const float4* __restric
                 for (int u = 0; u < 3; ++u)
                     while (a[u] < e[u]) {
                         const uint64_t key = knn_key<D>(x, c[u]);
-                        const bool hit = a[u] + lane < e[u] &&
-                                         __uint_as_float(uint32_t(key >> 32)) < f2;
+                        const bool hit = a[u] + lane < e[u] && key < lim;
                         const uint64_t m = __ballot(hit);
                         const int at = M + __popcll(m & below);
                         if (hit && at < kKnnKeep) keep[at] = key;
@@ -287,13 +293,9 @@ __device__ bool knn_box(const CellGrid& G, double inv_w, const float4* __restric
                     }
             }
             if (M < k) {  // the radius was too small; the whole bound, then a larger box
-                if (!(f2 < b2)) break;
-                f2 = b2;
-                continue;
-            }
-            if (M > kKnnKeep) {  // denser here than over the box
-                const float s = (1.75f * float(k) + 8.0f) / float(M);
-                f2 = fminf(f2, 3.0e38f) * (D == 3 ? exp2f(log2f(s) * (2.0f / 3.0f)) : s);
+                if (lim >= most) break;
+                lim = most;
+                shrink = false;
                 continue;
             }
             wave_lds_fence();
@@ -302,32 +304,67 @@ __device__ bool knn_box(const CellGrid& G, double inv_w, const float4* __restric
             for (int e = 0; e < kKnnKeep / 64; ++e)
                 key[e] = lane + 64 * e < M ? keep[lane + 64 * e] : kMaxKey;
             int C = M;
+            uint64_t t = lim;  // C of the kept keys are below t
             if (M > 64) {
-                // thresholds (distance bits) known to have fewer than k keys
-                // at or below them (lo) and more than 64 (hi); the middle by
-                // value, later by bits, which ends in at most 32 more steps
-                uint32_t lo = 0, hi = __float_as_uint(fminf(f2, 3.4e38f));
-                const float s = (float(k) + 0.5f * float(64 - k)) / float(M);
-                uint32_t mid = __float_as_uint(__uint_as_float(hi) *
-                                               (D == 3 ? exp2f(log2f(s) * (2.0f / 3.0f)) : s));
+                // bounds with fewer than k (lo) and more than 64 (hi) kept
+                // keys below them; the middle by distance, then one of the
+                // keys between them: they are distinct, so that some bound
+                // leaves k to 64 also where distances are equal
+                uint64_t lo = 0, hi = lim;
+                const float s = (float(k) + 0.5f * float(64 - k)) /
+                                float(M < kKnnKeep ? M : kKnnKeep);
+                float v = fminf(f2, 3.4e38f) * (D == 3 ? exp2f(log2f(s) * (2.0f / 3.0f)) : s);
                 for (int step = 0;; ++step) {
+                    if (step < 6) {
+                        t = uint64_t(__float_as_uint(v)) << 32;
+                    } else if (step < 64) {
+                        uint64_t p = 0;
+#pragma unroll
+                        for (int e = 0; e < kKnnKeep / 64; ++e) {
+                            const uint64_t m = __ballot(key[e] >= lo && key[e] < hi);
+                            if (m == 0) continue;
+                            const uint64_t r = m >> ((23 * step) & 63);  // any of them
+                            const int l = int(__ffsll((unsigned long long)(r ? r : m))) - 1 +
+                                          (r ? (23 * step) & 63 : 0);
+                            p = (uint64_t(uint32_t(__builtin_amdgcn_readlane(
+                                     int(uint32_t(key[e] >> 32)), l)))
+                                 << 32) |
+                                uint32_t(__builtin_amdgcn_readlane(int(uint32_t(key[e])), l));
+                        }
+                        t = p + 1 == hi ? p : p + 1;
+                    } else {
+                        return false;
+                    }
                     C = 0;
 #pragma unroll
-                    for (int e = 0; e < kKnnKeep / 64; ++e)
-                        C += __popcll(__ballot(uint32_t(key[e] >> 32) <= mid));
+                    for (int e = 0; e < kKnnKeep / 64; ++e) C += __popcll(__ballot(key[e] < t));
                     if (C >= k && C <= 64) break;
-                    if (C < k) lo = mid;
-                    else hi = mid;
-                    if (hi - lo <= 1) return false;  // ties across the window
-                    mid = step < 8 ? __float_as_uint(0.5f * (__uint_as_float(lo) +
-                                                             __uint_as_float(hi)))
-                                   : lo + (hi - lo) / 2;
+                    if (C < k) lo = t;
+                    else hi = t;
+                    v = 0.5f * (__uint_as_float(uint32_t(lo >> 32)) +
+                                __uint_as_float(uint32_t(hi >> 32)));
                 }
+            }
+            if (M > kKnnKeep) {  // denser here than over the box: t has k below it
+                most = t;
+                if (shrink) {
+                    const float s = (1.75f * float(k) + 8.0f) / float(M);
+                    f2 = fminf(f2, 3.0e38f) * (D == 3 ? exp2f(log2f(s) * (2.0f / 3.0f)) : s);
+                    const uint64_t by_count = uint64_t(__float_as_uint(f2)) << 32;
+                    lim = by_count < most ? by_count : most;
+                    shrink = false;
+                } else {
+                    lim = most;
+                }
+                f2 = fminf(f2, __uint_as_float(uint32_t(lim >> 32)));
+                continue;
+            }
+            if (M > 64) {
                 wave_lds_fence();  // the keys are in registers
                 int at = 0;
 #pragma unroll
                 for (int e = 0; e < kKnnKeep / 64; ++e) {
-                    const bool hit = uint32_t(key[e] >> 32) <= mid;
+                    const bool hit = key[e] < t;
                     const uint64_t m = __ballot(hit);
                     if (hit) keep[at + __popcll(m & below)] = key[e];
                     at += __popcll(m);

@@ -2,8 +2,11 @@
 (evenly spread points), radii retried (clusters, edges of the cloud), rings
 (ties beyond a wavefront, points far apart, distances past the largest
 float), against brute force with the same FP32 keys."""
+import time
+
 import numpy as np
 import pytest
+import torch
 
 import naga_amd
 
@@ -61,6 +64,51 @@ def test_knn_matches_brute_force(D, kind, n, k):
     want_d2, want_idx = _brute(ref, query, k)
     assert np.array_equal(idx, want_idx)
     assert np.array_equal(d2.view(np.uint32), want_d2.view(np.uint32))
+
+
+@pytest.mark.parametrize("D", [2, 3])
+@pytest.mark.parametrize("times", [65, 255, 257, 400, 1500])
+@pytest.mark.parametrize("k", [1, 17, 64])
+def test_repeated_points_match_brute_force(D, times, k):
+    """Groups of equal points around the sizes of a wavefront and of a query's
+    kept points, so that ties run through every bound: indices decide."""
+    rng = np.random.default_rng(times + k)
+    ref = np.repeat(rng.random((12, D)).astype(np.float32), times, axis=0)[rng.permutation(12 * times)]
+    query = np.concatenate([ref[:40], rng.random((60, D)).astype(np.float32)])
+    print(f"kNN D={D} times={times} k={k}", flush=True)
+    d2, idx = naga_amd.batched_nearest_neighbors(k, query, ref)
+    want_d2, want_idx = _brute(ref, query, k)
+    assert np.array_equal(idx, want_idx)
+    assert np.array_equal(d2.view(np.uint32), want_d2.view(np.uint32))
+
+
+def _device_time(ref, k):
+    """Median time (s) of the search of ref's own neighbours, on device arrays."""
+    n, D = ref.shape
+    r = torch.from_numpy(ref).cuda()
+    d2 = torch.empty(n, k, dtype=torch.float32, device="cuda")
+    idx = torch.empty(n, k, dtype=torch.int32, device="cuda")
+    t = []
+    for _ in range(7):
+        torch.cuda.synchronize()
+        t0 = time.perf_counter()
+        assert naga_amd.load().naga_knn_noalloc(
+            r.data_ptr(), n, r.data_ptr(), n, D, k, d2.data_ptr(), idx.data_ptr(),
+            torch.cuda.current_stream().cuda_stream) == 0
+        torch.cuda.synchronize()
+        t.append(time.perf_counter() - t0)
+    return float(np.median(t))
+
+
+@pytest.mark.parametrize("D", [2, 3])
+def test_repeated_points_take_no_rings(D):
+    """300-fold repeated points are searched in a few times the time of as many
+    random ones (by rings of cells it was eight to fourteen times)."""
+    rng = np.random.default_rng(D)
+    p = rng.random((199800, D)).astype(np.float32)
+    t = [_device_time(c, 16) for c in (p, np.repeat(p[:666], 300, axis=0))]
+    print(t, flush=True)
+    assert t[1] < 4.0 * t[0]
 
 
 @pytest.mark.parametrize("approx", [1, 8, 64, 5000])
