@@ -73,7 +73,7 @@ Advection::Advection(const float* pts, int64_t n, int D, int k, int rbf) : n_(n)
     try {
         DeviceBuffer<float> dp(n * D);
         dp.upload(pts, n * D, st_);
-        const DeviceCells cells = bin_points_device(D, dp.get(), n, st_, knn_points_per_cell(D, k));
+        const DeviceCells cells = knn_bins_device(D, dp.get(), n, k, st_);
         DeviceBuffer<float> d2(n * k);
         idx_.allocate(n * k);
         launch_knn(D, cells.bins, dp.get(), n, k, d2.get(), idx_.get(), st_);

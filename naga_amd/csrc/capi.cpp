@@ -928,7 +928,8 @@ int naga_knn_noalloc(const float* ref, int64_t n_ref, const float* query, int64_
         hipStream_t st = static_cast<hipStream_t>(stream);
         void* mem = scratch_of_current_device();
         const CellBins bins = launch_bin_points(
-            dims, ref, n_ref, knn_points_per_cell(dims, k), 0.0, mem, kNoAllocBytes, st);
+            dims, ref, n_ref, knn_points_per_cell(dims, k), 0.0, mem, kNoAllocBytes, st,
+            kKnnCrowdedPerCell);
         launch_knn(dims, bins, query, n_q, k, d2_out, idx_out, st);
     });
 }

@@ -79,7 +79,7 @@ void knn_host(int D, const float* ref, int64_t n_ref, const float* query, int64_
     DeviceBuffer<uint32_t> didx(n_q * k);
     dref.upload(ref, n_ref * D, st);
     dq.upload(query, n_q * D, st);
-    const DeviceCells cells = bin_points_device(D, dref.get(), n_ref, st, knn_points_per_cell(D, k));
+    const DeviceCells cells = knn_bins_device(D, dref.get(), n_ref, k, st);
     launch_knn(D, cells.bins, dq.get(), n_q, k, dd2.get(), didx.get(), st);
     dd2.download(d2, n_q * k, st);
     didx.download(idx, n_q * k, st);
@@ -168,7 +168,7 @@ void Engine::init_domain(const float* pts, int64_t nbulk, int64_t nlayer, int64_
 
     // divergence operator over all nodes (init_domain :169-181)
     {
-        const DeviceCells cells = bin_points_device(D, pts_.get(), N, st, knn_points_per_cell(D, k));
+        const DeviceCells cells = knn_bins_device(D, pts_.get(), N, k, st);
         DeviceBuffer<float> d2(N * k);
         idx_.allocate(N * k);
         launch_knn(D, cells.bins, pts_.get(), N, k, d2.get(), idx_.get(), st);
@@ -436,8 +436,7 @@ void Engine::init_domain(const float* pts, int64_t nbulk, int64_t nlayer, int64_
     // boundary interpolator (init_domain :223-258): kNN of boundary nodes
     // among the bulk and layer nodes, RPIM weights at spacing h
     if (nbnd > 0) {
-        const DeviceCells cells = bin_points_device(D, pts_.get(), nfluid, st,
-                                                    knn_points_per_cell(D, kb));
+        const DeviceCells cells = knn_bins_device(D, pts_.get(), nfluid, kb, st);
         DeviceBuffer<float> bd2(nbnd * kb);
         bidx_.allocate(nbnd * kb);
         launch_knn(D, cells.bins, pts_.get() + nfluid * D, nbnd, kb, bd2.get(),

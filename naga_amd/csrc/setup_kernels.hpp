@@ -22,6 +22,7 @@ struct CellGrid {
     double w;          // cell width
     int64_t dims[3];
     int64_t ncell;
+    double ext[3];     // extents of the points (at least 1e-3)
     int D;
 };
 
@@ -37,12 +38,12 @@ struct CellBins {
     int64_t n;
 };
 // Scratch layout of one binning of n points (offsets 256-byte aligned):
-// the grid, per-block bounds, cell counts and starts, scan block sums, the
-// sorted indices and the points in that order.
+// the grid, per-block bounds, cell counts and starts, scan block sums and pairs
+// of points sharing a cell, the sorted indices and the points in that order.
 constexpr int kBoundBlocks = 256;
 constexpr int kScanChunk = 2048;  // elements per scan block: 256 threads x 8
 struct BinLayout {
-    size_t grid, partial, counts, start, bsum, sorted, pts, total;
+    size_t grid, partial, counts, start, bsum, pairs, sorted, pts, total;
     int64_t cap, nblocks;
 };
 constexpr size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
@@ -62,6 +63,8 @@ constexpr BinLayout bin_layout(int64_t n) {
     off = align256(off + size_t(M) * 4);
     L.bsum = off;
     off = align256(off + size_t(L.nblocks) * 4);
+    L.pairs = off;
+    off = align256(off + size_t(L.nblocks) * 8);
     L.sorted = off;
     off = align256(off + size_t(n) * 4);
     L.pts = off;
@@ -75,19 +78,29 @@ size_t cell_bins_bytes(int64_t n);
 // Bins pts[n][D] (device) into scratch (device, at least cell_bins_bytes(n)
 // bytes, 256-byte aligned) on `stream`: per_cell > 0 sets the width from the
 // points per cell, else width > 0 is the cell width.  Allocates nothing.
+// crowded_per_cell (with per_cell, 0: none): the points per cell instead where
+// the cloud is crowded, that is where a point has on average more than
+// kCrowded times per_cell others in its cell.
+constexpr double kCrowded = 8.0;
 CellBins launch_bin_points(int D, const float* pts, int64_t n, double per_cell, double width,
-                           void* scratch, size_t bytes, hipStream_t stream);
+                           void* scratch, size_t bytes, hipStream_t stream,
+                           double crowded_per_cell = 0.0);
 // Binning with its own device memory.
 struct DeviceCells {
     DeviceBuffer<uint8_t> mem;
     CellBins bins{};
 };
 DeviceCells bin_points_device(int D, const float* pts, int64_t n, hipStream_t stream,
-                              double per_cell, double width = 0.0);
+                              double per_cell, double width = 0.0,
+                              double crowded_per_cell = 0.0);
 // Points per cell for a search of k neighbours: the cell width is then 1.1
 // times the radius that holds k points at the cloud's mean density, so the
-// 3^D cells around a query bound a ball that holds its k nearest.
+// 3^D cells around a query bound a ball that holds its k nearest.  Such cells
+// hold far more where the cloud is crowded (clusters, points on a curve), and
+// every query visits at least its own: kKnnCrowdedPerCell points per cell then.
 double knn_points_per_cell(int D, int k);
+constexpr double kKnnCrowdedPerCell = 2.0;
+DeviceCells knn_bins_device(int D, const float* pts, int64_t n, int k, hipStream_t stream);
 
 // Exact k-nearest neighbours of each query among ref, key (d2, index)
 // ascending, d2 in FP32 as dz^2 + (dy^2 + dx^2) with no contraction.

@@ -111,6 +111,43 @@ def test_repeated_points_take_no_rings(D):
     assert t[1] < 4.0 * t[0]
 
 
+def _crowded(kind, D, n, rng):
+    """Clouds that leave most of their bounding box empty."""
+    if kind == "circle":
+        p = rng.standard_normal((n, D))
+        p[:, 2:] *= 0.01
+        return (p / np.linalg.norm(p, axis=1, keepdims=True)).astype(np.float32)
+    p = rng.random((n, D))  # "blob": nine tenths within about 0.05
+    p[: 9 * n // 10] = 0.5 + 0.02 * rng.standard_normal((9 * n // 10, D))
+    return p.astype(np.float32)
+
+
+@pytest.mark.parametrize("D", [2, 3])
+@pytest.mark.parametrize("kind", ["circle", "blob"])
+@pytest.mark.parametrize("k", [2, 9, 32, 64])
+def test_crowded_clouds_match_brute_force(D, kind, k):
+    rng = np.random.default_rng(k)
+    ref = _crowded(kind, D, 6000, rng)
+    query = np.concatenate([ref[::20], rng.uniform(-1.2, 1.2, (100, D)).astype(np.float32)])
+    print(f"kNN D={D} {kind} k={k}", flush=True)
+    d2, idx = naga_amd.batched_nearest_neighbors(k, query, ref)
+    want_d2, want_idx = _brute(ref, query, k)
+    assert np.array_equal(idx, want_idx)
+    assert np.array_equal(d2.view(np.uint32), want_d2.view(np.uint32))
+
+
+@pytest.mark.parametrize("k", [32, 64])
+def test_crowded_clouds_get_narrow_cells(k):
+    """200,000 points on a circle are searched in less than three times the time
+    of as many random ones (in cells sized for k points at the mean density it
+    was four to five times)."""
+    rng = np.random.default_rng(k)
+    p = rng.random((200000, 2)).astype(np.float32)
+    t = [_device_time(c, k) for c in (p, _crowded("circle", 2, 200000, rng))]
+    print(t, flush=True)
+    assert t[1] < 3.0 * t[0]
+
+
 @pytest.mark.parametrize("approx", [1, 8, 64, 5000])
 def test_knn_of_segmentations_matches_brute_force(approx):
     """Cells of any size given by the caller."""
