@@ -67,6 +67,13 @@ typedef struct naga_scene_config {
 
 const char* naga_last_error(void);
 
+/* Device memory that handles release is kept for later ones, up to 4 GiB per
+ * process (past that the memory released first is freed).  Gives it back until
+ * at most keep_bytes are kept, for the program's own allocations or another
+ * library's; *kept_bytes (not NULL) receives what is kept then.  Waits for the
+ * device where it frees. */
+int naga_trim_memory(int64_t keep_bytes, int64_t* kept_bytes);
+
 /* Lattice tables: c[Q*D], w[Q], bb[Q], K[Q*Q] (row alpha, column j).
  * detail/d2q9_lattice.cuh:44-88,151-163; detail/d3q27_lattice.cuh:45-105,
  * 380-387. */
@@ -217,8 +224,9 @@ int naga_batch_step_timed(naga_batch* b, int32_t nsteps, double* ms);
  *      max_active are resident; setup_threads threads build admitted scenes
  *      (host node generation, GPU setup on each scene's own stream) while a
  *      stepping thread advances all resident scenes together in chunks of
- *      at most chunk_steps steps; finished scenes leave at once and free
- *      their memory.  Scenes are the unit box minus obstacles
+ *      at most chunk_steps steps; finished scenes leave at once and release
+ *      their memory (what is kept of it for later scenes, naga_trim_memory,
+ *      is cut to the rest of the budget when a request is admitted).  Scenes are the unit box minus obstacles
  *      (naga_obstacle_grid), dt = 0.4 of the finest spacing (h, or h/2
  *      with refinement), c = c_s, rho0 = 1, r^3 RBFs. */
 typedef struct naga_server naga_server;

@@ -91,6 +91,7 @@ def load() -> C.CDLL:
     i32, i64, f64, u64 = C.c_int32, C.c_int64, C.c_double, C.c_uint64
     sig = {
         "naga_last_error": (C.c_char_p, []),
+        "naga_trim_memory": (C.c_int, [i64, vp]),
         "naga_lattice_tables": (C.c_int, [i32, vp, vp, vp, vp]),
         "naga_collide": (C.c_int, [i32, vp, f64, vp, f64, f64, vp]),
         "naga_engine_create": (C.c_int, [C.POINTER(SceneConfig), C.POINTER(vp)]),
@@ -177,7 +178,7 @@ def load() -> C.CDLL:
 
 
 EXPORTED = [
-    "naga_last_error", "naga_lattice_tables", "naga_collide",
+    "naga_last_error", "naga_trim_memory", "naga_lattice_tables", "naga_collide",
     "naga_engine_create", "naga_engine_destroy", "naga_engine_init_domain",
     "naga_engine_set_pulse", "naga_engine_set_distributions", "naga_engine_step",
     "naga_engine_step_timed", "naga_engine_profile_step",
@@ -231,6 +232,14 @@ def _f32(a):
 
 def _f64(a):
     return np.ascontiguousarray(a, dtype=np.float64)
+
+
+def trim_memory(keep_bytes: int = 0) -> int:
+    """Gives device memory kept for later scenes back until at most keep_bytes
+    are kept (naga_trim_memory); returns what is kept then."""
+    kept = np.zeros(1, np.int64)
+    _check(load().naga_trim_memory(int(keep_bytes), _ptr(kept)))
+    return int(kept[0])
 
 
 # ---------------------------------------------------------------- lattices

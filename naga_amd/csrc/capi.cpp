@@ -179,6 +179,14 @@ extern "C" {
 
 const char* naga_last_error(void) { return g_last_error.c_str(); }
 
+int naga_trim_memory(int64_t keep_bytes, int64_t* kept_bytes) {
+    return guarded([&] {
+        require(keep_bytes >= 0, "keep_bytes must not be negative");
+        const size_t kept = device_trim(size_t(keep_bytes));
+        if (kept_bytes) *kept_bytes = int64_t(kept);
+    });
+}
+
 int naga_lattice_tables(int32_t q, double* c, double* w, int32_t* bb, double* K) {
     return guarded([&] {
         require(q == 9 || q == 27, "lattice must be 9 or 27");

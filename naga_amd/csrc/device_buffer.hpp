@@ -14,6 +14,9 @@ void* device_allocate(size_t bytes);
 // Gives a block back.  Work on any stream may still use it: it is handed out
 // again only after the device has been synchronised.
 void device_release(void* p) noexcept;
+// Frees the blocks kept longest until at most `keep` bytes are; returns what is
+// kept.  Any thread.
+size_t device_trim(size_t keep);
 
 template <class T>
 class DeviceBuffer {

@@ -183,7 +183,7 @@ naga_server_stats Server::stats() {
 void Server::setup_loop() {
     for (;;) {
         Pending p;
-        size_t bytes = 0;
+        size_t bytes = 0, left = 0;
         int64_t n = 0;
         {
             std::unique_lock<std::mutex> lk(mu_);
@@ -214,7 +214,10 @@ void Server::setup_loop() {
             queue_.pop_front();
             used_ += bytes;
             ++resident_;
+            left = budget_ > used_ ? budget_ - used_ : 0;
         }
+        // the memory kept for reuse counts against the budget too
+        device_trim(left);
         Active a;
         a.id = p.id;
         a.t_submit = p.t_submit;

@@ -6,7 +6,8 @@
 // GPU on the scene's own stream) while a stepping thread advances every
 // resident scene together through one Batch; scenes join at the next
 // chunk boundary and leave as soon as their step count is reached, their
-// results copied out and their memory released.  State and stencils stay
+// results copied out and their memory released (the blocks kept of it for the
+// next scenes are cut to the rest of the budget at each admission).  State and stencils stay
 // on the device for the whole solve.
 #pragma once
 

@@ -1,10 +1,12 @@
-"""Device blocks kept between allocations: scenes rebuilt in memory that other
-scenes used, one after another and from several threads at once, give the
-results of their first build bit for bit."""
+"""Device blocks kept between allocations: given back on request and within a
+server's budget, and scenes rebuilt in memory that other scenes used, one after
+another and from several threads at once, give the results of their first build
+bit for bit."""
 import threading
 
 import numpy as np
 import pytest
+import torch
 
 import naga_amd
 from tests.scenes import gpu_engine, grid_nodes
@@ -21,6 +23,35 @@ def _solve(nodes, Q, k, h):
     out = eng.macroscopic(fresh=True)
     eng.close()
     return out
+
+
+def test_kept_memory_is_given_back(oracle64):
+    """Closed scenes' memory is kept for the next, and returned to the driver by
+    trim_memory."""
+    nodes = grid_nodes(oracle64, 3, 0.04, 0.08)
+    gpu_engine(nodes, 27, 32, 0.04, kb=16).close()  # the process' own memory: code, queues
+    naga_amd.trim_memory()
+    free = torch.cuda.mem_get_info()[0]
+    gpu_engine(nodes, 27, 32, 0.04, kb=16).close()
+    kept = naga_amd.trim_memory(1 << 40)
+    assert kept > 10 << 20 and torch.cuda.mem_get_info()[0] < free
+    assert naga_amd.trim_memory(kept // 2) <= kept // 2
+    assert naga_amd.trim_memory() == 0
+    assert torch.cuda.mem_get_info()[0] >= free - (2 << 20)
+
+
+def test_server_keeps_within_its_budget(oracle64):
+    """Memory kept from earlier scenes counts against a server's budget."""
+    nodes = grid_nodes(oracle64, 3, 0.03, 0.06)
+    gpu_engine(nodes, 27, 32, 0.03, kb=16).close()
+    budget = 64 << 20
+    assert naga_amd.trim_memory(1 << 40) > budget
+    srv = naga_amd.SolveServer(hbm_budget_bytes=budget, max_active=4, chunk_steps=5)
+    rid = srv.submit(naga_amd.make_request(9, 0.03125, 5))
+    srv.drain()
+    srv.result(rid)
+    srv.close()
+    assert naga_amd.trim_memory(1 << 40) <= budget
 
 
 def _same(a, b):
