@@ -48,6 +48,11 @@ __device__ __forceinline__ BlockCtx locate(const BatchArgs& B, StepGeom& G, Step
     return {int64_t(blockIdx.x) - B.bstart[lo], int64_t(B.bstart[lo + 1] - B.bstart[lo]), lo};
 }
 
+// element e (compile-time after unrolling) of a 16-byte vector
+__device__ __forceinline__ float get(const float4& v, int e) {
+    return e == 0 ? v.x : e == 1 ? v.y : e == 2 ? v.z : v.w;
+}
+
 template <int Q>
 struct LaneMap {
     using L = Lattice<Q>;
@@ -470,19 +475,20 @@ template <int Q, int NC>
 __device__ __forceinline__ int rec_floats(int K) {
     return Q == 27 ? K * (1 + NC) : 4 * q9_units(K, NC);
 }
-// Field f (0: index) of record s in the row r.
-template <int Q, int NC>
-__device__ __forceinline__ float rec_field(const float* r, int s, int f) {
-    return Q == 27 ? r[s * (1 + NC) + f] : r[((s >> 2) * (1 + NC) + f) * 4 + (s & 3)];
-}
-
 // Copy the record rows (RW floats, a multiple of two) of nodes [node0, node0
-// + cnt) into lds.
+// + cnt) into lds, 16 bytes a lane where the rows are whole 16-byte units (all
+// but D3Q27 filter records of odd widths).
+template <class V>
+__device__ __forceinline__ void copy_units(const float* src, int n, float* lds) {
+    const V* s = reinterpret_cast<const V*>(src);
+    V* d = reinterpret_cast<V*>(lds);
+    for (int t = threadIdx.x; t < n; t += kBlock) d[t] = s[t];
+}
 __device__ __forceinline__ void stage_contiguous(const float* slab, int64_t node0, int cnt, int RW,
                                                  float* lds) {
-    const float2* s2 = reinterpret_cast<const float2*>(slab + node0 * int64_t(RW));
-    float2* d2 = reinterpret_cast<float2*>(lds);
-    for (int t = threadIdx.x; t < cnt * RW / 2; t += kBlock) d2[t] = s2[t];
+    const float* src = slab + node0 * int64_t(RW);
+    if (RW % 4 == 0) copy_units<float4>(src, cnt * (RW / 4), lds);
+    else copy_units<float2>(src, cnt * (RW / 2), lds);
 }
 
 // Copy the records of one node (lanes of the node share the work).
@@ -521,24 +527,44 @@ __device__ __forceinline__ float stencil_sum(const float* rp, int K, const float
     const int64_t pitch = row_pitch<Q>(a);
     const float cx = lane_c<Q>(a, 0), cy = lane_c<Q>(a, 1),
                 cz = D == 3 ? lane_c<Q>(a, 2) : 0.0f;
+    const float4* rp4 = reinterpret_cast<const float4*>(rp);
     float acc = 0.0f;
 #pragma unroll
     for (int s0 = 0; s0 < KMAX; s0 += BATCH) {
         if (!KT && s0 >= K) break;
         float v[BATCH], gv[BATCH];
         uint32_t j[BATCH];
+        if constexpr (Q == 9) {  // groups of four records; the fill's weights are zero
 #pragma unroll
-        for (int u = 0; u < BATCH; ++u) {
-            const int s = s0 + u;
-            const bool in = KT ? (s < KT) : (s < K);
-            const int t = in ? s : 0;
-            j[u] = __float_as_uint(rec_field<Q, D>(rp, t, 0));
-            float w = cx * rec_field<Q, D>(rp, t, 1) + cy * rec_field<Q, D>(rp, t, 2);
-            if (D == 3) w += cz * rec_field<Q, D>(rp, t, 3);
-            v[u] = in ? w : 0.0f;
+            for (int u = 0; u < BATCH; u += 4) {
+                const bool in = KT ? (s0 + u < KT) : (s0 + u < K);
+                const float4* r = rp4 + (in ? (s0 + u) / 4 * 3 : 0);
+                const float4 ji = r[0], wx = r[1], wy = r[2];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    j[u + e] = __float_as_uint(get(ji, e));
+                    v[u + e] = in ? cx * get(wx, e) + cy * get(wy, e) : 0.0f;
+                }
+            }
+        } else {
+#pragma unroll
+            for (int u = 0; u < BATCH; ++u) {
+                const int s = s0 + u;
+                const bool in = KT ? (s < KT) : (s < K);
+                const float4 r = rp4[in ? s : 0];
+                j[u] = __float_as_uint(r.x);
+                const float w = cx * r.y + cy * r.z + cz * r.w;
+                v[u] = in ? w : 0.0f;
+            }
         }
+        // the D2Q9 rest value lies apart from the row, and its weight is zero:
+        // its lane gathers nothing
 #pragma unroll
-        for (int u = 0; u < BATCH; ++u) gv[u] = col[int64_t(j[u]) * pitch];
+        for (int u = 0; u < BATCH; ++u) gv[u] = 0.0f;
+        if (Q != 9 || a != 0) {
+#pragma unroll
+            for (int u = 0; u < BATCH; ++u) gv[u] = col[int64_t(j[u]) * pitch];
+        }
 #pragma unroll
         for (int u = 0; u < BATCH; ++u) acc += v[u] * gv[u];
     }
@@ -555,7 +581,7 @@ __global__ __launch_bounds__(kBlock) void k_p2(StepGeom G, StepBuffers S, BatchA
     using L = Lattice<Q>;
     constexpr int D = L::D, REC = 1 + D, KMAX = KT ? KT : 64;
     constexpr int NPB = Tile<Q>::NPB;
-    __shared__ float srec[NPB * KMAX * REC];
+    __shared__ alignas(16) float srec[NPB * KMAX * REC];
     const BlockCtx bc = locate(B, G, S);
     const int K = KT ? KT : G.k;
     const Lanes<Q> ln;
@@ -611,7 +637,7 @@ __global__ __launch_bounds__(kBlock) void k_p4(StepGeom G, StepBuffers S, BatchA
     using L = Lattice<Q>;
     constexpr int D = L::D, KMAX = KT ? KT : 64;
     constexpr int NPB = Tile<Q>::NPB;
-    __shared__ float srec[NPB * KMAX * 2];
+    __shared__ alignas(16) float srec[NPB * KMAX * 2];
     const BlockCtx bc = locate(B, G, S);
     const int K = KT ? KT : G.k;
     const int64_t node0 = xcd_tile(bc.b, bc.nb) * NPB;
@@ -636,12 +662,27 @@ __global__ __launch_bounds__(kBlock) void k_p4(StepGeom G, StepBuffers S, BatchA
             if (!KT && s0 >= K) break;
             float w[8], gv[8];
             uint32_t j[8];
+            if constexpr (Q == 9) {  // groups of four records; the fill's weights are zero
 #pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const int s = s0 + u;
-                const bool in = KT ? (s < KT) : (s < K);
-                j[u] = __float_as_uint(rec_field<Q, 1>(rp, in ? s : 0, 0));
-                w[u] = in ? rec_field<Q, 1>(rp, s, 1) : 0.0f;
+                for (int u = 0; u < 8; u += 4) {
+                    const bool in = KT ? (s0 + u < KT) : (s0 + u < K);
+                    const float4* r = reinterpret_cast<const float4*>(rp) + (in ? (s0 + u) / 2 : 0);
+                    const float4 ji = r[0], wi = r[1];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        j[u + e] = __float_as_uint(get(ji, e));
+                        w[u + e] = in ? get(wi, e) : 0.0f;
+                    }
+                }
+            } else {
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    const int s = s0 + u;
+                    const bool in = KT ? (s < KT) : (s < K);
+                    const float2 r = reinterpret_cast<const float2*>(rp)[in ? s : 0];
+                    j[u] = __float_as_uint(r.x);
+                    w[u] = in ? r.y : 0.0f;
+                }
             }
 #pragma unroll
             for (int u = 0; u < 8; ++u) gv[u] = col[int64_t(j[u]) * pitch];
@@ -721,7 +762,7 @@ __global__ __launch_bounds__(kBlock) void k_stage(StepGeom G, StepBuffers S, Bat
     using L = Lattice<Q>;
     constexpr int D = L::D, REC = 1 + D, KMAX = KT ? KT : 64;
     constexpr int NPB = Tile<Q>::NPB;
-    __shared__ float srec[NPB * KMAX * REC];
+    __shared__ alignas(16) float srec[NPB * KMAX * REC];
     const BlockCtx bc = locate(B, G, S);
     const int K = KT ? KT : G.k;
     const int64_t node0 = xcd_tile(bc.b, bc.nb) * NPB;
@@ -797,9 +838,6 @@ __device__ __forceinline__ void st4(float* base, uint32_t off, float4 v) {
     *reinterpret_cast<float4*>(reinterpret_cast<char*>(base) + off) = v;
 }
 
-__device__ __forceinline__ float get(const float4& v, int e) {
-    return e == 0 ? v.x : e == 1 ? v.y : e == 2 ? v.z : v.w;
-}
 
 __device__ __forceinline__ void set(float4& v, int e, float x) {
     if (e == 0) v.x = x;
