@@ -1286,12 +1286,14 @@ __global__ __launch_bounds__(256) void k_grid(const double* partial, int D, int6
 // linear index with x fastest (the kNN's cell rows).
 __device__ __forceinline__ int64_t cell_of(const CellGrid& G, const float* p) {
     int64_t c = 0, mul = 1;
-    for (int d = 0; d < G.D; ++d) {
-        int64_t ci = int64_t(floor((double(p[d]) - G.lo[d]) / G.w));
-        ci = ci < 0 ? 0 : ci >= G.dims[d] ? G.dims[d] - 1 : ci;
-        c += ci * mul;
-        mul *= G.dims[d];
-    }
+#pragma unroll  // (indexed at run time the grid would be copied to scratch memory)
+    for (int d = 0; d < 3; ++d)
+        if (d < G.D) {
+            int64_t ci = int64_t(floor((double(p[d]) - G.lo[d]) / G.w));
+            ci = ci < 0 ? 0 : ci >= G.dims[d] ? G.dims[d] - 1 : ci;
+            c += ci * mul;
+            mul *= G.dims[d];
+        }
     return c;
 }
 
@@ -1348,7 +1350,7 @@ __device__ __forceinline__ void scan_chunk(uint32_t* in, int64_t M, uint32_t* ou
     for (int e = 0; e < 8; ++e) {
         if (base + e < M) {
             out[base + e] = run;
-            in[base + e] = 0u;
+            if (v[e]) in[base + e] = 0u;
         }
         run += v[e];
     }
@@ -1439,7 +1441,9 @@ __global__ __launch_bounds__(256) void k_scatter_cells(const float* pts, int64_t
     if (j >= n) return;
     const CellGrid G = *gp;
     float p[3] = {0.f, 0.f, 0.f};
-    for (int d = 0; d < G.D; ++d) p[d] = pts[j * G.D + d];
+#pragma unroll
+    for (int d = 0; d < 3; ++d)
+        if (d < G.D) p[d] = pts[j * G.D + d];
     const int64_t c = cell_of(G, p);
     const uint32_t at = start[c] + atomicAdd(&fill[c], 1u);
     sorted[at] = uint32_t(j);
