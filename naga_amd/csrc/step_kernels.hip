@@ -404,8 +404,9 @@ __host__ __device__ __forceinline__ bool means_in_field(const StepBuffers& S) {
 // The rows of k_pml_field for D2Q9, two lanes per node; the rest
 // distribution's field is not read.  Where the partial sums are few (means_in_field) each block forms the
 // layer means from them (8 bytes per column and 64 layer nodes), else they are
-// read from k_means.  IN_FIELD false: a launch whose scenes all read them.
-template <bool IN_FIELD>
+// read from k_means: MEANS says which, or that each scene of a batch decides.
+enum Means { kMeansRead, kMeansFormed, kMeansByScene };
+template <Means MEANS>
 __global__ __launch_bounds__(kBlock) void k_pml_field_q9(StepGeom G, StepBuffers S, BatchArgs B) {
     __shared__ double part[kBlock / 16][16];
     __shared__ float means[16];
@@ -422,7 +423,7 @@ __global__ __launch_bounds__(kBlock) void k_pml_field_q9(StepGeom G, StepBuffers
         q2 = reinterpret_cast<const float4*>(S.Q2v)[2 * p + q];
     }
     float m1[4], m2[4];
-    if (IN_FIELD && means_in_field<9>(S)) {
+    if (MEANS == kMeansFormed || (MEANS == kMeansByScene && means_in_field<9>(S))) {
         const int c = threadIdx.x & 15, r = threadIdx.x >> 4;  // Q1 of alpha 1 .. 8, then Q2
         const double* col = S.partial + int64_t((c >> 3) * 9 + 1 + (c & 7)) * S.nparts;
         double s = 0.0;
@@ -2559,12 +2560,15 @@ void launch_pass(int pass, int64_t nb, const StepGeom& G, const StepBuffers& S,
         case kPf:
             if (Q == 27 && !v4) {
                 k_pml_field<27><<<nb, kBlock, 0, st>>>(G, S, c.B);
-            } else if (c.B.scenes || means_in_field<Q>(S)) {
-                if (Q == 27) k_pml_field_v4<true><<<nb, kBlock, 0, st>>>(G, S, c.B);
-                else k_pml_field_q9<true><<<nb, kBlock, 0, st>>>(G, S, c.B);
+            } else if (Q == 27) {
+                if (c.B.scenes || means_in_field<27>(S))
+                    k_pml_field_v4<true><<<nb, kBlock, 0, st>>>(G, S, c.B);
+                else k_pml_field_v4<false><<<nb, kBlock, 0, st>>>(G, S, c.B);
             } else {
-                if (Q == 27) k_pml_field_v4<false><<<nb, kBlock, 0, st>>>(G, S, c.B);
-                else k_pml_field_q9<false><<<nb, kBlock, 0, st>>>(G, S, c.B);
+                if (c.B.scenes) k_pml_field_q9<kMeansByScene><<<nb, kBlock, 0, st>>>(G, S, c.B);
+                else if (means_in_field<9>(S))
+                    k_pml_field_q9<kMeansFormed><<<nb, kBlock, 0, st>>>(G, S, c.B);
+                else k_pml_field_q9<kMeansRead><<<nb, kBlock, 0, st>>>(G, S, c.B);
             }
             break;
         case kP2:
