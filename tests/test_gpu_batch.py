@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 
 import naga_amd
-from tests.scenes import gpu_engine, grid_nodes, rel_l2
+from tests.scenes import gpu_engine, grid_nodes, oracle_engine, rel_l2
 
 pytestmark = pytest.mark.gpu
 
@@ -112,12 +112,11 @@ def test_autotune_leaves_scenes_unchanged(oracle64):
 
 
 @pytest.mark.parametrize("form", [(3, False), (9, False)])
-def test_q9_kernel_forms(oracle64, monkeypatch, form):
-    """The autotuner's D2Q9 kernel forms advance every scene alike: three
-    distributions per lane reading the tile unions staged in LDS (scenes
-    set up with NAGA_Q9_UNIONS=1), the same gathering directly, one
-    distribution per lane."""
-    monkeypatch.setenv("NAGA_Q9_UNIONS", "1")
+def test_q9_kernel_forms(oracle64, form):
+    """The D2Q9 kernel forms, two lanes per node (lanes 3) and one lane per
+    distribution (9), advance every scene alike and as the oracle does; the
+    unions flag, which selects no kernel, is kept and reported with lanes 3 and
+    rejected with 9."""
     specs = [s for s in _specs() if s[0] == 2]
     runs = {}
     for lanes, unions in ((3, True), form):
@@ -132,9 +131,16 @@ def test_q9_kernel_forms(oracle64, monkeypatch, form):
         batch.set_q9_kernels(4)
     with pytest.raises(ValueError):
         batch.set_q9_kernels(9, True)
-    for a, b in zip(runs[(3, True)], runs[form]):
-        assert rel_l2(a["drho"], b["drho"]) < 1e-6
-        assert rel_l2(a["u"], b["u"]) < 1e-6
+    for (_, h, k, layer_cells, centre), a, b in zip(specs, runs[(3, True)], runs[form]):
+        ref = oracle_engine(oracle64, grid_nodes(oracle64, 2, h, layer=layer_cells * h), 9, k, h)
+        ref.set_pulse(centre, 1e-3, 0.1)
+        ref.step(20)
+        want = ref.get(fresh=True)
+        for f in ("drho", "u"):
+            assert rel_l2(a[f], b[f]) < 1e-6
+            assert rel_l2(b[f], want[f]) < 1e-5
+            if form[0] == 3:
+                assert np.array_equal(a[f], b[f])
 
 
 def test_batch_mixes_union_and_direct_scenes(oracle64, monkeypatch):
