@@ -53,9 +53,12 @@ struct StepGeom {
     int64_t nfluid;   // nbulk + nlayer; [nfluid, N) boundary
     int k;            // divergence stencil width of the records (step_width)
     int kb;           // boundary interpolation stencil width
-    int pml64;        // fused D3Q27 collision: PML local terms in FP64 (stencil widths other
-                      // than 16, 32 and 48; in FP32 the pass is 2 to 3 us shorter at
-                      // 10k to 130k nodes, which these three widths rely on)
+    int pml64;        // fused D3Q27 collision: PML local terms in FP64, for the stencil
+                      // widths whose own kernels formed them so (all but 16, 32 and
+                      // 48: none loses precision by sharing the pass).  Against the
+                      // FP64 oracle, cubes with 0.3 wide layers after 60 to 100 steps
+                      // differ by 1.0 to 3.1e-7 in FP32, 1.0 to 3.1e-7 in FP64 (at most
+                      // 1.6 times less); FP32 steps are 1 us (1.5 %) shorter there
     int pml_ref;      // layer field reads Q at (j - nbulk) as the reference
     float dt;         // lattice time step
     float rho0;       // nominal density
