@@ -292,8 +292,8 @@ __global__ __launch_bounds__(kP1Block) void k_p1_9(StepGeom G, StepBuffers S, Co
     if (lane < 18) S.partial[int64_t(lane) * S.nparts + w0 / 64] = mine;
 }
 
-template <int Q>
 __global__ __launch_bounds__(kBlock) void k_pml_local(StepGeom G, StepBuffers S, BatchArgs B) {
+    constexpr int Q = 27;
     using L = Lattice<Q>;
     constexpr int NPB = kBlock / 64 * L::NPW;
     __shared__ double red[NPB][2][Q];
@@ -371,8 +371,8 @@ __global__ __launch_bounds__(256) void k_means(StepGeom G, StepBuffers S, BatchA
 // Gf_a(j) = -2 sigma_j (Q1_a(p) - m1_a) + sigma_j^2 (Q2_a(p) - m2_a),
 // p = j - num_bulk (reference indexing) or j.  Rows outside the layer stay
 // zero, so the divergence pass needs no branch.
-template <int Q>
 __global__ __launch_bounds__(kBlock) void k_pml_field(StepGeom G, StepBuffers S, BatchArgs B) {
+    constexpr int Q = 27;
     const BlockCtx bc = locate(B, G, S);
     const LaneMap<Q> m(xcd_tile(bc.b, bc.nb));
     if (m.node >= G.nlayer || !m.active) return;
@@ -2554,12 +2554,12 @@ void launch_pass(int pass, int64_t nb, const StepGeom& G, const StepBuffers& S,
             break;
         case kPl:
             if (v4) k_pml_local_v4<<<nb, kBlock, 0, st>>>(G, S, c.B);
-            else k_pml_local<27><<<nb, kBlock, 0, st>>>(G, S, c.B);
+            else k_pml_local<<<nb, kBlock, 0, st>>>(G, S, c.B);
             break;
         case kPm: k_means<Q><<<nb, 256, 0, st>>>(G, S, c.B); break;
         case kPf:
             if (Q == 27 && !v4) {
-                k_pml_field<27><<<nb, kBlock, 0, st>>>(G, S, c.B);
+                k_pml_field<<<nb, kBlock, 0, st>>>(G, S, c.B);
             } else if (Q == 27) {
                 if (c.B.scenes || means_in_field<27>(S))
                     k_pml_field_v4<true><<<nb, kBlock, 0, st>>>(G, S, c.B);
