@@ -1,7 +1,8 @@
 """Exact kNN of clouds that each part of the search serves: boxes of cells
-(evenly spread points), radii retried (clusters, edges of the cloud), rings
-(ties beyond a wavefront, points far apart, distances past the largest
-float), against brute force with the same FP32 keys."""
+(evenly spread points), radii retried (clusters, edges of the cloud, ties),
+narrow cells (crowded clouds), rings (points far apart, distances past the
+largest float), against brute force with the same FP32 keys; and the time of
+repeated points and crowded clouds against random ones."""
 import time
 
 import numpy as np
