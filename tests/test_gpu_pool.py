@@ -26,7 +26,7 @@ def _solve(nodes, Q, k, h):
 
 
 def test_kept_memory_is_given_back(oracle64):
-    """Closed scenes' memory is kept for the next, and returned to the driver by
+    """Closed scenes' memory is kept for the next, and given back to the device by
     trim_memory."""
     nodes = grid_nodes(oracle64, 3, 0.04, 0.08)
     gpu_engine(nodes, 27, 32, 0.04, kb=16).close()  # the process' own memory: code, queues
